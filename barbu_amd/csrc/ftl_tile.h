@@ -24,12 +24,14 @@
 //   * Only the last iteration's velocity reaches the output (every iteration
 //     overwrites u_i for i >= 1 before reading it), so velocity work, the
 //     damped shift and the reflections are done in the last iteration only.
+//     With G > 1 the lanes of a strand reach it at different time steps; each
+//     then parks its points' positions before the sweep, skips its collisions,
+//     and all lanes form their velocities and collide together after the
+//     pipeline drains (settle).
 //   * Store: the inverse of the load, through the same LDS buffer, so every
-//     global store writes whole 128-byte lines.  With G = 1, velocities leave
-//     chunk by chunk during the last sweep and positions after it.  With G > 1
-//     the lanes of a strand finish at different time steps, so velocities are
-//     written by each lane as they become final; positions leave coalesced
-//     after the pipeline drains.
+//     global store writes whole 128-byte lines.  Velocities leave chunk by
+//     chunk (G = 1: during the last sweep; G > 1: as they settle), positions
+//     after them.
 //   * In place: a tile owns its strands, so no second buffer and no copy-back.
 
 #pragma once
@@ -63,12 +65,21 @@ struct Tile {
   static constexpr int SPT = FTL_WAVE / G;   // strands per tile
 };
 
-// Pipelined forms stage their final velocities through LDS (whole-line
-// stores) when a lane holds at most two chunks; with more, the flushes inside
-// the unrolled sweep cost more registers than the partial-line stores they
-// replace, and each lane stores its velocities directly.
-template <int M, int G>
-constexpr bool kStagedVel = (M / Tile<M, G, false>::C) <= 2;
+// Points of a lane that a pipelined form parks in LDS for the settle pass
+// (their positions before the last iteration's sweep, three floats each): the
+// first chunk, in the load/store stage, which is idle between the load and the
+// stores.  The others wait in registers.  Forms with at most 8 points per lane
+// park all of theirs in registers: their budget holds them.  The 24-point form
+// parks two chunks (at its three waves per SIMD the LDS has room for them, and
+// its registers do not: 14 spilled with one).
+template <int M, int G, bool GUARD>
+constexpr int kParkLds = M <= 8 ? 0 : (M == 24 ? 2 : 1) * Tile<M, G, GUARD>::C;
+
+// Component c of chunk point j of a lane, in the stage seen as floats (parked
+// positions, then the chunk's velocities): 24 columns of 65 floats, so that
+// neither a wave's own accesses (lane by lane) nor the flush's (8 points of 8
+// lanes) fall on one bank.
+__device__ __forceinline__ int park_slot(int j, int c, int lane) { return (3 * j + c) * (FTL_WAVE + 1) + lane; }
 
 // LDS slot of (owner lane r, point j of the chunk): XOR swizzle, conflict-free
 // for both the per-lane and the coalesced access order.
@@ -153,15 +164,13 @@ __device__ __forceinline__ void tile_sync() {
 }
 
 // Writes chunk c of the tile (C points per lane, staged in LDS) to dst in
-// the coalesced order of the load.  Called by the whole wave.  gsel >= 0
-// writes only the points owned by lanes with g == gsel (the lanes of a
-// strand finish at different time steps in the pipelined forms).  NT: the
+// the coalesced order of the load.  Called by the whole wave.  NT: the
 // stores carry the non-temporal hint (launches whose state is too large for
 // the next step to find any of it in the caches).
 typedef float ftl_nt_f4 __attribute__((ext_vector_type(4)));
 template <int M, int G, bool GUARD, bool NT>
 __device__ __forceinline__ void flush_chunk(float4* __restrict__ dst, int strand0, int nstr, int N, int c,
-                                            const float4* __restrict__ stage, int lane, int gsel = -1) {
+                                            const float4* __restrict__ stage, int lane) {
   constexpr int C = Tile<M, G, GUARD>::C;
   // Row k holds, in lane ln, point ln % C of the chunk of owner lane
   // r = k * (64 / C) + ln / C.  64 / C is a multiple of G and of C, so from row
@@ -176,7 +185,7 @@ __device__ __forceinline__ void flush_chunk(float4* __restrict__ dst, int strand
   const int r0 = ln / C, j = ln % C;
   const int s0 = strand0 + r0 / G;
   const int cp = (r0 % G) * M + c * C + j;
-  const bool mine = (!GUARD || cp < N) && (gsel < 0 || r0 % G == gsel);
+  const bool mine = !GUARD || cp < N;
   float4* __restrict__ d0 = dst + ((size_t)s0 * N + cp);
   const float4* __restrict__ t0 = stage + slot<C>(r0, j);
   tile_sync();
@@ -192,26 +201,32 @@ __device__ __forceinline__ void flush_chunk(float4* __restrict__ dst, int strand
   tile_sync();
 }
 
-// Lane-predicated collisions of one point: lanes with `on` false are left
-// untouched; `reflect` also reflects u (last iteration).
-__device__ __forceinline__ void collide_pred(const Spheres& S, float3& p, float3& u, bool on, bool reflect,
-                                             unsigned cmask) {
+// The same for velocities, staged as three floats per point (park_slot).
+template <int M, int G, bool GUARD, bool NT>
+__device__ __forceinline__ void flush_velocities(float4* __restrict__ dst, int strand0, int nstr, int N, int c,
+                                                 const float* stage, int lane) {
+  constexpr int C = Tile<M, G, GUARD>::C;
+  constexpr int RS = FTL_WAVE / C / G;
+  int ln = lane;
+  asm volatile("" : "+v"(ln));
+  const int r0 = ln / C, j = ln % C;
+  const int s0 = strand0 + r0 / G;
+  const int cp = (r0 % G) * M + c * C + j;
+  const bool mine = !GUARD || cp < N;
+  float4* __restrict__ d0 = dst + ((size_t)s0 * N + cp);
+  const float* t0 = stage + park_slot(j, 0, r0);
+  tile_sync();
 #pragma unroll
-  for (int k = 0; k < FTL_NCOL; ++k) {
-    if (!has_collider(cmask, k)) continue;
-    const float3 c = f3(S.c[k][0], S.c[k][1], S.c[k][2]);
-    const float3 w = sub3(p, c);
-    const float dp = dot3(w, w);
-    if (on && dp < S.r2[k]) {
-      const float is = rsqrt_c(dp);
-      const float3 n = mul3(w, is);
-      p = fma3(S.r[k], n, c);
-      if (reflect) {
-        const float d2 = 2.0f * dot3(n, u);
-        u = fma3(-d2, n, u);
-      }
+  for (int k = 0; k < C; ++k)
+    if (mine && s0 + k * RS < nstr) {
+      const float* t = t0 + k * (FTL_WAVE / C);
+      const float x = t[0], y = t[FTL_WAVE + 1], z = t[2 * (FTL_WAVE + 1)];
+      if constexpr (NT)
+        __builtin_nontemporal_store(ftl_nt_f4{x, y, z, 0.0f}, (ftl_nt_f4*)&d0[(size_t)(k * RS) * N]);
+      else
+        d0[(size_t)(k * RS) * N] = make_float4(x, y, z, 0.0f);
     }
-  }
+  tile_sync();
 }
 
 // Collisions of a sweep's points (not its last iteration), after all of the
@@ -312,100 +327,44 @@ __device__ __forceinline__ float from_prev_lane(float x) {
 }
 
 // One time step of the lane pipeline (G > 1): every lane runs the same code;
-// `active` lanes perform iteration t - g, `fin` lanes are in their last
-// iteration and also write their final velocities (lanes finish at different
-// time steps, so these go straight to memory; positions leave coalesced after
-// the pipeline drains).  FINS: some lane may be in its last
-// iteration (the last G time steps); the earlier steps skip the velocity work.
-// GUARD (strands of N = NS points, the last lane of a strand holding fewer
-// than M): tip is that lane's slot of the strand's last point (-1 on the other
-// lanes).  The slots after it hold copies of the last input point; they are
-// swept (finite, never stored) but take no velocity work, and the tip itself
-// is finished at its own slot in the last iteration (its velocity is its own
-// correction, as for the last lane of a full strand).
-template <int M, int G, bool FINS, bool GUARD, bool NT>
-__device__ __forceinline__ void sweep_pipe(const FtlStep& A, const VelArgs& V, const Spheres& S, float3 (&p)[M],
-                                           const LenRegs<M>& l,
-                                           float3 lead, int g, bool active, bool fin, int gfin,
-                                           const float4* __restrict__ pp, float4* __restrict__ stage, int strand0,
-                                           int lane, float3 u0, float3& last_pre, float3& cfirst, float3& clast,
-                                           unsigned cm, int NS = M * G, int tip = -1, bool* tbad = nullptr) {
-  constexpr int C = Tile<M, G, GUARD>::C;
-  // The final steps' velocity constants in vector registers (vector-only
-  // operands issue at twice the rate of a scalar operand).
-  float dl = V.delta;
-  VelArgs Vv = V;
-  if constexpr (FINS) asm volatile("" : "+v"(dl), "+v"(Vv.inv_dt), "+v"(Vv.maxv2));
-  if (!FINS) fin = false;
+// `active` lanes perform iteration t - g.  PARK: some lane may be in its last
+// iteration (the last G time steps): those lanes (`fin`) keep their points'
+// positions before the sweep (PL of them in LDS, the others in q) and leave
+// their collisions to the settle pass.  lead: the previous lane's last point
+// of the same iteration, before its collision; the next step's is fetched
+// here, between the sweep and the collisions.
+// GUARD: the last lane of a strand may hold fewer than M points; the slots
+// after its last one hold copies of the last input point, which are swept
+// (finite, never stored).
+template <int M, int G, bool GUARD, bool PARK, int PL, int NQ>
+__device__ __forceinline__ void sweep_pipe(const Spheres& S, float3 (&p)[M], const LenRegs<M>& l, float3& lead, int g,
+                                           bool active, bool fin, float* park, float3 (&q)[NQ],
+                                           unsigned cm) {
+  if (PARK && fin) {
+#pragma unroll
+    for (int j = 0; j < M; ++j) {
+      if (j < PL) {
+        park[park_slot(j, 0, 0)] = p[j].x;
+        park[park_slot(j, 1, 0)] = p[j].y;
+        park[park_slot(j, 2, 0)] = p[j].z;
+      } else {
+        q[j - PL] = p[j];
+      }
+    }
+  }
 #pragma unroll
   for (int j = 0; j < M; ++j) {
-    const float3 q = p[j];
     const bool upd = active && (j != 0 || g != 0);  // lane 0's slot 0 is the root
     // The point is updated in its own registers under the lane mask (a select
     // would be three vector instructions with a scalar mask operand); its
     // leader is the previous point before that point's collision.
     if (upd) ftl_point(p[j], j == 0 ? lead : p[j - 1], l.get(j));  // l holds sigma * rest length
-    const float3 pn = p[j];
-    if (FINS) {
-      const float3 c = sub3(pn, q);
-      if (j == 0) cfirst = sel3(fin, c, cfirst);
-      if (j >= 1) {
-        const int m = j - 1;
-        const bool root = (m == 0) && (g == 0);
-        // GUARD: m is a real point before the tip (or any point of a full lane)
-        const bool real = !GUARD || tip < 0 || m < tip;
-        const bool skip = GUARD && fin && m == tip;  // finished at its own slot
-        float3 pm = p[m];
-        float3 u = mul3(c, dl);
-        if (m == 0) u = sel3(g == 0, u0, u);
-        collide_pred(S, pm, u, active && !root && !skip, fin, cm);
-        p[m] = pm;
-        // Final velocities go through the LDS stage; a completed chunk of the
-        // finishing lanes leaves coalesced.  The last chunk waits for the
-        // lane's last point (after the pipeline drains).
-        if constexpr (kStagedVel<M, G>) {
-          if (fin && real) {
-            const float3 v = out_velocity(Vv, pp, m, pm, u);
-            stage[slot<C>(lane, m % C)] = make_float4(v.x, v.y, v.z, 0.0f);
-          }
-          if (m % C == C - 1 && m / C < M / C - 1)
-            flush_chunk<M, G, GUARD, NT>(A.vel, strand0, A.nstrands, NS, m / C, stage, lane, gfin);
-        } else if (fin && real && strand0 + lane / G < A.nstrands) {
-          const float3 v = out_velocity(Vv, pp, m, pm, u);
-          A.vel[(size_t)(strand0 + lane / G) * NS + g * M + m] = make_float4(v.x, v.y, v.z, 0.0f);
-        }
-      }
-      if constexpr (GUARD) {
-        if (fin && j == tip) {
-          // the strand's last point: its own correction, collided and reflected
-          float3 pt = pn, ut = c;
-          collide_pred(S, pt, ut, true, true, cm);
-          p[j] = pt;
-          const float3 v = out_velocity(Vv, pp, j, pt, ut);
-          if constexpr (kStagedVel<M, G>) {
-            stage[slot<C>(lane, j % C)] = make_float4(v.x, v.y, v.z, 0.0f);
-          } else if (strand0 + lane / G < A.nstrands) {
-            A.vel[(size_t)(strand0 + lane / G) * NS + g * M + j] = make_float4(v.x, v.y, v.z, 0.0f);
-          }
-          *tbad = !(isfinite(pt.x) && isfinite(pt.y) && isfinite(pt.z) && isfinite(v.x) && isfinite(v.y) &&
-                    isfinite(v.z));
-        }
-      }
-      if (j == M - 1) clast = sel3(fin, c, clast);
-    }
-    if (j == M - 1) {
-      // An inactive lane's value is read only by the next lane while that lane
-      // is inactive too (fill and drain shift by one step per lane).
-      last_pre = pn;
-      if (FINS) {
-        float3 dummy = f3(0.f, 0.f, 0.f);
-        collide_pred(S, p[j], dummy, active && !fin, false, cm);  // deferred when final
-      }
-    }
   }
-  // Before the final steps every point collides after the whole sweep (the
-  // root of lane 0 excepted).
-  if (!FINS) collide_sweep<M>(S, p, active, g != 0, M, cm);
+  // (An inactive lane's value is read only by the next lane while that lane is
+  // inactive too: fill and drain shift by one step per lane.)
+  lead = f3(from_prev_lane(p[M - 1].x), from_prev_lane(p[M - 1].y), from_prev_lane(p[M - 1].z));
+  // Every point collides after the whole sweep (the root of lane 0 excepted).
+  collide_sweep<M>(S, p, PARK ? active && !fin : active, g != 0, M, cm);
 }
 
 // Shared memory of one tile: the load/store stage, and the rest lengths of
@@ -420,7 +379,9 @@ struct TileLens<M, false> {};
 
 template <int M, int G, bool GUARD>
 struct TileLds : TileLens<M, G == 1> {
-  float4 stage[FTL_WAVE * Tile<M, G, GUARD>::C];
+  static constexpr int kStage = FTL_WAVE * Tile<M, G, GUARD>::C;
+  static constexpr int kPark = (3 * kParkLds<M, G, GUARD> * (FTL_WAVE + 1) + 3) / 4;
+  float4 stage[G > 1 && kPark > kStage ? kPark : kStage];
 };
 
 // PD: rows of the load phase whose loads are in flight ahead of the row being
@@ -587,11 +548,11 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
   // Lane's own points, for the DFTL re-read of x (never stored through).
   const float4* __restrict__ pp = A.pos + (size_t)(valid ? strand : 0) * N + (size_t)g * M;
   const int K = A.iterations;
-  float3 last_pre = p[0];
-  float3 cfirst = f3(0.f, 0.f, 0.f), clast = f3(0.f, 0.f, 0.f);
-  float3 u;
   bool bad = false;
   if constexpr (G == 1) {
+    float3 last_pre = p[0];
+    float3 clast = f3(0.f, 0.f, 0.f);
+    float3 u;
     for (int it = 0; it < K - 1; ++it)
       sweep<M, GUARD, false, NT>(A, V, S, p, l, nl, pp, last_pre, clast, stage, strand0, N, lane, cm);
     sweep<M, GUARD, true, NT>(A, V, S, p, l, nl, pp, last_pre, clast, stage, strand0, N, lane, cm);
@@ -611,49 +572,60 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
       }
     }
   } else {
-    // No lane is in its last iteration before time step K - 1.
-    // GUARD: the last lane of a strand finishes its tip (slot nl - 1) in its
-    // last sweep; the other lanes keep the post-drain path below.
     static_assert(16 % G == 0, "a strand's lanes lie in one row of 16 lanes");
-    const int tip = (GUARD && g == G - 1) ? nl - 1 : -1;
-    bool tbad = false;
-    for (int t = 0; t < K - 1; ++t) {
-      const float3 li = f3(from_prev_lane(last_pre.x), from_prev_lane(last_pre.y), from_prev_lane(last_pre.z));
-      // (lane 0 of a strand never reads its lead: its slot 0 is the root)
-      const float3 lead = li;
-      sweep_pipe<M, G, false, GUARD, NT>(A, V, S, p, l, lead, g, t >= g, false, -1, pp, stage, strand0, lane, u0,
-                                     last_pre, cfirst, clast, cm, N, tip, &tbad);
-    }
+    constexpr int PL = kParkLds<M, G, GUARD>;
+    constexpr int NQ = M - PL;
+    float* const park = (float*)stage + lane;
+    float3 q[NQ];  // every lane fills it in its last iteration
+    // No lane is in its last iteration before time step K - 1.  (lane 0 of a
+    // strand never reads its lead: its slot 0 is the root)
+    float3 lead = p[0];
+    for (int t = 0; t < K - 1; ++t)
+      sweep_pipe<M, G, GUARD, false, PL, NQ>(S, p, l, lead, g, t >= g, false, park, q, cm);
     for (int t = K - 1; t < K + G - 1; ++t) {
-      const float3 li = f3(from_prev_lane(last_pre.x), from_prev_lane(last_pre.y), from_prev_lane(last_pre.z));
-      const float3 lead = li;
       const int it = t - g;
-      sweep_pipe<M, G, true, GUARD, NT>(A, V, S, p, l, lead, g, it >= 0 && it < K, it == K - 1, t - (K - 1), pp,
-                                    stage, strand0, lane, u0, last_pre, cfirst, clast, cm, N, tip, &tbad);
+      sweep_pipe<M, G, GUARD, true, PL, NQ>(S, p, l, lead, g, it >= 0 && it < K, it == K - 1, park, q, cm);
     }
-    // The lane's last point: its velocity needs the next lane's correction.
-    const float3 cn = f3(__shfl_down(cfirst.x, 1, G), __shfl_down(cfirst.y, 1, G),
-                         __shfl_down(cfirst.z, 1, G));
-    u = sel3(g == G - 1, clast, mul3(cn, V.delta));
-    float3 pm = p[M - 1];
-    const bool own = !GUARD || tip < 0;  // GUARD: the tip lane is done
-    if constexpr (GUARD)
-      collide_pred(S, pm, u, own, true, cm);
-    else
-      collide<true>(S, pm, u, cm);
-    p[M - 1] = pm;
-    // (GUARD: the tip lane's slot M - 1 may lie past the strand; it reads the
-    // strand's first point instead, and the result is dropped)
-    const float3 v = out_velocity(V, pp, own ? M - 1 : 0, pm, u);
-    if constexpr (kStagedVel<M, G>) {
-      if (own) stage[slot<C>(lane, (M - 1) % C)] = make_float4(v.x, v.y, v.z, 0.0f);
-      flush_chunk<M, G, GUARD, NT>(A.vel, strand0, nstr, N, M / C - 1, stage, lane);
-    } else if (valid && own) {
-      A.vel[(size_t)strand * N + g * M + (M - 1)] = make_float4(v.x, v.y, v.z, 0.0f);
+    // Settle: the last iteration's corrections c_j = p_j - parked p_j give the
+    // velocities u_j = delta * c_(j+1) (the next lane's first for a lane's last
+    // point; the strand's last point keeps its own, the root p0 - x0), then the
+    // iteration's collisions push the points and reflect the velocities.  Once
+    // per lane: done inside the pipeline's last G steps, this work ran in every
+    // one of them for one lane group in G (about 16 vector instructions per
+    // point and step).  The long forms are bound by vector issue: 50,021 x 64
+    // at 16 iterations 95.0 -> 87.7 us, 60,013 x 20 with wind 42.8 -> 40.1, a
+    // frame of 32 uneven grooms 540 -> 525, 262,144 x 32 with wind 137.1 -> 135.1.
+    auto parked = [&](int j) -> float3 {
+      return j < PL ? f3(park[park_slot(j, 0, 0)], park[park_slot(j, 1, 0)], park[park_slot(j, 2, 0)])
+                    : q[j < PL ? 0 : j - PL];
+    };
+    const float3 c0 = sub3(p[0], parked(0));
+    const float3 cn = f3(__shfl_down(c0.x, 1, G), __shfl_down(c0.y, 1, G), __shfl_down(c0.z, 1, G));
+    const int tip = g == G - 1 ? nl - 1 : -1;  // slot of the strand's last point on its lane
+    const bool root = g == 0;
+    float dl = V.delta;
+    asm volatile("" : "+v"(dl));
+    float3 c = c0;
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const float3 own = c;
+      c = m + 1 < M ? sub3(p[m + 1 < M ? m + 1 : m], parked(m + 1 < M ? m + 1 : m)) : cn;
+      float3 u = mul3(c, dl);
+      if (m == 0) u = sel3(root, u0, u);
+      if (GUARD || m == M - 1) u = sel3(tip == m, own, u);
+      if (m > 0 || !root) collide<true>(S, p[m], u, cm);
+      // GUARD: slots past the strand's last point read its first point
+      // instead, and the result is dropped
+      const float3 v = out_velocity(V, pp, GUARD && m >= nl ? 0 : m, p[m], u);
+      // (the point's own parked words, no longer needed)
+      park[park_slot(m % C, 0, 0)] = v.x;
+      park[park_slot(m % C, 1, 0)] = v.y;
+      park[park_slot(m % C, 2, 0)] = v.z;
+      if (GUARD ? m == nl - 1 : m == M - 1)
+        bad = !(isfinite(p[m].x) && isfinite(p[m].y) && isfinite(p[m].z) && isfinite(v.x) && isfinite(v.y) &&
+                isfinite(v.z));
+      if (m % C == C - 1) flush_velocities<M, G, GUARD, NT>(A.vel, strand0, nstr, N, m / C, (float*)stage, lane);
     }
-    bad = own ? !(isfinite(pm.x) && isfinite(pm.y) && isfinite(pm.z) && isfinite(v.x) && isfinite(v.y) &&
-                  isfinite(v.z))
-              : tbad;
   }
   // positions, after every velocity (DFTL reads the step's input positions)
 #pragma unroll
