@@ -41,6 +41,8 @@ def _units():
         # (The other classes compile to the same code with or without it.)
         units.append(("ftl_plain.hip", ["-DFTL_CLASS_ID=%d" % k, "-mllvm", "-pragma-unroll-threshold=200000"],
                       "plain_%d.o" % k))
+    for g in (2, 4, 8, 16, 0):  # the wide forms by lanes per strand; 0: all of them in one kernel
+        units.append(("ftl_wide.hip", ["-DFTL_WIDE_LANES=%d" % g], "wide_%d.o" % g))
     for src in ("ftl_misc.hip", "ftl_render.hip", "ftl_init.hip", "ftl_marschner.hip", "ftl_api.cpp", "ftl_batch_api.cpp", "ftl_autotune.cpp",
                 "ftl_scenario.cpp", "ftl_server.cpp"):
         units.append((src, [], os.path.splitext(src)[0] + ".o"))

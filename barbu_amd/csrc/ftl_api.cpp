@@ -577,11 +577,19 @@ static ftl_status groom_step(ftl_groom* g, float dt, void* stream, hipEvent_t st
   FtlStep A;
   ftl_status st = ftl_make_step(g, dt, &A);
   if (st != FTL_OK) return st;
-  const int cls = ftl_class_for(g->ctx, g->npoints, g->lanes, FTL_MAX_POINTS, A.wind_grid != 0);
-  if (cls < 0) return ftl_fail(FTL_ERR_UNSUPPORTED, "no launch class for npoints=%d", g->npoints);
+  // lanes left to the library: by the size of the launch
+  const int form =
+      g->lanes == 0 ? ftl_wide_form(ftl_wide_level(g->ctx->ncu, &g->nstrands, &g->npoints, 1), g->npoints) : -1;
+  const int cls = form >= 0 ? -1 : ftl_class_for(g->ctx, g->npoints, g->lanes, FTL_MAX_POINTS, A.wind_grid != 0);
+  if (form < 0 && cls < 0) return ftl_fail(FTL_ERR_UNSUPPORTED, "no launch class for npoints=%d", g->npoints);
   hipError_t e;
   if ((e = hipSetDevice(g->ctx->device)) != hipSuccess) return ftl_hip_fail(e, "hipSetDevice");
   const bool nt = (size_t)g->nstrands * g->npoints * 2 * sizeof(float4) > ftl_stream_store_bytes();
+  if (form >= 0) {
+    if ((e = ftl_launch_wide(form, A, (hipStream_t)stream, start, stop, nt)) != hipSuccess)
+      return ftl_hip_fail(e, "FTL step launch");
+    return FTL_OK;
+  }
   if ((e = ftl_launch_plain(cls, A, (hipStream_t)stream, start, stop, nt)) != hipSuccess)
     return ftl_hip_fail(e, "FTL step launch");
   return FTL_OK;

@@ -46,44 +46,57 @@ struct ftl_batch {
 // Time per control point of a launch class in ns for K iterations: measured
 // by the autotuner (at 8 iterations) where available, otherwise estimated.
 static double class_ns_per_cp(const ftl_ctx* ctx, int cls, int K) {
-  const FtlClassInfo& k = kFtlClasses[cls];
+  const bool wide = cls >= FTL_NCLASSES;
+  const int g = wide ? ftl_wide_g(cls) : kFtlClasses[cls].g;
   // per-lane work: M points through K + G - 1 pipeline steps, plus about
   // three steps' worth of loads, wind and stores
-  const double steps = (double)(K + k.g + 2) / (double)(8 + k.g + 2);
-  double ns = ctx->cls_ns_cp[cls];
-  if (!(ns > 0.0)) ns = (k.guarded ? 0.028 : 0.022) * (k.g == 1 ? 1.0 : 1.0 + 0.1 * (k.g - 1));
+  const double steps = (double)(K + g + 2) / (double)(8 + g + 2);
+  double ns = wide ? 0.0 : ctx->cls_ns_cp[cls];
+  if (!(ns > 0.0)) ns = (!wide && kFtlClasses[cls].guarded ? 0.028 : 0.022) * (g == 1 ? 1.0 : 1.0 + 0.1 * (g - 1));
   return ns * steps;
 }
 
-// Plans the tiles of a set of grooms, grouped by launch class (the class with
-// the most expected work first; within a class, grooms with more iterations
-// first), as one span per groom.  Linear in the number of grooms: the serving
-// loop plans a batch per launch.
+// Plans the tiles of a set of grooms as one span per groom: a batch whose
+// waves all fit the chip at once is one launch of the wide forms' common
+// kernel, each groom in the form of the batch's level; otherwise the grooms
+// are grouped by launch class or wide form (the one with the most expected
+// work first; within it, grooms with more iterations first).  Linear in the
+// number of grooms: the serving loop plans a batch per launch.
 ftl_status ftl_plan_tiles(ftl_ctx* ctx, ftl_groom* const* grooms, int n, std::vector<FtlSpan>& spans,
                           std::vector<ClassRun>& runs) {
   spans.clear();
   runs.clear();
-  struct GroomPlan {
-    int idx, cls, cost, ntiles;
-    double ns_tile;
-  };
-  std::vector<GroomPlan> plan;
-  plan.reserve(n);
-  std::vector<double> work(FTL_NCLASSES, 0.0);
-  size_t total_tiles = 0, state_bytes = 0;
+  bool automatic = true;  // every groom leaves its lanes to the library
+  std::vector<int> nstrands(n), npoints(n);
   for (int i = 0; i < n; ++i) {
     ftl_groom* g = grooms[i];
     if (!g) return ftl_fail(FTL_ERR_INVALID_ARGUMENT, "groom %d is NULL", i);
     if (g->ctx != ctx) return ftl_fail(FTL_ERR_INVALID_ARGUMENT, "groom %d belongs to another context", i);
-    const int cls = ftl_class_for(ctx, g->npoints, g->lanes, FTL_MAX_POINTS);
+    automatic = automatic && g->lanes == 0;
+    nstrands[i] = g->nstrands;
+    npoints[i] = g->npoints;
+  }
+  const int level = automatic ? ftl_wide_level(ctx->ncu, nstrands.data(), npoints.data(), n) : 0;
+  struct GroomPlan {
+    int idx, cls, run, cost, ntiles;
+  };
+  std::vector<GroomPlan> plan;
+  plan.reserve(n);
+  std::vector<double> work(ftl_wide_id(8, 31) + 1, 0.0);
+  size_t total_tiles = 0, state_bytes = 0;
+  for (int i = 0; i < n; ++i) {
+    ftl_groom* g = grooms[i];
+    int cls = g->lanes == 0 ? ftl_wide_form(level, g->npoints) : -1;
+    const bool wide = cls >= 0;
+    if (!wide) cls = ftl_class_for(ctx, g->npoints, g->lanes, FTL_MAX_POINTS);
     if (cls < 0) return ftl_fail(FTL_ERR_UNSUPPORTED, "no batched launch class for npoints=%d", g->npoints);
-    const FtlClassInfo& k = kFtlClasses[cls];
-    const int spt = FTL_WAVE / k.g;
+    const int km = wide ? ftl_wide_m(cls) : kFtlClasses[cls].m, kg = wide ? ftl_wide_g(cls) : kFtlClasses[cls].g;
+    const int spt = FTL_WAVE / kg;
     const int nt = (g->nstrands + spt - 1) / spt;
-    const int cost = k.m * (g->params.iterations + k.g - 1);
-    const double ns_tile = class_ns_per_cp(ctx, cls, g->params.iterations) * (double)FTL_WAVE * k.m;
-    plan.push_back(GroomPlan{i, cls, cost, nt, ns_tile});
-    work[cls] += ns_tile * nt;
+    const int cost = km * (g->params.iterations + kg - 1);
+    const int run = level > 0 ? FTL_WIDE_ALL : cls;
+    plan.push_back(GroomPlan{i, cls, run, cost, nt});
+    work[run] += class_ns_per_cp(ctx, cls, g->params.iterations) * (double)FTL_WAVE * km * nt;
     total_tiles += (size_t)nt;
     state_bytes += (size_t)g->nstrands * g->npoints * 2 * sizeof(float4);
   }
@@ -99,9 +112,9 @@ ftl_status ftl_plan_tiles(ftl_ctx* ctx, ftl_groom* const* grooms, int n, std::ve
   // Classes with the most expected work first (they start first and run
   // longest); within a class, the costliest grooms first.
   std::stable_sort(plan.begin(), plan.end(), [&](const GroomPlan& a, const GroomPlan& b) {
-    if (a.cls != b.cls) {
-      if (work[a.cls] != work[b.cls]) return work[a.cls] > work[b.cls];
-      return a.cls < b.cls;
+    if (a.run != b.run) {
+      if (work[a.run] != work[b.run]) return work[a.run] > work[b.run];
+      return a.run < b.run;
     }
     return a.cost > b.cost;
   });
@@ -109,17 +122,17 @@ ftl_status ftl_plan_tiles(ftl_ctx* ctx, ftl_groom* const* grooms, int n, std::ve
   // One workgroup per tile: the classes' kernels run side by side and the
   // hardware dispatcher hands free wave slots to whichever has tiles left.
   for (size_t i = 0; i < plan.size();) {
-    const int cls = plan[i].cls;
+    const int run = plan[i].run;
     const int first = (int)spans.size();
     int ntiles = 0;
-    for (; i < plan.size() && plan[i].cls == cls; ++i) {
+    for (; i < plan.size() && plan[i].run == run; ++i) {
       const GroomPlan& gp = plan[i];
       if (gp.ntiles <= 0) continue;  // no strands: nothing to step
-      spans.push_back(FtlSpan{gp.idx, ntiles, cls, gp.cost});
+      spans.push_back(FtlSpan{gp.idx, ntiles, gp.cls, gp.cost});
       ntiles += gp.ntiles;
     }
     const int count = (int)spans.size() - first;
-    if (count > 0) runs.push_back(ClassRun{cls, first, count, ntiles, ntiles, stream_stores});
+    if (count > 0) runs.push_back(ClassRun{run, first, count, ntiles, ntiles, stream_stores});
   }
   if (runs.size() > 64) return ftl_fail(FTL_ERR_UNSUPPORTED, "too many launch classes");
   return FTL_OK;
@@ -307,9 +320,10 @@ extern "C" ftl_status ftl_batch_create(ftl_ctx* ctx, ftl_groom* const* grooms, i
   b->grooms.assign(grooms, grooms + n);
   b->nspans = (int)spans.size();
   b->runs = runs;
-  for (const ClassRun& r : runs) {
-    b->ntiles += r.ntiles;
-    b->grid += r.grid;
+  for (const ClassRun& r : runs) b->grid += r.grid;
+  for (int i = 0; i < n; ++i) {
+    const int spt = FTL_WAVE / kFtlClasses[ftl_class_for(ctx, grooms[i]->npoints, grooms[i]->lanes, FTL_MAX_POINTS)].g;
+    b->ntiles += (grooms[i]->nstrands + spt - 1) / spt;
   }
   const size_t sb = (size_t)n * sizeof(FtlStep), tb = spans.size() * sizeof(FtlSpan);
   auto bail = [&](ftl_status s) {

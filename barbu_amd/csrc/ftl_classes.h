@@ -75,3 +75,19 @@ constexpr int ftl_chunk_of(int m, int g, bool guarded) {
   return m < 4 ? m : 4;
 #endif
 }
+
+// Wide forms (ftl_wide.h): X(points per lane M, lanes per strand G); a form
+// takes any point count N with M = ceil(N / G).  Not launch classes: the
+// library picks them by the size of a launch (ftl_wide_lanes).
+#define FTL_WIDE_FORMS_2(X) X(3, 2) X(4, 2) X(5, 2) X(6, 2) X(7, 2) X(8, 2)
+#define FTL_WIDE_FORMS_4(X) X(1, 4) X(2, 4) X(3, 4) X(4, 4) X(5, 4) X(6, 4) X(7, 4) X(8, 4)
+#define FTL_WIDE_FORMS_8(X) X(1, 8) X(2, 8) X(3, 8) X(4, 8) X(5, 8) X(6, 8) X(7, 8) X(8, 8)
+#define FTL_WIDE_FORMS_16(X) X(1, 16) X(2, 16) X(3, 16) X(4, 16)
+#define FTL_WIDE_FORMS(X) FTL_WIDE_FORMS_2(X) FTL_WIDE_FORMS_4(X) FTL_WIDE_FORMS_8(X) FTL_WIDE_FORMS_16(X)
+
+// Form ids, beside the class ids in a batch's runs and spans: the form with M
+// points on each of G lanes, and all forms in one kernel.
+constexpr int ftl_wide_id(int m, int g) { return 256 + 32 * m + g; }
+constexpr int ftl_wide_m(int id) { return (id - 256) / 32; }
+constexpr int ftl_wide_g(int id) { return (id - 256) % 32; }
+#define FTL_WIDE_ALL 128

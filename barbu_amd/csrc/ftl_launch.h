@@ -23,9 +23,19 @@ size_t ftl_stream_store_bytes();
 // nt: non-temporal stores (state above ftl_stream_store_bytes()).
 hipError_t ftl_launch_plain(int cls, const FtlStep& A, hipStream_t stream, hipEvent_t start = nullptr,
                             hipEvent_t stop = nullptr, bool nt = false);
+// Wide forms (ftl_wide.h).  The level of a launch over n grooms (16, 8 or 4:
+// the lanes per strand its long strands take), or 0 when it fills the chip.
+int ftl_wide_level(int ncu, const int* nstrands, const int* npoints, int n);
+// The form of a groom in a launch of that level; at level 0, the form of the
+// point counts no exact launch class holds, or -1 (a launch class is faster).
+int ftl_wide_form(int level, int npoints);
+// The plain step of one groom by a wide form.
+hipError_t ftl_launch_wide(int form, const FtlStep& A, hipStream_t stream, hipEvent_t start = nullptr,
+                           hipEvent_t stop = nullptr, bool nt = false);
 // Tile-list kernel of one class over the ntiles tiles of spans[0..nspans)
 // (every groom of that class, in tile order): workgroup b steps tiles b,
-// b + grid, ...
+// b + grid, ...  cls may be a wide form (ftl_wide_id) or FTL_WIDE_ALL, one
+// workgroup per tile.
 hipError_t ftl_launch_tiles(int cls, const FtlStep* grooms, const FtlSpan* spans, int nspans, int ntiles, int grid,
                             hipStream_t stream, bool nt);
 // Resident tile-list workgroups per CU for a class.

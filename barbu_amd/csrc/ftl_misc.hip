@@ -1,5 +1,6 @@
 // Small kernels and host dispatch: mesh skinning and root frames, the copy
-// reference, and the class table -> per-class launcher map.
+// reference, the class table -> per-class launcher map, and the choice of wide
+// forms.
 #include "ftl_classes.h"
 #include "ftl_device.h"
 #include "ftl_launch.h"
@@ -200,8 +201,95 @@ hipError_t ftl_launch_plain(int cls, const FtlStep& A, hipStream_t stream, hipEv
   return hipErrorInvalidValue;
 }
 
+#define FTL_WDECL(G)                                                                                               \
+  hipError_t ftl_launch_wide_##G(int m, const FtlStep& A, hipStream_t, hipEvent_t, hipEvent_t, bool);              \
+  hipError_t ftl_launch_wide_tiles_##G(int m, const FtlStep*, const FtlSpan*, int, int, hipStream_t, bool);
+FTL_WDECL(2)
+FTL_WDECL(4)
+FTL_WDECL(8)
+FTL_WDECL(16)
+#undef FTL_WDECL
+hipError_t ftl_launch_wide_all(const FtlStep*, const FtlSpan*, int, int, hipStream_t);
+
+// Lanes per strand of an npoints groom in a launch of this level.
+static int wide_lanes(int level, int npoints) {
+  if (level == 16) return npoints > 8 ? 16 : npoints > 4 ? 8 : 4;
+  if (level == 8) return npoints > 4 ? 8 : 4;
+  return npoints > 32 ? 8 : 4;
+}
+
+// More lanes per strand shorten a wave's chain and cost vector work, so a
+// launch takes the most lanes whose waves still leave the vector units free:
+// 2 waves per SIMD at 16 lanes, 4 at 8 and at 4.  Kernel us around the lines
+// (8 iterations, 2 colliders, no wind; class = the launch class):
+//   16 points:  8,192 strands  16 lanes 11.1, 8 lanes 11.6, class 19.0;  16,384  13.6, 12.3, 20.0
+//              32,768           8 lanes 15.6, 4 lanes 16.6, class 21.3;  65,536  24.1, 20.2, 23.3
+//             131,072           4 lanes 33.3, class 32.6
+//   32 points: 16,384          16 lanes 20.1, 8 lanes 19.5, class 36.4
+//              32,768           8 lanes 23.7, 4 lanes 26.4, class 37.3;  65,536  42.4, 37.4, 46.8
+//             131,072           4 lanes 64.3, class 59.6
+//   64 points: 16,384          16 lanes 32.1, 8 lanes 33.1, class 43.6
+//              32,768           8 lanes 44.0, class 52.0;                65,536  74.7, class 68.2
+//    4 points: 65,536           4 lanes 8.8, class 10.1;                131,072  13.3, class 11.9
+int ftl_wide_level(int ncu, const int* nstrands, const int* npoints, int n) {
+  for (int level = 16; level >= 4; level /= 2) {
+    int64_t waves = 0;
+    for (int i = 0; i < n; ++i) {
+      const int spt = FTL_WAVE / wide_lanes(level, npoints[i]);
+      waves += ((int64_t)nstrands[i] + spt - 1) / spt;
+    }
+    if (waves <= (int64_t)(level == 16 ? 8 : 16) * ncu) return level;
+  }
+  return 0;
+}
+
+// In a launch that fills the chip a point count with an exact launch class
+// takes it (and 2 and 3 points the one-lane guarded class).  The others pad
+// a guarded class's lanes; a wide form pads none of its loads and stores, and
+// at most its last lanes' sweeps (us at 262,144 strands, guarded class against
+// wide form: 6 points 29.8, 25.9; 9 points 51.6, 35.7; 20 points 81.6, 65.2;
+// 40 points 199, 160; 48 points 215, 192; 63 points 393, 276).
+int ftl_wide_form(int level, int npoints) {
+  int g;
+  if (level > 0) {
+    g = wide_lanes(level, npoints);
+  } else {
+    if (npoints < 5 || npoints == 8 || npoints == 16 || npoints == 32 || npoints == 64) return -1;
+    g = npoints <= 16 ? 2 : npoints <= 32 ? 4 : 8;
+  }
+  return ftl_wide_id((npoints + g - 1) / g, g);
+}
+
+hipError_t ftl_launch_wide(int form, const FtlStep& A, hipStream_t stream, hipEvent_t start, hipEvent_t stop,
+                           bool nt) {
+  const int m = ftl_wide_m(form), g = ftl_wide_g(form);
+  if (A.nstrands <= 0) return hipSuccess;
+  if (A.npoints > m * g || A.npoints <= (m - 1) * g) return hipErrorInvalidValue;
+  switch (g) {
+    case 2: return ftl_launch_wide_2(m, A, stream, start, stop, nt);
+    case 4: return ftl_launch_wide_4(m, A, stream, start, stop, nt);
+    case 8: return ftl_launch_wide_8(m, A, stream, start, stop, nt);
+    case 16: return ftl_launch_wide_16(m, A, stream, start, stop, nt);
+  }
+  return hipErrorInvalidValue;
+}
+
 hipError_t ftl_launch_tiles(int cls, const FtlStep* grooms, const FtlSpan* spans, int nspans, int ntiles, int grid,
                             hipStream_t stream, bool nt) {
+  if (cls == FTL_WIDE_ALL) {
+    if (ntiles <= 0 || nspans <= 0) return hipSuccess;
+    return ftl_launch_wide_all(grooms, spans, nspans, ntiles, stream);
+  }
+  if (cls >= ftl_wide_id(0, 0)) {
+    if (ntiles <= 0 || nspans <= 0) return hipSuccess;
+    const int m = ftl_wide_m(cls);
+    switch (ftl_wide_g(cls)) {
+      case 2: return ftl_launch_wide_tiles_2(m, grooms, spans, nspans, ntiles, stream, nt);
+      case 4: return ftl_launch_wide_tiles_4(m, grooms, spans, nspans, ntiles, stream, nt);
+      case 8: return ftl_launch_wide_tiles_8(m, grooms, spans, nspans, ntiles, stream, nt);
+    }
+    return hipErrorInvalidValue;
+  }
   switch (cls) {
 #define FTL_LB(id, M, G, GU, W, CH) \
   case id:                   \

@@ -187,7 +187,9 @@ ftl_status ftl_groom_info(ftl_groom* g, int* nstrands, int* npoints);
    holds NaN/Inf at a strand tip).  Synchronises the context's device. */
 ftl_status ftl_groom_status(ftl_groom* g, int* nonfinite);
 
-/* Launch shape of plain steps: lanes per strand (1, 2 or 4; 0 = automatic).
+/* Launch shape of plain steps: lanes per strand (1, 2 or 4; 0 = automatic: by
+   point count, and up to 16 lanes when the launch is too small to fill the
+   device).
    A point count that no class of that shape holds exactly runs a guarded
    class: one lane per strand if 1 was asked for, else the pipelined guarded
    class with the fewest points per lane.  Results do not depend on it. */
@@ -306,8 +308,9 @@ void ftl_batch_destroy(ftl_batch* b);
    with FTL_ERR_INVALID_ARGUMENT once one of the batch's grooms has been
    destroyed. */
 ftl_status ftl_batch_launch(ftl_batch* b, const float* dt, void* stream);
-/* Tiles (64-lane work units) in the batch and the total number of
-   workgroups its kernels launch. */
+/* Tiles (64-lane work units of the grooms' launch classes) in the batch and
+   the total number of workgroups its kernels launch (more than the tiles when
+   the batch is small: its strands then take more lanes). */
 ftl_status ftl_batch_info(ftl_batch* b, int* ntiles, int* grid);
 
 /* -- helpers -------------------------------------------------------------- */
@@ -341,8 +344,10 @@ int ftl_lanes_for(ftl_ctx* ctx, int npoints);
 /* The same for plain steps with wind.  No counterpart in the reference (its
    workgroup shape is fixed). */
 int ftl_lanes_for_wind(ftl_ctx* ctx, int npoints);
-/* The launch class the context picks for npoints (a plain step with wind
-   when wind != 0; batched and served steps use wind = 0), -1 if none.  A class
+/* The launch class the context picks for npoints in launches that fill the
+   device (a plain step with wind when wind != 0; batched and served steps use
+   wind = 0), -1 if none.  Smaller launches, and most point counts that no
+   exact class holds, run forms of their own (ftl_groom_set_lanes).  A class
    is a tile shape: points per lane, lanes per strand, the occupancy target the
    registers are allocated for and the load/store chunk; the tuning tables may
    pick a variant of a base class. */

@@ -1,0 +1,101 @@
+"""The wide forms (2 to 16 lanes per strand, at most 8 points per lane): small
+launches at each level, point counts around the edges of the lanes' shares,
+partial tiles, and the ragged point counts of launches that fill the chip.
+They perform the oracle's operations in the oracle's order: bit for bit."""
+import numpy as np
+import pytest
+
+import barbu_amd as ba
+from tests.helpers import assert_bitexact
+from tests.test_gpu_parity import DT, _oracle_frame, _rigid, run_compare
+
+pytestmark = pytest.mark.gpu
+
+SPHERES = [(0, 0, 0, 1), (0.3, 1.1, 0.0, 0.35)]
+
+
+def scene(nstrands, npoints, seed):
+    pos, vel, roots = ba.sphere_groom(nstrands, npoints, radius=1.0, length=0.3, seed=seed)
+    pos[:, 1:, :3] += np.float32([0.0, -0.05, 0.0])  # towards the colliders
+    vel[:, 1:, :3] = np.random.default_rng(seed).normal(scale=0.3, size=vel[:, 1:, :3].shape)
+    return pos, vel, roots
+
+
+@pytest.mark.parametrize("npoints", [2, 3, 4, 5, 7, 8, 9, 12, 15, 16, 17, 20, 31, 32, 33, 48, 49, 63, 64])
+@pytest.mark.parametrize("nstrands,iterations,dftl,scale,wind", [(1, 8, 0, 1.0, 0), (37, 1, 1, 1.45, 1), (517, 2, 0, 1.45, 1),
+                                                                 (2049, 8, 1, 1.0, 0)])
+def test_small_launches(ctx, npoints, nstrands, iterations, dftl, scale, wind):
+    pos, vel, roots = scene(nstrands, npoints, npoints)
+    params = ba.make_params(force_scale=1.0, damping=0.9, length_scale=scale, iterations=iterations, velocity_mode=dftl,
+                            max_velocity=2.0, wind_amplitude=2.0 * wind, wind_frequency=2.0, wind_seed=5)
+    run_compare(ctx, pos, vel, params, SPHERES, 2, roots=roots, root_mode=ba.FTL_ROOT_REST,
+                models=lambda k: _rigid(0, 0.1 * k), label="N=%d S=%d" % (npoints, nstrands))
+
+
+@pytest.mark.parametrize("nstrands", [8193, 32769, 70001])
+@pytest.mark.parametrize("npoints", [3, 4, 5, 6, 8, 10, 12, 13, 16, 20, 24, 27, 29, 32, 40, 47, 56, 64])
+def test_levels(ctx, npoints, nstrands):
+    """Past the lines between the levels (8,192 and 32,768 strands for the
+    longer strands) and between the wide forms and the launch classes."""
+    pos, vel, _ = scene(nstrands, npoints, 100 + npoints)
+    params = ba.make_params(force_scale=1.0, damping=0.9, length_scale=-1.1 if npoints == 20 else 1.0)
+    run_compare(ctx, pos, vel, params, SPHERES, 1, label="N=%d S=%d" % (npoints, nstrands))
+
+
+@pytest.mark.parametrize("npoints", [7, 20])
+def test_streaming_stores(ctx, npoints):
+    """A ragged groom above the state size from which stores are hinted."""
+    nstrands = (384 << 20) // (32 * npoints) + 1001
+    pos, vel, _ = ba.sphere_groom(nstrands, npoints, radius=1.0, length=0.3, seed=3)
+    run_compare(ctx, pos, vel, ba.make_params(force_scale=1.0, damping=0.9, length_scale=1.0), SPHERES, 1,
+                label="streaming N=%d" % npoints)
+
+
+def test_nan_stays_in_its_strand(ctx):
+    pos, vel, _ = scene(300, 20, 9)
+    g = ba.Groom(ctx, pos, vel)
+    g.step(DT)
+    assert g.status() is False
+    p, v = g.download()
+    v[17, 5, 0] = np.nan
+    p[40, 19, 1] = np.inf
+    g.upload(p, v)
+    g.step(DT)
+    assert g.status() is True
+    p, v = g.download()
+    bad = ~np.isfinite(p).all((1, 2))
+    assert bad[17] and set(np.nonzero(bad)[0]) <= {17, 40}
+    g.close()
+
+
+@pytest.mark.parametrize("scale", [1, 40, 400])
+def test_batch_levels(ctx, scale):
+    """The same scene as one launch of the common kernel (small), at the last
+    level, and grouped by classes and ragged forms (large)."""
+    grooms, states = [], []
+    for i, (s, n) in enumerate([(1, 8), (13, 16), (77, 32), (64, 64), (24, 4), (5, 2), (90, 20), (30, 5), (20, 48),
+                                (11, 9), (50, 33), (41, 63)]):
+        pos, vel, roots = scene(s * scale, n, 200 + i)
+        params = ba.make_params(force_scale=1.0, damping=0.9, length_scale=1.0, iterations=4 + i % 5)
+        g = ba.Groom(ctx, pos, vel, rest_roots=roots)
+        g.set_params(params)
+        g.set_root_mode(ba.FTL_ROOT_REST)
+        spheres = np.float32(SPHERES)[: 1 + i % 2]
+        g.set_colliders(spheres)
+        grooms.append(g)
+        states.append(dict(pos=pos.copy(), vel=vel.copy(), roots=roots, params=params, spheres=spheres, N=n))
+    b = ba.Batch(ctx, grooms)
+    for k in range(3):
+        models = [_rigid(k, i) for i in range(len(grooms))]
+        for g, m in zip(grooms, models):
+            g.set_root_transform(m)
+        if k < 2:
+            b.launch([DT] * len(grooms))
+        else:
+            ba.batch_step(ctx, grooms, [DT] * len(grooms))
+        _oracle_frame(states, [DT] * len(grooms), models)
+        for i, (g, s) in enumerate(zip(grooms, states)):
+            p, v = g.download()
+            assert_bitexact(p, s["pos"], "groom %d frame %d positions" % (i, k))
+            assert_bitexact(v, s["vel"], "groom %d frame %d velocities" % (i, k))
+    b.close()
