@@ -5,7 +5,7 @@
 // A batch is planned once: each groom is cut into 64-lane tiles of its launch
 // class (points per lane x lanes per strand), and the grooms are grouped by
 // class, each a span of consecutive tiles of its class's launch (one record
-// per groom: the kernel maps a tile to its groom by a binary search over the
+// per groom: the kernel maps a tile to its groom by a search over the
 // spans).  Every class has its own tile-list kernel, compiled with the register
 // budget of that class (one kernel for all classes would carry the register
 // count of the heaviest one).  A frame is [upload the per-groom descriptors

@@ -42,11 +42,11 @@ struct FtlStep {
 // One groom's share of a class's batched launch: tiles tile0, tile0 + 1, ...
 // of the class's kernel step the groom's strands, 64 / G strands a tile.  A
 // launch's spans are in tile order, and each workgroup finds its own by a
-// binary search, so a batch uploads one record per groom, not per tile.
+// search, so a batch uploads one record per groom, not per tile.
 struct FtlSpan {
   int groom;  // index into the FtlStep table
   int tile0;  // first tile of the groom in its class's launch
-  int cls;    // launch class (points per lane, lanes per strand)
+  int cls;    // launch class or wide form (points per lane, lanes per strand)
   int cost;   // relative cost of a tile, for ordering
 };
 
@@ -351,8 +351,9 @@ __device__ __forceinline__ float3 wind_blend(const WindTaps& t) {
   return r;
 }
 
-// The colliders of one step, read once per tile into scalar registers and
-// made opaque there, so the per-point collision code never reloads them.
+// The colliders a tile meets this step (those some strand of the wave can
+// reach, in order), read once per tile into scalar registers and made opaque
+// there, so the per-point collision code never reloads them.
 struct Spheres {
   float c[FTL_NCOL][3];
   float r[FTL_NCOL];
@@ -380,51 +381,54 @@ __device__ __forceinline__ T* pin_p(T* p) {
   return (T*)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo);
 }
 
-__device__ __forceinline__ Spheres load_spheres(const FtlStep& A, unsigned cmask) {
+// Packs the colliders of `mask` to the front of the struct; n: how many.
+__device__ __forceinline__ Spheres load_spheres(const FtlStep& A, unsigned mask, int& n) {
   Spheres S;
+  n = __builtin_popcount(mask);
 #pragma unroll
   for (int k = 0; k < FTL_NCOL; ++k) {
-    if (!(cmask & (1u << k))) {
-      S.c[k][0] = S.c[k][1] = S.c[k][2] = S.r[k] = S.r2[k] = 0.0f;
-      continue;
-    }
-    S.c[k][0] = pin_s(A.sph[k][0]);
-    S.c[k][1] = pin_s(A.sph[k][1]);
-    S.c[k][2] = pin_s(A.sph[k][2]);
-    S.r[k] = pin_s(A.sph[k][3]);
-    S.r2[k] = pin_s(A.r2[k]);
+    S.c[k][0] = S.c[k][1] = S.c[k][2] = S.r[k] = S.r2[k] = 0.0f;
+    if (mask == 0u) continue;
+    const int i = __builtin_ctz(mask);
+    mask &= mask - 1u;
+    S.c[k][0] = pin_s(A.sph[i][0]);
+    S.c[k][1] = pin_s(A.sph[i][1]);
+    S.c[k][2] = pin_s(A.sph[i][2]);
+    S.r[k] = pin_s(A.sph[i][3]);
+    S.r2[k] = pin_s(A.r2[i]);
   }
   return S;
 }
 
-// CollideSphere(+1, c_k, r_k, p) for the colliders of `cmask`, in order
-// (cs_simulation.glsl:129-153).  cmask is wave-uniform: the colliders some
-// strand of the wave can reach (the others cannot change any result).
-// REFLECT: also reflect u on each hit; only the last constraint iteration's
-// velocity reaches the output.
-// Test of bit k of the wave-uniform collider mask as a scalar branch.  The
-// mask is made opaque at each test: hoisted out of the iteration loop, the
-// test becomes a per-lane boolean that costs two vector instructions a use.
-__device__ __forceinline__ bool has_collider(unsigned cmask, int k) {
-  asm volatile("" : "+s"(cmask));
-  return (cmask >> k) & 1u;
+// Whether the tile meets more than k colliders, as a scalar branch: the
+// collision loops stop at the first k it does not (with the colliders packed,
+// a tile that meets one tests one branch, not four).  The count is made opaque
+// at each test: hoisted out of the iteration loop, the test becomes a per-lane
+// boolean that costs two vector instructions a use.
+__device__ __forceinline__ bool more_colliders(int n, int k) {
+  asm volatile("" : "+s"(n));
+  return k < n;
 }
 
+// CollideSphere(+1, c_k, r_k, p) for the tile's n colliders, in order
+// (cs_simulation.glsl:129-153); the colliders no strand of the wave can reach
+// cannot change any result.  REFLECT: also reflect u on each hit; only the
+// last constraint iteration's velocity reaches the output.
 template <bool REFLECT>
-__device__ __forceinline__ void collide(const Spheres& S, float3& p, float3& u, unsigned cmask) {
+__device__ __forceinline__ void collide(const Spheres& S, float3& p, float3& u, int n) {
 #pragma unroll
   for (int k = 0; k < FTL_NCOL; ++k) {
-    if (!has_collider(cmask, k)) continue;
+    if (!more_colliders(n, k)) break;
     const float3 c = f3(S.c[k][0], S.c[k][1], S.c[k][2]);
     const float3 w = sub3(p, c);
     const float dp = dot3(w, w);
     if (dp < S.r2[k]) {
       const float is = rsqrt_c(dp);
-      const float3 n = mul3(w, is);
-      p = fma3(S.r[k], n, c);
+      const float3 nrm = mul3(w, is);
+      p = fma3(S.r[k], nrm, c);
       if (REFLECT) {
-        const float d2 = 2.0f * dot3(n, u);
-        u = fma3(-d2, n, u);
+        const float d2 = 2.0f * dot3(nrm, u);
+        u = fma3(-d2, nrm, u);
       }
     }
   }
@@ -436,16 +440,22 @@ __device__ __forceinline__ void collide(const Spheres& S, float3& p, float3& u, 
 // at most r_j - |p0 - c_j| + D when D bounds the point's distance to p0, so
 // D grows by that much for each collider that can touch the strand.  A
 // collider farther than r_k + D (with a generous rounding margin) can never
-// contain a point of the strand in this step.
+// contain a point of the strand in this step.  The margin covers the
+// instruction's square root (1 ulp) and bounds lengths by sums of components:
+// the mask only has to hold every collider that could matter.
+__device__ __forceinline__ float norm1(float3 x) { return fabsf(x.x) + fabsf(x.y) + fabsf(x.z); }
 __device__ __forceinline__ unsigned reachable_colliders(const FtlStep& A, float3 p0, float L) {
   float D = L * 1.001f + 1e-4f;
-  const float a = sqrtf(dot3(p0, p0));
+  const float a = norm1(p0);
   unsigned mask = 0u;
-  for (int k = 0; k < A.ncol; ++k) {
+#pragma unroll
+  for (int k = 0; k < FTL_NCOL; ++k) {
+    if (k >= A.ncol) break;
     const float3 c = f3(A.sph[k][0], A.sph[k][1], A.sph[k][2]);
     const float r = A.sph[k][3];
-    const float dc = sqrtf(dot3(sub3(p0, c), sub3(p0, c)));
-    const float tol = 1e-4f * (a + sqrtf(dot3(c, c)) + r + D + 1.0f);
+    const float3 w = sub3(p0, c);
+    const float dc = __builtin_amdgcn_sqrtf(dot3(w, w));
+    const float tol = 1e-4f * (a + norm1(c) + r + D + 1.0f);
     if (!(dc - r > D + tol)) {  // NaN keeps the collider
       mask |= 1u << k;
       D += fmaxf(0.0f, r - dc + D) + tol;

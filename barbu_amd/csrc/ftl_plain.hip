@@ -137,8 +137,7 @@ hipError_t FTL_PASTE(ftl_launch_plain_, FTL_CLASS_ID)(const FtlStep& A, hipStrea
 // Tile-list form of the same class for batched frames: workgroup b steps the
 // tiles b, b + grid, b + 2 grid, ... of the 64-lane tiles of any grooms of
 // this class, each groom a span of consecutive tiles; a workgroup finds its
-// tile's groom by a binary search over the spans' first tiles (scalar loads,
-// a few per tile).  With grid = number of tiles (the batched default)
+// tile's groom by a search over the spans' first tiles.  With grid = number of tiles (the batched default)
 // each workgroup takes one tile and the hardware dispatcher balances the
 // load; a smaller grid makes the workgroups persistent.  (A shared atomic
 // work counter was measured 2-5x slower: every claim contends on one address
@@ -153,15 +152,7 @@ void ftl_tiles_kernel(const FtlStep* __restrict__ grooms, const FtlSpan* __restr
   __shared__ ftl_tile_impl::TileLds<CL::M, CL::G, CL::GU> sh;
   constexpr int spt = FTL_WAVE / CL::G;
   for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    // the last span whose first tile is at or before t (spans[0].tile0 == 0)
-    int lo = 0, hi = nspans - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (__builtin_amdgcn_readfirstlane(spans[mid].tile0) <= t)
-        lo = mid;
-      else
-        hi = mid - 1;
-    }
+    const int lo = ftl_tile_impl::span_of(spans, nspans, t);
     const int gi = __builtin_amdgcn_readfirstlane(spans[lo].groom);
     const int s0 = (t - __builtin_amdgcn_readfirstlane(spans[lo].tile0)) * spt;
     ftl_tile_impl::ftl_tile<CL::M, CL::G, CL::GU, NT, kLoadAhead>(grooms[gi], s0, sh);

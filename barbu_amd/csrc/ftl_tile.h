@@ -240,12 +240,13 @@ __device__ __forceinline__ void flush_velocities(float4* __restrict__ dst, int s
 // || on0).
 template <int M>
 __device__ __forceinline__ void collide_sweep(const Spheres& S, float3 (&p)[M], bool on, bool on0, int jend,
-                                              unsigned cmask) {
+                                              int n) {
 #pragma unroll
   for (int k = 0; k < FTL_NCOL; ++k) {
-    if (!has_collider(cmask, k)) continue;
+    if (!more_colliders(n, k)) break;
     float cx = S.c[k][0], cy = S.c[k][1], cz = S.c[k][2], r2 = S.r2[k];
-    asm volatile("" : "+v"(cx), "+v"(cy), "+v"(cz), "+v"(r2));
+    // (with one or two points the copies cost more than they save)
+    if constexpr (M > 2) asm volatile("" : "+v"(cx), "+v"(cy), "+v"(cz), "+v"(r2));
     const float3 c = f3(cx, cy, cz);
 #pragma unroll
     for (int j = 0; j < M; ++j) {
@@ -254,8 +255,7 @@ __device__ __forceinline__ void collide_sweep(const Spheres& S, float3 (&p)[M], 
       const float dp = dot3(w, w);
       if (on && (j > 0 || on0) && dp < r2) {
         const float is = rsqrt_c(dp);
-        const float3 n = mul3(w, is);
-        p[j] = fma3(S.r[k], n, c);
+        p[j] = fma3(S.r[k], mul3(w, is), c);
       }
     }
   }
@@ -270,7 +270,7 @@ template <int M, bool GUARD, bool FINAL, bool NT>
 __device__ __forceinline__ void sweep(const FtlStep& A, const VelArgs& V, const Spheres& S, float3 (&p)[M],
                                       const LenLds& l, int nl,
                                       const float4* __restrict__ pp, float3& last_pre, float3& clast,
-                                      float4* __restrict__ stage, int strand0, int N, int lane, unsigned cm) {
+                                      float4* __restrict__ stage, int strand0, int N, int lane, int cm) {
   constexpr int C = Tile<M, 1, GUARD>::C;
   // Opaque per sweep: keeps the compiler from hoisting sigma * l[j] out of the
   // iteration loop into M extra registers (one multiply per point instead).
@@ -339,7 +339,7 @@ __device__ __forceinline__ float from_prev_lane(float x) {
 template <int M, int G, bool GUARD, bool PARK, int PL, int NQ>
 __device__ __forceinline__ void sweep_pipe(const Spheres& S, float3 (&p)[M], const LenRegs<M>& l, float3& lead, int g,
                                            bool active, bool fin, float* park, float3 (&q)[NQ],
-                                           unsigned cm) {
+                                           int cm) {
   if (PARK && fin) {
 #pragma unroll
     for (int j = 0; j < M; ++j) {
@@ -521,7 +521,7 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
   }
 
   // ---- colliders the wave can reach this step ----------------------------
-  unsigned cm;
+  unsigned reach;
   {
     float L = 0.0f;
 #pragma unroll
@@ -537,11 +537,13 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
     }
     const unsigned mine = valid ? reachable_colliders(A, root, L) : 0u;
     unsigned any = 0u;
-    for (int k = 0; k < A.ncol; ++k)
+#pragma unroll
+    for (int k = 0; k < FTL_NCOL; ++k)
       if (__ballot((mine >> k) & 1u) != 0ull) any |= 1u << k;
-    cm = __builtin_amdgcn_readfirstlane(any);
+    reach = __builtin_amdgcn_readfirstlane(any);
   }
-  const Spheres S = load_spheres(A, cm);
+  int cm;  // colliders the tile meets
+  const Spheres S = load_spheres(A, reach, cm);
   const VelArgs V = vel_args(A);
 
   // ---- constraints ------------------------------------------------------
@@ -655,6 +657,24 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
   // every writer stores the same value.
   if (b != 0ull && lane == (int)(__ffsll((long long)b) - 1))
     __hip_atomic_store(A.status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The span of tile t of a launch: the last whose first tile is at or before t
+// (spans[0].tile0 == 0).  The wave's lanes read 64 first tiles at a time, so a
+// search over n spans makes log64(n) dependent loads (a scalar binary search
+// makes log2(n), each a round trip at the head of the tile).
+__device__ __forceinline__ int span_of(const FtlSpan* __restrict__ spans, int nspans, int t) {
+  const int lane = (int)threadIdx.x & (FTL_WAVE - 1);
+  int lo = 0, n = nspans;
+  for (;;) {
+    const int stride = (n + FTL_WAVE - 1) / FTL_WAVE;
+    const int i = lane * stride;
+    const bool before = i < n && spans[lo + min(i, n - 1)].tile0 <= t;
+    const int k = max((int)__builtin_popcountll(__ballot(before)) - 1, 0);
+    lo += k * stride;
+    if (stride == 1) return lo;
+    n = min(stride, n - k * stride);
+  }
 }
 
 }  // namespace ftl_tile_impl

@@ -158,7 +158,7 @@ __device__ __forceinline__ void ftl_wide_tile(const FtlStep& A, int strand0, flo
     for (int j = 0; j < M; ++j) l.set(j, sg * l.get(j));
   }
 
-  unsigned cm;
+  unsigned reach;
   {
     float L = 0.0f;
 #pragma unroll
@@ -167,11 +167,13 @@ __device__ __forceinline__ void ftl_wide_tile(const FtlStep& A, int strand0, flo
     L = lanes_sum<G>(L);
     const unsigned mine = valid ? reachable_colliders(A, p0, L) : 0u;
     unsigned any = 0u;
-    for (int k = 0; k < A.ncol; ++k)
+#pragma unroll
+    for (int k = 0; k < FTL_NCOL; ++k)
       if (__ballot((mine >> k) & 1u) != 0ull) any |= 1u << k;
-    cm = __builtin_amdgcn_readfirstlane(any);
+    reach = __builtin_amdgcn_readfirstlane(any);
   }
-  const Spheres S = load_spheres(A, cm);
+  int cm;  // colliders the tile meets
+  const Spheres S = load_spheres(A, reach, cm);
   const VelArgs V = vel_args(A);
 
   const int K = A.iterations;

@@ -18,19 +18,6 @@ using namespace ftl_wide_impl;
 #define FTL_PASTE2(a, b) a##b
 #define FTL_PASTE(a, b) FTL_PASTE2(a, b)
 
-// The span of tile t (as in ftl_tiles_kernel).
-__device__ __forceinline__ int span_of(const FtlSpan* __restrict__ spans, int nspans, int t) {
-  int lo = 0, hi = nspans - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (__builtin_amdgcn_readfirstlane(spans[mid].tile0) <= t)
-      lo = mid;
-    else
-      hi = mid - 1;
-  }
-  return lo;
-}
-
 #if FTL_WIDE_LANES > 0
 
 template <int M, int G, bool NT>
