@@ -298,9 +298,10 @@ ftl_status ftl_batch_step(ftl_ctx* ctx, ftl_groom* const* grooms, int n, const f
    be read by anything else. */
 ftl_status ftl_batch_step_noalloc(ftl_ctx* ctx, ftl_groom* const* grooms, int n, const float* dt, void* stream);
 
-/* A fixed set of grooms stepped as one frame, captured once into a HIP graph
-   (parameter upload + one kernel per launch class) and replayed by
-   ftl_batch_launch. */
+/* A fixed set of grooms stepped as one frame, planned once: a HIP graph
+   (parameter upload + one kernel per launch class) replayed by
+   ftl_batch_launch, or, when one kernel steps them all, the upload and that
+   kernel. */
 ftl_status ftl_batch_create(ftl_ctx* ctx, ftl_groom* const* grooms, int n, ftl_batch** out);
 void ftl_batch_destroy(ftl_batch* b);
 /* One frame: per-groom dt (n values).  Colliders, transforms, params and time
