@@ -14,7 +14,8 @@
 // At the settings where it measured faster (the reference's among them), a
 // second form batches patches per wave instead: their guides are loaded once
 // into LDS and each lane stores several vertices' blends
-// (ftl_expand_batched_kernel).
+// (ftl_expand_batched_kernel); a third goes by pages of the output
+// (ftl_expand_page_kernel).
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -60,10 +61,12 @@ __device__ __forceinline__ float hmix(const Basis& h, float p0, float p1, float 
 
 // smoothstep2(0, 1, j / N + u / N) (tes_stream_hair.glsl:64-65,
 // inc_maths.glsl:263-266); maprange(0, 1, x) is clamp(x, 0, 1).
-__device__ __forceinline__ float rel_pos(int j, float u, float n) {
-  const float r = (float)j / n + u / n;
+__device__ __forceinline__ float rel_step(float r) {
   const float t = fminf(fmaxf(r, 0.0f), 1.0f);
   return ((t * t) * t) * (10.0f + t * (-15.0f + 6.0f * t));
+}
+__device__ __forceinline__ float rel_pos(int j, float u, float n) {
+  return rel_step((float)j / n + u / n);
 }
 
 // Barycentric weights of (instance, line): the random entry the evaluation
@@ -292,6 +295,140 @@ __global__ __launch_bounds__(64) void ftl_expand_batched_kernel(ExpandArgs A) {
     expand_batch<NV, NC, true, B>(A, gd, wts, b, npatch, lane);
 }
 
+// The same pass by pages of the output.  For one instance the capture of
+// consecutive patches is one contiguous run of float4s, `run` = nlines * 2 nsub
+// of them a patch, so a workgroup (one wave) takes 256 consecutive vertices
+// (4 KB) of every instance: four rows of 64, each stored by one instruction as
+// 1 KB.  It loads the guides of the patches those vertices lie in (two round
+// trips, as ftl_expand_batched_kernel), tabulates the basis, and each lane
+// evaluates its four vertices once and then blends and stores them instance by
+// instance.  Same operations per output vertex as ftl_expand_kernel.
+//
+// The store pattern is what bounds a pass beyond the Infinity Cache: probes of
+// stores alone, 917 MB, ran 135 us with one 4 KB page a workgroup, 143 with a
+// page in each of three instances, 152 with the other forms' 512-byte runs (a
+// page then belongs to one XCD's L2; a page dealt out to several took 192 for
+// 1.07 GB against 159).  The per-vertex form's runs of 2 nsub vertices start at
+// odd multiples of 32 bytes when nsub is odd, and half-written 64-byte sectors
+// cost it more: 3 x 2 x 15 216 against 150 us, 4 x 3 x 7 157 against 142.
+constexpr int kPage = 256, kPageRows = kPage / 64;
+
+// Patches a page of 256 vertices can touch.
+constexpr int page_patches(int run) { return (kPage - 1 + run - 1) / run + 1; }
+
+// ONE: one line per patch.
+template <bool ONE>
+__global__ __launch_bounds__(64) void ftl_expand_page_kernel(ExpandArgs A, long long total) {
+  extern __shared__ float4 sm[];
+  const int nlines = ONE ? 1 : A.nlines, nv = 2 * A.nsub;
+  const int run = nlines * nv, nc = A.ninst * nlines;
+  const int np = page_patches(run);
+  float4* wts = sm;                      // [nc] weights of (instance, line)
+  float4* hb = wts + nc;                 // [nv] Hermite basis at vertex v
+  float4* gd = hb + nv;                  // [np * kGuideF4] guides, tangents scaled
+  int4* td = (int4*)(gd + np * kGuideF4);  // [np] triangles
+  float* ju = (float*)(td + np);         // [np] j / N of the patch's segment, then [nv] u / N
+  float* uu = ju + np;
+  const int lane = (int)threadIdx.x;
+  const int nseg = A.nseg;
+  const long long base = (long long)blockIdx.x * kPage;
+  const int first = (int)(base / run);  // the page's first patch, and the vertex of it the page starts at
+  const int r0 = (int)(base - (long long)first * run);
+  const int last = A.ntris * nseg - 1;
+  const float fpts = (float)A.npoints, scale = A.scale;
+  for (int i = lane; i < np; i += 64) {
+    const int patch = min(first + i, last);
+    td[i] = A.tris[patch / nseg];
+    ju[i] = (float)(patch % nseg) / fpts;
+  }
+  for (int c = lane; c < nc; c += 64) {
+    const float3 bw = bary(A.rnd, c / nlines, c % nlines, nlines);
+    wts[c] = make_float4(bw.x, bw.y, bw.z, 0.0f);
+  }
+  for (int v = lane; v < nv; v += 64) {
+    const float u = (float)((v >> 1) + (v & 1)) / (float)(nv / 2);
+    const Basis h = basis(u);
+    hb[v] = make_float4(h.h0, h.h1, h.h2, h.h3);
+    uu[v] = u / fpts;
+  }
+  expand_sync();
+  for (int e = lane; e < np * kGuideF4; e += 64) {
+    const int i = e / kGuideF4, k = (e % kGuideF4) / 4, w = e % 4;
+    const int4 tv = td[i];
+    const int root = k == 0 ? tv.x : (k == 1 ? tv.y : tv.z);
+    const size_t at = (size_t)root * A.npoints + min(first + i, last) % nseg + (w & 1);
+    float4 q = (w >> 1) ? A.tan[at] : A.pos[at];
+    // tangent * uScaleFactor (tcs_stream_hair.glsl:41)
+    if (w >> 1) q = make_float4(q.x * scale, q.y * scale, q.z * scale, 0.0f);
+    gd[e] = q;
+  }
+  expand_sync();
+  float3 g[kPageRows][3];
+  float w[kPageRows];
+  int line[kPageRows];
+#pragma unroll
+  for (int s = 0; s < kPageRows; ++s) {
+    const int o = r0 + 64 * s + lane;
+    const int i = o / run, q = o - i * run;
+    line[s] = ONE ? 0 : q / nv;
+    const int v = q - line[s] * nv;
+    const float4* G = gd + i * kGuideF4;
+    const float4 hv = hb[v];
+    const Basis h{hv.x, hv.y, hv.z, hv.w};
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const float4 p0 = G[4 * k + 0], p1 = G[4 * k + 1], t0 = G[4 * k + 2], t1 = G[4 * k + 3];
+      g[s][k] = f3(hmix(h, p0.x, p1.x, t0.x, t1.x), hmix(h, p0.y, p1.y, t0.y, t1.y), hmix(h, p0.z, p1.z, t0.z, t1.z));
+    }
+    w[s] = rel_step(ju[i] + uu[v]);
+  }
+  float4* __restrict__ out = A.out + base + lane;
+  const bool whole = base + kPage <= total;
+  for (int inst = 0; inst < A.ninst; ++inst, out += total) {
+    float4 o[kPageRows];
+#pragma unroll
+    for (int s = 0; s < kPageRows; ++s) {
+      const float4 c = wts[inst * nlines + line[s]];
+      o[s] = make_float4(__builtin_fmaf(c.z, g[s][2].x, __builtin_fmaf(c.y, g[s][1].x, c.x * g[s][0].x)),
+                         __builtin_fmaf(c.z, g[s][2].y, __builtin_fmaf(c.y, g[s][1].y, c.x * g[s][0].y)),
+                         __builtin_fmaf(c.z, g[s][2].z, __builtin_fmaf(c.y, g[s][1].z, c.x * g[s][0].z)), w[s]);
+    }
+#pragma unroll
+    for (int s = 0; s < kPageRows; ++s)
+      if (whole || base + 64 * s + lane < total) out[64 * s] = o[s];
+  }
+}
+
+// Launches the page form where it measured faster than ftl_expand_kernel
+// (page against per-vertex, 4-point guides; the batched form's settings are
+// taken before):
+// * one line and at most two instances, 6 or more subsegments: the per-vertex
+//   form makes 13 loads for one or two stores a thread (1 x 1 x 7 27 against
+//   34 us, 1 x 1 x 15 46, 65; 2 x 1 x 10 34, 50; 1 x 1 x 4 26, 21);
+// * outputs above 384 MB (the same line as the step's streaming stores: an
+//   output the Infinity Cache holds merges there) with two or more instances
+//   and 5 or more subsegments, odd (3 x 2 x 7 82 against 121 us, 8 x 4 x 15
+//   130, 168; but 8 x 1 x 13 145, 135) or with at most 9 blends (3 x 2 x 10
+//   106, 143; 6 x 1 x 14 115, 141; but 6 x 2 x 14 115, 109).
+bool launch_expand_page_if_faster(const ExpandArgs& A, int nc, hipStream_t stream) {
+  const int nv = 2 * A.nsub, run = nv * A.nlines, np = page_patches(run);
+  const long long total = (long long)A.ntris * A.nseg * run;
+  if (A.nlines == 1 && A.ninst <= 2) {
+    if (A.nsub < 6) return false;
+  } else {
+    if (total * A.ninst * (long long)sizeof(float4) <= (384ll << 20) || A.ninst < 2 || A.nsub < 5) return false;
+    if (A.nsub % 2 == 1 ? A.nlines == 1 && A.ninst > 6 : nc > 9) return false;
+  }
+  const size_t lds = ((size_t)nc + nv + (size_t)np * kGuideF4 + np) * sizeof(float4) + (size_t)(np + nv) * sizeof(float);
+  if (lds > 64 * 1024) return false;
+  const dim3 grid((unsigned)((total + kPage - 1) / kPage)), block(64);
+  if (A.nlines == 1)
+    hipLaunchKernelGGL(ftl_expand_page_kernel<true>, grid, block, lds, stream, A, total);
+  else
+    hipLaunchKernelGGL(ftl_expand_page_kernel<false>, grid, block, lds, stream, A, total);
+  return true;
+}
+
 // The batched pass at nsub = NSUB subsegments (nc blends).
 template <int NSUB>
 void launch_expand_batched(const ExpandArgs& A, int nc, hipStream_t stream) {
@@ -493,7 +630,8 @@ extern "C" ftl_status ftl_expand_run(ftl_expand* e, const ftl_expand_params* p, 
   A.scale = p->tangent_scale;
   const size_t lds = (size_t)p->ninstances * p->nlines * sizeof(float4);
   const int nc = p->ninstances * p->nlines;
-  if (!launch_expand_batched_if_faster(A, p->nsubsegments, nc, (hipStream_t)stream)) {
+  if (!launch_expand_batched_if_faster(A, p->nsubsegments, nc, (hipStream_t)stream) &&
+      !launch_expand_page_if_faster(A, nc, (hipStream_t)stream)) {
     const int blocks = (int)((nthreads + 255) / 256);
     hipLaunchKernelGGL(ftl_expand_kernel, dim3(blocks), dim3(256), lds, (hipStream_t)stream, A);
   }
