@@ -6,23 +6,24 @@
 
 // X(id, points per lane, lanes per strand, guarded, waves per SIMD targeted
 // by the register allocator: the highest at which neither the plain nor the
-// tile-list kernel of the class spills, points per lane of a load/store
+// tile-list kernel of the class spills (12 and 14 spill three and one), points
+// per lane of a load/store
 // chunk: 8 float4 make one 128-byte line, so each line of the groom is read
 // by one request; 4 halves the LDS stage where a bigger one would cost
 // occupancy, at the price of two requests per line)
 #define FTL_CLASSES(X)        \
   X(0, 4, 1, false, 8, 4)     \
-  X(1, 8, 1, false, 6, 4)     \
+  X(1, 8, 1, false, 5, 4)     \
   X(2, 16, 1, false, 4, 4)    \
   X(3, 32, 1, false, 2, 8)    \
   X(4, 8, 2, false, 4, 8)     \
-  X(5, 16, 2, false, 2, 8)    \
+  X(5, 16, 2, false, 4, 8)    \
   X(6, 32, 2, false, 2, 8)    \
   X(7, 4, 4, false, 6, 4)     \
   X(8, 8, 4, false, 4, 8)     \
-  X(9, 16, 4, false, 3, 8)    \
+  X(9, 16, 4, false, 4, 8)    \
   X(10, 4, 1, true, 6, 4)     \
-  X(11, 8, 1, true, 6, 4)     \
+  X(11, 8, 1, true, 5, 4)     \
   X(12, 16, 1, true, 4, 4)    \
   X(13, 32, 1, true, 2, 4)    \
   X(14, 64, 1, true, 1, 8)    \

@@ -42,22 +42,6 @@ constexpr int kWavesPerEu = CL::W;
 // waves per SIMD (their register budget), FTL_LOAD_AHEAD for the others.
 constexpr int kLoadAhead = kWavesPerEu >= 6 ? 1 : FTL_LOAD_AHEAD;
 
-template <bool NT>
-__global__ __launch_bounds__(FTL_WAVE) __attribute__((amdgpu_waves_per_eu(kWavesPerEu, 8)))
-void ftl_plain_kernel(FtlStep arg) {
-  (void)arg;
-  // The descriptor is read in place from the kernel-argument segment (scalar
-  // loads, runtime-indexed collider array) instead of through a private copy
-  // of the by-value argument.
-#if defined(__HIP_DEVICE_COMPILE__)
-  const FtlStep& A = *(const FtlStep*)__builtin_amdgcn_kernarg_segment_ptr();
-#else
-  const FtlStep& A = arg;
-#endif
-  __shared__ ftl_tile_impl::TileLds<CL::M, CL::G, CL::GU> sh;
-  ftl_tile_impl::ftl_tile<CL::M, CL::G, CL::GU, NT, kLoadAhead>(A, blockIdx.x * (FTL_WAVE / CL::G), sh);
-}
-
 // With wind: four tiles (waves) per workgroup share one LDS copy of the wind
 // lattice, so the load phase's gathers are LDS reads (their waits are
 // independent of the HBM row loads in flight) instead of global gathers.
@@ -81,6 +65,26 @@ constexpr size_t kWindGroupLds =
 constexpr int kWindGroupsPerCu = (kWavesPerEu == 2 ? 8 : 16) / kWindWaves;
 constexpr bool kWindLds = (kWavesPerEu == 4 || kWavesPerEu == 2) && kWindGroupsPerCu * kWindGroupLds <= 160 * 1024;
 
+// A class with the LDS form never runs its plain kernel with wind.
+constexpr int kPlainWind = kWindLds && FTL_WIND_LDS ? ftl_tile_impl::kWindOff : ftl_tile_impl::kWindAny;
+
+template <bool NT>
+__global__ __launch_bounds__(FTL_WAVE) __attribute__((amdgpu_waves_per_eu(kWavesPerEu, 8)))
+void ftl_plain_kernel(FtlStep arg) {
+  (void)arg;
+  // The descriptor is read in place from the kernel-argument segment (scalar
+  // loads, runtime-indexed collider array) instead of through a private copy
+  // of the by-value argument.
+#if defined(__HIP_DEVICE_COMPILE__)
+  const FtlStep& A = *(const FtlStep*)__builtin_amdgcn_kernarg_segment_ptr();
+#else
+  const FtlStep& A = arg;
+#endif
+  __shared__ ftl_tile_impl::TileLds<CL::M, CL::G, CL::GU> sh;
+  ftl_tile_impl::ftl_tile<CL::M, CL::G, CL::GU, NT, kPlainWind, kLoadAhead>(
+      A, blockIdx.x * (FTL_WAVE / CL::G), sh);
+}
+
 template <bool NT>
 __global__ __launch_bounds__(FTL_WAVE * kWindWaves) __attribute__((amdgpu_waves_per_eu(kWavesPerEu, 8)))
 void ftl_plain_wind_kernel(FtlStep arg) {
@@ -102,7 +106,8 @@ void ftl_plain_wind_kernel(FtlStep arg) {
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / FTL_WAVE);
     const int t = (int)blockIdx.x * kWindWaves + w;
     if (t < ntiles)
-      ftl_tile_impl::ftl_tile<CL::M, CL::G, CL::GU, NT, kLoadAhead, kWindHalf ? 2 : 1>(A, t * spt, sh[w], lattice);
+      ftl_tile_impl::ftl_tile<CL::M, CL::G, CL::GU, NT, ftl_tile_impl::kWindOn, kLoadAhead, kWindHalf ? 2 : 1>(
+          A, t * spt, sh[w], lattice);
   }
 }
 
@@ -155,7 +160,7 @@ void ftl_tiles_kernel(const FtlStep* __restrict__ grooms, const FtlSpan* __restr
     const int lo = ftl_tile_impl::span_of(spans, nspans, t);
     const int gi = __builtin_amdgcn_readfirstlane(spans[lo].groom);
     const int s0 = (t - __builtin_amdgcn_readfirstlane(spans[lo].tile0)) * spt;
-    ftl_tile_impl::ftl_tile<CL::M, CL::G, CL::GU, NT, kLoadAhead>(grooms[gi], s0, sh);
+    ftl_tile_impl::ftl_tile<CL::M, CL::G, CL::GU, NT, ftl_tile_impl::kWindAny, kLoadAhead>(grooms[gi], s0, sh);
   }
 }
 

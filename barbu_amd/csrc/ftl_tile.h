@@ -43,9 +43,6 @@
 #ifndef FTL_NO_DFTL
 #define FTL_NO_DFTL 0
 #endif
-#ifndef FTL_WIND_ON
-#define FTL_WIND_ON 1
-#endif
 // Rows of the load phase whose loads are in flight ahead of the row being
 // integrated (default of the forms with at most four waves per SIMD).
 #ifndef FTL_LOAD_AHEAD
@@ -163,69 +160,90 @@ __device__ __forceinline__ void tile_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Writes chunk c of the tile (C points per lane, staged in LDS) to dst in
-// the coalesced order of the load.  Called by the whole wave.  NT: the
-// stores carry the non-temporal hint (launches whose state is too large for
-// the next step to find any of it in the caches).
-typedef float ftl_nt_f4 __attribute__((ext_vector_type(4)));
-template <int M, int G, bool GUARD, bool NT>
-__device__ __forceinline__ void flush_chunk(float4* __restrict__ dst, int strand0, int nstr, int N, int c,
-                                            const float4* __restrict__ stage, int lane) {
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef unsigned u4v __attribute__((ext_vector_type(4)));
+typedef __amdgpu_buffer_rsrc_t BufferRsrc;
+
+// Raw buffer of `bytes` from p: dword offsets at or past its end load 0 and
+// store nothing.  A tile's rows go through one whose end is the tile's, so a
+// partial tile needs no clamp and no store mask, and a row's address is the
+// lane's first plus a constant.
+__device__ __forceinline__ BufferRsrc buffer_of(const void* p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)bytes, 0x00027000);
+}
+__device__ __forceinline__ float4 buffer_load4(BufferRsrc r, unsigned byte) {
+  const f4v t = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(r, (int)byte, 0, 0));
+  return make_float4(t.x, t.y, t.z, t.w);
+}
+template <bool NT>
+__device__ __forceinline__ void buffer_store4(BufferRsrc r, unsigned byte, float4 v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, f4v{v.x, v.y, v.z, v.w}), r, (int)byte, 0, NT ? 2 : 0);
+}
+
+// Byte offset, within the tile, of the lane's point in row 0 of chunk c (row k
+// is RS * N points further).  Row k of a chunk holds, in lane ln, point ln % C
+// of the chunk of owner lane r = k * (64 / C) + ln / C.  64 / C is a multiple
+// of G and of C, so from row to row only the strand moves, by RS = 64 / C / G,
+// and the stage slot by 64.  GUARD: points past the strand read its last one
+// (CLAMP) or address past the tile, which stores nothing.
+template <int M, int G, bool GUARD, bool CLAMP>
+__device__ __forceinline__ unsigned row_offset(int N, int c, int lane) {
   constexpr int C = Tile<M, G, GUARD>::C;
-  // Row k holds, in lane ln, point ln % C of the chunk of owner lane
-  // r = k * (64 / C) + ln / C.  64 / C is a multiple of G and of C, so from row
-  // to row only the strand moves, by RS strands, and the LDS slot by 64: the
-  // lane's address and slot are formed once and stepped.
   static_assert((FTL_WAVE / C) % G == 0 && (FTL_WAVE / C) % C == 0, "rows of a chunk hold whole strands");
+  const int r0 = lane / C, j = lane % C;
+  int cp = (r0 % G) * M + c * C + j;
+  if (GUARD && CLAMP) cp = min(cp, N - 1);
+  const unsigned off = 16u * (unsigned)((r0 / G) * N + cp);
+  return GUARD && !CLAMP && cp >= N ? 0x80000000u : off;
+}
+
+// Rows of a flush read from the stage together: all eight at once would need
+// 32 registers beside the strand's.
+#ifndef FTL_FLUSH_ROWS
+#define FTL_FLUSH_ROWS 2
+#endif
+constexpr int kFlushRows = FTL_FLUSH_ROWS;
+
+// Writes chunk c of the tile (C points per lane, staged in LDS) to dst in the
+// coalesced order of the load.  Called by the whole wave.  NT: the stores carry
+// the non-temporal hint (launches whose state is too large for the next step
+// to find any of it in the caches).
+template <int M, int G, bool GUARD, bool NT>
+__device__ __forceinline__ void flush_chunk(BufferRsrc dst, int N, int c, const float4* __restrict__ stage, int lane) {
+  constexpr int C = Tile<M, G, GUARD>::C;
   constexpr int RS = FTL_WAVE / C / G;
   // Recomputed here (opaque lane): keeping the load phase's addresses alive
   // until the stores would cost registers for the whole step.
   int ln = lane;
   asm volatile("" : "+v"(ln));
-  const int r0 = ln / C, j = ln % C;
-  const int s0 = strand0 + r0 / G;
-  const int cp = (r0 % G) * M + c * C + j;
-  const bool mine = !GUARD || cp < N;
-  float4* __restrict__ d0 = dst + ((size_t)s0 * N + cp);
-  const float4* __restrict__ t0 = stage + slot<C>(r0, j);
+  const unsigned off = row_offset<M, G, GUARD, false>(N, c, ln);
+  const float4* __restrict__ t0 = stage + slot<C>(ln / C, ln % C);
   tile_sync();
 #pragma unroll
-  for (int k = 0; k < C; ++k)
-    if (mine && s0 + k * RS < nstr) {
-      const float4 t = t0[k * FTL_WAVE];
-      if constexpr (NT)
-        __builtin_nontemporal_store(ftl_nt_f4{t.x, t.y, t.z, t.w}, (ftl_nt_f4*)&d0[(size_t)(k * RS) * N]);
-      else
-        d0[(size_t)(k * RS) * N] = t;
-    }
+  for (int k = 0; k < C; ++k) {
+    buffer_store4<NT>(dst, off + 16u * (unsigned)(k * RS * N), t0[k * FTL_WAVE]);
+    if (k % kFlushRows == kFlushRows - 1) __builtin_amdgcn_sched_barrier(0);
+  }
   tile_sync();
 }
 
 // The same for velocities, staged as three floats per point (park_slot).
 template <int M, int G, bool GUARD, bool NT>
-__device__ __forceinline__ void flush_velocities(float4* __restrict__ dst, int strand0, int nstr, int N, int c,
-                                                 const float* stage, int lane) {
+__device__ __forceinline__ void flush_velocities(BufferRsrc dst, int N, int c, const float* stage, int lane) {
   constexpr int C = Tile<M, G, GUARD>::C;
   constexpr int RS = FTL_WAVE / C / G;
   int ln = lane;
   asm volatile("" : "+v"(ln));
-  const int r0 = ln / C, j = ln % C;
-  const int s0 = strand0 + r0 / G;
-  const int cp = (r0 % G) * M + c * C + j;
-  const bool mine = !GUARD || cp < N;
-  float4* __restrict__ d0 = dst + ((size_t)s0 * N + cp);
-  const float* t0 = stage + park_slot(j, 0, r0);
+  const unsigned off = row_offset<M, G, GUARD, false>(N, c, ln);
+  const float* t0 = stage + park_slot(ln % C, 0, ln / C);
   tile_sync();
 #pragma unroll
-  for (int k = 0; k < C; ++k)
-    if (mine && s0 + k * RS < nstr) {
-      const float* t = t0 + k * (FTL_WAVE / C);
-      const float x = t[0], y = t[FTL_WAVE + 1], z = t[2 * (FTL_WAVE + 1)];
-      if constexpr (NT)
-        __builtin_nontemporal_store(ftl_nt_f4{x, y, z, 0.0f}, (ftl_nt_f4*)&d0[(size_t)(k * RS) * N]);
-      else
-        d0[(size_t)(k * RS) * N] = make_float4(x, y, z, 0.0f);
-    }
+  for (int k = 0; k < C; ++k) {
+    const float* t = t0 + k * (FTL_WAVE / C);
+    buffer_store4<NT>(dst, off + 16u * (unsigned)(k * RS * N),
+                      make_float4(t[0], t[FTL_WAVE + 1], t[2 * (FTL_WAVE + 1)], 0.0f));
+    if (k % kFlushRows == kFlushRows - 1) __builtin_amdgcn_sched_barrier(0);
+  }
   tile_sync();
 }
 
@@ -270,7 +288,7 @@ template <int M, bool GUARD, bool FINAL, bool NT>
 __device__ __forceinline__ void sweep(const FtlStep& A, const VelArgs& V, const Spheres& S, float3 (&p)[M],
                                       const LenLds& l, int nl,
                                       const float4* __restrict__ pp, float3& last_pre, float3& clast,
-                                      float4* __restrict__ stage, int strand0, int N, int lane, int cm) {
+                                      float4* __restrict__ stage, BufferRsrc bvel, int N, int lane, int cm) {
   constexpr int C = Tile<M, 1, GUARD>::C;
   // Opaque per sweep: keeps the compiler from hoisting sigma * l[j] out of the
   // iteration loop into M extra registers (one multiply per point instead).
@@ -302,7 +320,7 @@ __device__ __forceinline__ void sweep(const FtlStep& A, const VelArgs& V, const 
         p[m] = pm;
         const float3 v = out_velocity(V, pp, m, pm, u);
         stage[slot<C>(lane, m % C)] = make_float4(v.x, v.y, v.z, 0.0f);
-        if (m % C == C - 1) flush_chunk<M, 1, GUARD, NT>(A.vel, strand0, A.nstrands, N, m / C, stage, lane);
+        if (m % C == C - 1) flush_chunk<M, 1, GUARD, NT>(bvel, N, m / C, stage, lane);
       }
       if (GUARD ? (j == nl - 1) : (j == M - 1)) {
         clast = c;
@@ -389,7 +407,9 @@ struct TileLds : TileLens<M, G == 1> {
 // LW: where the wind gathers read the groom's wind lattice: 0 global memory,
 // 1 wl = the whole lattice copied to LDS by the workgroup, 2 wl = its half
 // lattice (first float4 of each node) in LDS.
-template <int M, int G, bool GUARD, bool NT, int PD_ = FTL_LOAD_AHEAD, int LW = 0>
+// WIND: whether the launch has wind, where the kernel knows.
+enum { kWindOff = 0, kWindOn = 1, kWindAny = 2 };
+template <int M, int G, bool GUARD, bool NT, int WIND, int PD_ = FTL_LOAD_AHEAD, int LW = 0>
 __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<M, G, GUARD>& sh,
                                          const float4* wl = nullptr) {
   float4* __restrict__ stage = sh.stage;
@@ -420,11 +440,10 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
   // in the coalesced order (64 consecutive float4 per instruction).  Loads run
   // PD rows ahead of the row being integrated, and a row's wind gathers are
   // issued before the loads of row i + PD: loads return in issue order, so
-  // waiting for the gathers never waits for HBM.  Loads are clamped into the
-  // groom (out-of-range lanes read valid data that is never stored).
+  // waiting for the gathers never waits for HBM.  (Lanes past a partial tile
+  // read zeros, and what they compute is never stored.)
   const float dt = pin_s(A.dt), dt2 = pin_s(A.dt2);
   const float3 F0 = f3(pin_s(A.force[0]), pin_s(A.force[1]), pin_s(A.force[2]));
-  const bool wind = FTL_WIND_ON && A.wind_grid;
   WindArgs W;
   W.T = (GlobalFloat4*)pin_p(A.wind);
   W.freq = pin_s(A.wind_freq);
@@ -439,73 +458,86 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
   if (owns_root && A.rmode != kRootModel) rsrc = root_source(A, min(strand, slast));
   __builtin_amdgcn_sched_barrier(0);
 
-  constexpr int PD = PD_ < M ? PD_ : M;
-  float4 xr[PD + 1], vr[PD + 1];
-  auto row_index = [&](int i) -> size_t {
-    const int q = (i % C) * FTL_WAVE + lane;
-    const int r = q / C;
-    const int s = min(strand0 + r / G, slast);
-    int cp = (r % G) * M + (i / C) * C + (q % C);
-    if (GUARD) cp = min(cp, N - 1);
-    return (size_t)s * N + cp;
-  };
-  auto load_row = [&](int i) {
-    const size_t idx = row_index(i);
-    xr[i % (PD + 1)] = A.pos[idx];
-    vr[i % (PD + 1)] = A.vel[idx];
-  };
-#pragma unroll
-  for (int i = 0; i < PD; ++i) load_row(i);
+  const size_t at = (size_t)strand0 * N;
+  const unsigned bytes = 16u * (unsigned)(min(Tile<M, G, GUARD>::SPT, nstr - strand0) * N);
+  const BufferRsrc bpos = buffer_of(A.pos + at, bytes), bvel = buffer_of(A.vel + at, bytes);
   float3 u0 = f3(0.f, 0.f, 0.f);
+  // With and without wind are two copies of the phase, so that neither tests
+  // it row by row.
+  auto load_phase = [&](auto wind_on) {
+    constexpr bool wind = decltype(wind_on)::value;
+    constexpr int RS = FTL_WAVE / C / G;
+    // (the global gathers' taps leave the registers for two rows)
+    constexpr int PD = wind && LW == 0 && PD_ > 2 ? 2 : PD_ < M ? PD_ : M;
+    float4 xr[PD + 1], vr[PD + 1];
+    const int r0 = lane / C;
+    float4* const row_slot = stage + slot<C>(r0, lane % C);
+    const bool root_row = r0 % G == 0 && lane % C == 0;  // in the rows of chunk 0
+    const unsigned off0 = row_offset<M, G, GUARD, true>(N, 0, lane);
+    auto load_row = [&](int i) {
+      const unsigned first = GUARD ? row_offset<M, G, GUARD, true>(N, i / C, lane) : off0 + 16u * (i / C * C);
+      const unsigned off = first + 16u * (unsigned)(i % C * RS * N);
+      xr[i % (PD + 1)] = buffer_load4(bpos, off);
+      vr[i % (PD + 1)] = buffer_load4(bvel, off);
+    };
 #pragma unroll
-  for (int i = 0; i < M; ++i) {
-    const int c = i / C;
-    const int q = (i % C) * FTL_WAVE + lane;
-    const int r = q / C;
-    const int j = q % C;
-    const int cp = (r % G) * M + c * C + j;
-    const float4 x = xr[i % (PD + 1)], v = vr[i % (PD + 1)];
-    WindTaps wt;
-    if (wind) {
-      if constexpr (LW == 2)
-        wt = wind_fetch_half(wl, W, f3(x.x, x.y, x.z));
-      else if constexpr (LW == 1)
-        wt = wind_fetch_from(wl, W, f3(x.x, x.y, x.z));
-      else
-        wt = wind_fetch(W, f3(x.x, x.y, x.z));
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    if (i + PD < M) load_row(i + PD);
-    __builtin_amdgcn_sched_barrier(0);
-    float3 F = F0;
-    if (wind) {
-      const float3 w = wind_blend(wt);
-      F = f3(F0.x + w.x, F0.y + w.y, F0.z + w.z);
-    }
-    float3 pr = f3(__builtin_fmaf(dt2, F.x, __builtin_fmaf(dt, v.x, x.x)),
-                   __builtin_fmaf(dt2, F.y, __builtin_fmaf(dt, v.y, x.y)),
-                   __builtin_fmaf(dt2, F.z, __builtin_fmaf(dt, v.z, x.z)));
-    if (cp == 0) pr = f3(x.x, x.y, x.z);
-    stage[slot<C>(r, j)] = make_float4(pr.x, pr.y, pr.z, x.w);
-    __builtin_amdgcn_sched_barrier(0);
-    if (i % C == C - 1) {
-      tile_sync();
+    for (int i = 0; i < PD; ++i) load_row(i);
 #pragma unroll
-      for (int k = 0; k < C; ++k) {
-        const float4 t = stage[slot<C>(lane, k)];
-        p[c * C + k] = f3(t.x, t.y, t.z);
-        l.set(c * C + k, t.w);
+    for (int i = 0; i < M; ++i) {
+      const int c = i / C;
+      const float4 x = xr[i % (PD + 1)], v = vr[i % (PD + 1)];
+      WindTaps wt;
+      if constexpr (wind) {
+        if constexpr (LW == 2)
+          wt = wind_fetch_half(wl, W, f3(x.x, x.y, x.z));
+        else if constexpr (LW == 1)
+          wt = wind_fetch_from(wl, W, f3(x.x, x.y, x.z));
+        else
+          wt = wind_fetch(W, f3(x.x, x.y, x.z));
       }
-      tile_sync();
-      if (c == 0 && owns_root) {
-        // root: p0 = M * source (:190-193); the pipelined forms keep u0 = p0 - x0
-        const float3 x0 = p[0];
-        const float3 src = A.rmode == kRootModel ? x0 : rsrc;
-        p[0] = A.model_ident ? src : transform(A, src);
-        if (G > 1) u0 = sub3(p[0], x0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (i + PD < M) load_row(i + PD);
+      __builtin_amdgcn_sched_barrier(0);
+      float3 F = F0;
+      if constexpr (wind) {
+        const float3 w = wind_blend(wt);
+        F = f3(F0.x + w.x, F0.y + w.y, F0.z + w.z);
+      }
+      float3 pr = f3(__builtin_fmaf(dt2, F.x, __builtin_fmaf(dt, v.x, x.x)),
+                     __builtin_fmaf(dt2, F.y, __builtin_fmaf(dt, v.y, x.y)),
+                     __builtin_fmaf(dt2, F.z, __builtin_fmaf(dt, v.z, x.z)));
+      if (c == 0 && root_row) pr = f3(x.x, x.y, x.z);
+      row_slot[i % C * FTL_WAVE] = make_float4(pr.x, pr.y, pr.z, x.w);
+      __builtin_amdgcn_sched_barrier(0);
+      if (i % C == C - 1) {
+        tile_sync();
+#pragma unroll
+        for (int k = 0; k < C; ++k) {
+          const float4 t = stage[slot<C>(lane, k)];
+          p[c * C + k] = f3(t.x, t.y, t.z);
+          // The copy takes the length out of the read's four registers, which the
+          // allocator otherwise keeps together: 126 -> 109 VGPRs at M = 16, and
+          // with that four waves per SIMD instead of two (50k strands of 64
+          // points with wind 86.6 -> 84.8 us, 262k of 32 133.1 -> 131.7 us).
+          float len = t.w;
+          if constexpr (G > 1) asm volatile("v_mov_b32 %0, %1" : "=v"(len) : "v"(t.w));
+          l.set(c * C + k, len);
+        }
+        tile_sync();
+        if (c == 0 && owns_root) {
+          // root: p0 = M * source (:190-193); the pipelined forms keep u0 = p0 - x0
+          const float3 x0 = p[0];
+          const float3 src = A.rmode == kRootModel ? x0 : rsrc;
+          p[0] = A.model_ident ? src : transform(A, src);
+          if (G > 1) u0 = sub3(p[0], x0);
+        }
       }
     }
-  }
+  };
+  if (WIND == kWindOn || (WIND == kWindAny && A.wind_grid))
+    load_phase(std::true_type{});
+  else
+    load_phase(std::false_type{});
 
   // ---- rest lengths scaled once per tile (pipelined forms) ---------------
   // Every sweep uses sigma * l[j]: formed here once, the same product each
@@ -556,8 +588,8 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
     float3 clast = f3(0.f, 0.f, 0.f);
     float3 u;
     for (int it = 0; it < K - 1; ++it)
-      sweep<M, GUARD, false, NT>(A, V, S, p, l, nl, pp, last_pre, clast, stage, strand0, N, lane, cm);
-    sweep<M, GUARD, true, NT>(A, V, S, p, l, nl, pp, last_pre, clast, stage, strand0, N, lane, cm);
+      sweep<M, GUARD, false, NT>(A, V, S, p, l, nl, pp, last_pre, clast, stage, bvel, N, lane, cm);
+    sweep<M, GUARD, true, NT>(A, V, S, p, l, nl, pp, last_pre, clast, stage, bvel, N, lane, cm);
     // The last point: velocity = raw correction, collisions deferred to here.
     u = clast;
 #pragma unroll
@@ -570,7 +602,7 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
         bad = !(isfinite(pm.x) && isfinite(pm.y) && isfinite(pm.z) && isfinite(v.x) && isfinite(v.y) &&
                 isfinite(v.z));
         stage[slot<C>(lane, j % C)] = make_float4(v.x, v.y, v.z, 0.0f);
-        flush_chunk<M, G, GUARD, NT>(A.vel, strand0, nstr, N, j / C, stage, lane);
+        flush_chunk<M, G, GUARD, NT>(bvel, N, j / C, stage, lane);
       }
     }
   } else {
@@ -626,10 +658,14 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
       if (GUARD ? m == nl - 1 : m == M - 1)
         bad = !(isfinite(p[m].x) && isfinite(p[m].y) && isfinite(p[m].z) && isfinite(v.x) && isfinite(v.y) &&
                 isfinite(v.z));
-      if (m % C == C - 1) flush_velocities<M, G, GUARD, NT>(A.vel, strand0, nstr, N, m / C, (float*)stage, lane);
+      if (m % C == C - 1) flush_velocities<M, G, GUARD, NT>(bvel, N, m / C, (float*)stage, lane);
     }
   }
-  // positions, after every velocity (DFTL reads the step's input positions)
+  // positions, after every velocity (DFTL reads the step's input positions);
+  // the stage addresses are formed anew (opaque lane): kept from the load
+  // phase they would hold eight registers through the sweeps
+  int sl = lane;
+  asm volatile("" : "+v"(sl));
 #pragma unroll
   for (int c = 0; c < M / C; ++c) {
     if (GUARD && G == 1 && c * C >= nl) continue;
@@ -646,9 +682,9 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
 #pragma unroll
     for (int j = 0; j < C; ++j) {
       const float3 q = p[c * C + j];
-      stage[slot<C>(lane, j)] = make_float4(q.x, q.y, q.z, w[j]);
+      stage[slot<C>(sl, j)] = make_float4(q.x, q.y, q.z, w[j]);
     }
-    flush_chunk<M, G, GUARD, NT>(A.pos, strand0, nstr, N, c, stage, lane);
+    flush_chunk<M, G, GUARD, NT>(bpos, N, c, stage, lane);
   }
   bad = bad && valid;
   const unsigned long long b = __ballot(bad);

@@ -24,24 +24,6 @@ namespace ftl_wide_impl {
 
 using namespace ftl_tile_impl;
 
-typedef float f4v __attribute__((ext_vector_type(4)));
-typedef unsigned u4v __attribute__((ext_vector_type(4)));
-typedef __amdgpu_buffer_rsrc_t BufferRsrc;
-
-// Raw buffer of `bytes` from p: dword offsets at or past its end load 0 and
-// store nothing.
-__device__ __forceinline__ BufferRsrc buffer_of(const void* p, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)bytes, 0x00027000);
-}
-__device__ __forceinline__ float4 buffer_load4(BufferRsrc r, unsigned byte) {
-  const f4v t = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(r, (int)byte, 0, 0));
-  return make_float4(t.x, t.y, t.z, t.w);
-}
-template <bool NT>
-__device__ __forceinline__ void buffer_store4(BufferRsrc r, unsigned byte, float4 v) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, f4v{v.x, v.y, v.z, v.w}), r, (int)byte, 0, NT ? 2 : 0);
-}
-
 // Stage slot of element e: permuted within its block of 8 so that lanes that
 // read at a stride of 2, 4 or 8 elements fall on different banks.
 __device__ __forceinline__ int element_slot(int e) { return e ^ ((e >> 3) & 7); }
