@@ -584,13 +584,12 @@ static ftl_status groom_step(ftl_groom* g, float dt, void* stream, hipEvent_t st
   if (form < 0 && cls < 0) return ftl_fail(FTL_ERR_UNSUPPORTED, "no launch class for npoints=%d", g->npoints);
   hipError_t e;
   if ((e = hipSetDevice(g->ctx->device)) != hipSuccess) return ftl_hip_fail(e, "hipSetDevice");
-  const bool nt = (size_t)g->nstrands * g->npoints * 2 * sizeof(float4) > ftl_stream_store_bytes();
   if (form >= 0) {
-    if ((e = ftl_launch_wide(form, A, (hipStream_t)stream, start, stop, nt)) != hipSuccess)
+    if ((e = ftl_launch_wide(form, A, (hipStream_t)stream, start, stop)) != hipSuccess)
       return ftl_hip_fail(e, "FTL step launch");
     return FTL_OK;
   }
-  if ((e = ftl_launch_plain(cls, A, (hipStream_t)stream, start, stop, nt)) != hipSuccess)
+  if ((e = ftl_launch_plain(cls, A, (hipStream_t)stream, start, stop)) != hipSuccess)
     return ftl_hip_fail(e, "FTL step launch");
   return FTL_OK;
 }

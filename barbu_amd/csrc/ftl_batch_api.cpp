@@ -103,7 +103,7 @@ ftl_status ftl_plan_tiles(ftl_ctx* ctx, ftl_groom* const* grooms, int n, std::ve
     state_bytes += (size_t)g->nstrands * g->npoints * 2 * sizeof(float4);
   }
   // the class kernels of a batch run together: the batch's whole state decides
-  const bool stream_stores = state_bytes > ftl_stream_store_bytes();
+  const FtlCache cp = ftl_cache_for(state_bytes);
   if (total_tiles > (size_t)INT32_MAX) return ftl_fail(FTL_ERR_UNSUPPORTED, "too many tiles in one batch");
   {
     std::vector<ftl_groom*> seen(grooms, grooms + n);
@@ -134,7 +134,7 @@ ftl_status ftl_plan_tiles(ftl_ctx* ctx, ftl_groom* const* grooms, int n, std::ve
       ntiles += gp.ntiles;
     }
     const int count = (int)spans.size() - first;
-    if (count > 0) runs.push_back(ClassRun{run, first, count, ntiles, ntiles, stream_stores});
+    if (count > 0) runs.push_back(ClassRun{run, first, count, ntiles, ntiles, cp});
   }
   if (runs.size() > 64) return ftl_fail(FTL_ERR_UNSUPPORTED, "too many launch classes");
   return FTL_OK;
@@ -153,7 +153,7 @@ hipError_t ftl_enqueue_runs(const std::vector<ClassRun>& runs, const FtlStep* d_
     hipStream_t rs = (par && r > 0) ? (*side)[r - 1] : s;
     if (par && r > 0 && (e = hipStreamWaitEvent(rs, fork, 0)) != hipSuccess) return e;
     const ClassRun& cr = runs[r];
-    if ((e = ftl_launch_tiles(cr.cls, d_steps, d_spans + cr.first, cr.count, cr.ntiles, cr.grid, rs, cr.nt)) !=
+    if ((e = ftl_launch_tiles(cr.cls, d_steps, d_spans + cr.first, cr.count, cr.ntiles, cr.grid, rs, cr.cp)) !=
         hipSuccess)
       return e;
     if (par && r > 0) {

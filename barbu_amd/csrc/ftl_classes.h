@@ -86,6 +86,9 @@ constexpr int ftl_chunk_of(int m, int g, bool guarded) {
 #define FTL_WIDE_FORMS_16(X) X(1, 16) X(2, 16) X(3, 16) X(4, 16)
 #define FTL_WIDE_FORMS(X) FTL_WIDE_FORMS_2(X) FTL_WIDE_FORMS_4(X) FTL_WIDE_FORMS_8(X) FTL_WIDE_FORMS_16(X)
 
+// How a step kernel's loads and stores use the caches (ftl_cache_for).
+enum FtlCache : int { kCacheDefault, kCacheThrough, kCacheStream };
+
 // Form ids, beside the class ids in a batch's runs and spans: the form with M
 // points on each of G lanes, and all forms in one kernel.
 constexpr int ftl_wide_id(int m, int g) { return 256 + 32 * m + g; }

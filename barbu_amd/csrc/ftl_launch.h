@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "ftl_classes.h"
 #include "ftl_device.h"
 
 // Launch classes: (points per lane M, lanes per strand G, guarded).
@@ -11,18 +12,33 @@ int ftl_class_m(int cls);
 int ftl_class_g(int cls);
 int ftl_class_guarded(int cls);
 
-// State size (positions and velocities of every strand a launch steps)
-// above which the step kernels store with the non-temporal hint.  A step
-// rewrites all of its state; when that exceeds the device's last-level cache
-// (256 MB Infinity Cache) by enough that none of it is still cached when the
-// next step reads it back, keeping the stores out of the caches measured
-// faster (single grooms of 537 MB to 2.1 GB: -2 to -4%; the 64-groom frame,
-// 1.9 GB: -2.5%); a 268 MB groom measured 4-7% slower with the hint.
-size_t ftl_stream_store_bytes();
+// How a launch that steps state_bytes (positions and velocities, read and
+// rewritten in place) uses the caches.  By the size of that state against the
+// 256 MB Infinity Cache, in us per step, one groom stepped over and over:
+//   up to 144 MB through: its lines do not wait dirty in the XCDs' L2s for the
+//     end of the kernel to write them out (against default: 32 MB of 16 points
+//     29.2 -> 27.2 and 31.6 -> 29.9 with wind, 134 MB of 4 points 53.0 -> 50.0
+//     and 58.0 -> 56.2, 102 MB of 64 points 58.2 -> 56.4);
+//   up to 384 MB default: part of the state is still cached when the next step
+//     reads it, which both of the others lose (268 MB of 32 points with wind
+//     111.5, through 113.3, stream 120; 201 MB 105.2 -> 106.7 with through
+//     where three grooms take turns);
+//   above it stream: none of it would still be cached, so neither loads nor
+//     stores keep their lines (1 GB of 32 points: default 435, stores alone
+//     405, with the loads 391; 922 MB of 24 points, three grooms in turn, 347
+//     -> 323).  The launch classes' loads stay cached with wind (405 against
+//     413); the wide forms' do not (-1 to +1.5%, and a test of the wind ahead
+//     of their loads costs as much).
+FtlCache ftl_cache_for(size_t state_bytes);
+#define FTL_WITH_CACHE(cp, ...)                                                      \
+  switch (cp) {                                                                      \
+    case kCacheThrough: { constexpr FtlCache CP = kCacheThrough; __VA_ARGS__; break; } \
+    case kCacheStream: { constexpr FtlCache CP = kCacheStream; __VA_ARGS__; break; }   \
+    default: { constexpr FtlCache CP = kCacheDefault; __VA_ARGS__; break; }            \
+  }
 // start / stop: optional events bracketing the kernel itself (timing).
-// nt: non-temporal stores (state above ftl_stream_store_bytes()).
 hipError_t ftl_launch_plain(int cls, const FtlStep& A, hipStream_t stream, hipEvent_t start = nullptr,
-                            hipEvent_t stop = nullptr, bool nt = false);
+                            hipEvent_t stop = nullptr);
 // Wide forms (ftl_wide.h).  The level of a launch over n grooms (16, 8 or 4:
 // the lanes per strand its long strands take), or 0 when it fills the chip.
 int ftl_wide_level(int ncu, const int* nstrands, const int* npoints, int n);
@@ -31,13 +47,13 @@ int ftl_wide_level(int ncu, const int* nstrands, const int* npoints, int n);
 int ftl_wide_form(int level, int npoints);
 // The plain step of one groom by a wide form.
 hipError_t ftl_launch_wide(int form, const FtlStep& A, hipStream_t stream, hipEvent_t start = nullptr,
-                           hipEvent_t stop = nullptr, bool nt = false);
+                           hipEvent_t stop = nullptr);
 // Tile-list kernel of one class over the ntiles tiles of spans[0..nspans)
 // (every groom of that class, in tile order): workgroup b steps tiles b,
 // b + grid, ...  cls may be a wide form (ftl_wide_id) or FTL_WIDE_ALL, one
 // workgroup per tile.
 hipError_t ftl_launch_tiles(int cls, const FtlStep* grooms, const FtlSpan* spans, int nspans, int ntiles, int grid,
-                            hipStream_t stream, bool nt);
+                            hipStream_t stream, FtlCache cp);
 // Resident tile-list workgroups per CU for a class.
 int ftl_tiles_blocks_per_cu(int cls);
 // Skinning of mesh vertices (and normals when nout is not null): mode 0 dual

@@ -165,8 +165,8 @@ __global__ __launch_bounds__(256) void ftl_upload_kernel(const uint4* __restrict
 // Host dispatch.
 
 #define FTL_DECL(id, M, G, GU, W, CH)                                                                    \
-  hipError_t ftl_launch_plain_##id(const FtlStep& A, hipStream_t stream, hipEvent_t, hipEvent_t, bool); \
-  hipError_t ftl_launch_tiles_##id(const FtlStep*, const FtlSpan*, int, int, int, hipStream_t, bool);    \
+  hipError_t ftl_launch_plain_##id(const FtlStep& A, hipStream_t stream, hipEvent_t, hipEvent_t, FtlCache); \
+  hipError_t ftl_launch_tiles_##id(const FtlStep*, const FtlSpan*, int, int, int, hipStream_t, FtlCache);    \
   int ftl_tiles_occ_##id();
 FTL_CLASSES(FTL_DECL)
 #undef FTL_DECL
@@ -187,14 +187,19 @@ int ftl_class_m(int cls) { return (cls >= 0 && cls < FTL_NCLASSES) ? kFtlClasses
 int ftl_class_g(int cls) { return (cls >= 0 && cls < FTL_NCLASSES) ? kFtlClasses[cls].g : 0; }
 int ftl_class_guarded(int cls) { return (cls >= 0 && cls < FTL_NCLASSES) ? kFtlClasses[cls].guarded : 0; }
 
-size_t ftl_stream_store_bytes() { return (size_t)384 << 20; }
+FtlCache ftl_cache_for(size_t state_bytes) {
+  return state_bytes <= (size_t)144 << 20 ? kCacheThrough : state_bytes <= (size_t)384 << 20 ? kCacheDefault : kCacheStream;
+}
+static FtlCache step_cache(const FtlStep& A) {
+  return ftl_cache_for((size_t)A.nstrands * A.npoints * 2 * sizeof(float4));
+}
 
-hipError_t ftl_launch_plain(int cls, const FtlStep& A, hipStream_t stream, hipEvent_t start, hipEvent_t stop,
-                            bool nt) {
+hipError_t ftl_launch_plain(int cls, const FtlStep& A, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
+  const FtlCache cp = step_cache(A);
   switch (cls) {
 #define FTL_LP(id, M, G, GU, W, CH) \
   case id:                   \
-    return ftl_launch_plain_##id(A, stream, start, stop, nt);
+    return ftl_launch_plain_##id(A, stream, start, stop, cp);
     FTL_CLASSES(FTL_LP)
 #undef FTL_LP
   }
@@ -202,8 +207,8 @@ hipError_t ftl_launch_plain(int cls, const FtlStep& A, hipStream_t stream, hipEv
 }
 
 #define FTL_WDECL(G)                                                                                               \
-  hipError_t ftl_launch_wide_##G(int m, const FtlStep& A, hipStream_t, hipEvent_t, hipEvent_t, bool);              \
-  hipError_t ftl_launch_wide_tiles_##G(int m, const FtlStep*, const FtlSpan*, int, int, hipStream_t, bool);
+  hipError_t ftl_launch_wide_##G(int m, const FtlStep& A, hipStream_t, hipEvent_t, hipEvent_t, FtlCache);              \
+  hipError_t ftl_launch_wide_tiles_##G(int m, const FtlStep*, const FtlSpan*, int, int, hipStream_t, FtlCache);
 FTL_WDECL(2)
 FTL_WDECL(4)
 FTL_WDECL(8)
@@ -260,22 +265,22 @@ int ftl_wide_form(int level, int npoints) {
   return ftl_wide_id((npoints + g - 1) / g, g);
 }
 
-hipError_t ftl_launch_wide(int form, const FtlStep& A, hipStream_t stream, hipEvent_t start, hipEvent_t stop,
-                           bool nt) {
+hipError_t ftl_launch_wide(int form, const FtlStep& A, hipStream_t stream, hipEvent_t start, hipEvent_t stop) {
+  const FtlCache cp = step_cache(A);
   const int m = ftl_wide_m(form), g = ftl_wide_g(form);
   if (A.nstrands <= 0) return hipSuccess;
   if (A.npoints > m * g || A.npoints <= (m - 1) * g) return hipErrorInvalidValue;
   switch (g) {
-    case 2: return ftl_launch_wide_2(m, A, stream, start, stop, nt);
-    case 4: return ftl_launch_wide_4(m, A, stream, start, stop, nt);
-    case 8: return ftl_launch_wide_8(m, A, stream, start, stop, nt);
-    case 16: return ftl_launch_wide_16(m, A, stream, start, stop, nt);
+    case 2: return ftl_launch_wide_2(m, A, stream, start, stop, cp);
+    case 4: return ftl_launch_wide_4(m, A, stream, start, stop, cp);
+    case 8: return ftl_launch_wide_8(m, A, stream, start, stop, cp);
+    case 16: return ftl_launch_wide_16(m, A, stream, start, stop, cp);
   }
   return hipErrorInvalidValue;
 }
 
 hipError_t ftl_launch_tiles(int cls, const FtlStep* grooms, const FtlSpan* spans, int nspans, int ntiles, int grid,
-                            hipStream_t stream, bool nt) {
+                            hipStream_t stream, FtlCache cp) {
   if (cls == FTL_WIDE_ALL) {
     if (ntiles <= 0 || nspans <= 0) return hipSuccess;
     return ftl_launch_wide_all(grooms, spans, nspans, ntiles, stream);
@@ -284,16 +289,16 @@ hipError_t ftl_launch_tiles(int cls, const FtlStep* grooms, const FtlSpan* spans
     if (ntiles <= 0 || nspans <= 0) return hipSuccess;
     const int m = ftl_wide_m(cls);
     switch (ftl_wide_g(cls)) {
-      case 2: return ftl_launch_wide_tiles_2(m, grooms, spans, nspans, ntiles, stream, nt);
-      case 4: return ftl_launch_wide_tiles_4(m, grooms, spans, nspans, ntiles, stream, nt);
-      case 8: return ftl_launch_wide_tiles_8(m, grooms, spans, nspans, ntiles, stream, nt);
+      case 2: return ftl_launch_wide_tiles_2(m, grooms, spans, nspans, ntiles, stream, cp);
+      case 4: return ftl_launch_wide_tiles_4(m, grooms, spans, nspans, ntiles, stream, cp);
+      case 8: return ftl_launch_wide_tiles_8(m, grooms, spans, nspans, ntiles, stream, cp);
     }
     return hipErrorInvalidValue;
   }
   switch (cls) {
 #define FTL_LB(id, M, G, GU, W, CH) \
   case id:                   \
-    return ftl_launch_tiles_##id(grooms, spans, nspans, ntiles, grid, stream, nt);
+    return ftl_launch_tiles_##id(grooms, spans, nspans, ntiles, grid, stream, cp);
     FTL_CLASSES(FTL_LB)
 #undef FTL_LB
   }

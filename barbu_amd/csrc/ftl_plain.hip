@@ -2,8 +2,7 @@
 // time with -DFTL_CLASS_ID=<id>: one wave64 workgroup per tile of strands, or,
 // for launches with wind, workgroups of four tiles sharing an LDS copy of the
 // wind lattice; and the tile-list kernel of batched frames.  Each kernel comes
-// in two forms, NT (non-temporal stores, for launches whose state exceeds
-// ftl_stream_store_bytes()) and not.
+// in three forms, by how its loads and stores use the caches (ftl_cache_for).
 #include <hip/hip_ext.h>
 
 #include "ftl_classes.h"
@@ -68,7 +67,7 @@ constexpr bool kWindLds = (kWavesPerEu == 4 || kWavesPerEu == 2) && kWindGroupsP
 // A class with the LDS form never runs its plain kernel with wind.
 constexpr int kPlainWind = kWindLds && FTL_WIND_LDS ? ftl_tile_impl::kWindOff : ftl_tile_impl::kWindAny;
 
-template <bool NT>
+template <FtlCache CP>
 __global__ __launch_bounds__(FTL_WAVE) __attribute__((amdgpu_waves_per_eu(kWavesPerEu, 8)))
 void ftl_plain_kernel(FtlStep arg) {
   (void)arg;
@@ -81,11 +80,11 @@ void ftl_plain_kernel(FtlStep arg) {
   const FtlStep& A = arg;
 #endif
   __shared__ ftl_tile_impl::TileLds<CL::M, CL::G, CL::GU> sh;
-  ftl_tile_impl::ftl_tile<CL::M, CL::G, CL::GU, NT, kPlainWind, kLoadAhead>(
+  ftl_tile_impl::ftl_tile<CL::M, CL::G, CL::GU, CP, kPlainWind, kLoadAhead>(
       A, blockIdx.x * (FTL_WAVE / CL::G), sh);
 }
 
-template <bool NT>
+template <FtlCache CP>
 __global__ __launch_bounds__(FTL_WAVE * kWindWaves) __attribute__((amdgpu_waves_per_eu(kWavesPerEu, 8)))
 void ftl_plain_wind_kernel(FtlStep arg) {
   (void)arg;
@@ -106,7 +105,7 @@ void ftl_plain_wind_kernel(FtlStep arg) {
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / FTL_WAVE);
     const int t = (int)blockIdx.x * kWindWaves + w;
     if (t < ntiles)
-      ftl_tile_impl::ftl_tile<CL::M, CL::G, CL::GU, NT, ftl_tile_impl::kWindOn, kLoadAhead, kWindHalf ? 2 : 1>(
+      ftl_tile_impl::ftl_tile<CL::M, CL::G, CL::GU, CP, ftl_tile_impl::kWindOn, kLoadAhead, kWindHalf ? 2 : 1>(
           A, t * spt, sh[w], lattice);
   }
 }
@@ -119,22 +118,16 @@ void ftl_plain_wind_kernel(FtlStep arg) {
 // start / stop (may be null): events that take the kernel's own start and end
 // timestamps (hipExtLaunchKernelGGL), for per-launch timing.
 hipError_t FTL_PASTE(ftl_launch_plain_, FTL_CLASS_ID)(const FtlStep& A, hipStream_t stream, hipEvent_t start,
-                                                      hipEvent_t stop, bool nt) {
+                                                      hipEvent_t stop, FtlCache cp) {
   constexpr int spt = FTL_WAVE / CL::G;
   const int nblocks = (A.nstrands + spt - 1) / spt;
   if (nblocks <= 0) return hipSuccess;
   if (kWindLds && FTL_WIND_LDS && A.wind_grid) {
     const dim3 grid((nblocks + kWindWaves - 1) / kWindWaves), block(FTL_WAVE * kWindWaves);
-    if (nt)
-      hipExtLaunchKernelGGL(ftl_plain_wind_kernel<true>, grid, block, 0, stream, start, stop, 0, A);
-    else
-      hipExtLaunchKernelGGL(ftl_plain_wind_kernel<false>, grid, block, 0, stream, start, stop, 0, A);
+    FTL_WITH_CACHE(cp, hipExtLaunchKernelGGL(ftl_plain_wind_kernel<CP>, grid, block, 0, stream, start, stop, 0, A))
     return hipGetLastError();
   }
-  if (nt)
-    hipExtLaunchKernelGGL(ftl_plain_kernel<true>, dim3(nblocks), dim3(FTL_WAVE), 0, stream, start, stop, 0, A);
-  else
-    hipExtLaunchKernelGGL(ftl_plain_kernel<false>, dim3(nblocks), dim3(FTL_WAVE), 0, stream, start, stop, 0, A);
+  FTL_WITH_CACHE(cp, hipExtLaunchKernelGGL(ftl_plain_kernel<CP>, dim3(nblocks), dim3(FTL_WAVE), 0, stream, start, stop, 0, A))
   return hipGetLastError();
 }
 
@@ -150,7 +143,7 @@ hipError_t FTL_PASTE(ftl_launch_plain_, FTL_CLASS_ID)(const FtlStep& A, hipStrea
 
 namespace {
 
-template <bool NT>
+template <FtlCache CP>
 __global__ __launch_bounds__(FTL_WAVE) __attribute__((amdgpu_waves_per_eu(kWavesPerEu, 8)))
 void ftl_tiles_kernel(const FtlStep* __restrict__ grooms, const FtlSpan* __restrict__ spans, int nspans,
                       int ntiles) {
@@ -160,25 +153,23 @@ void ftl_tiles_kernel(const FtlStep* __restrict__ grooms, const FtlSpan* __restr
     const int lo = ftl_tile_impl::span_of(spans, nspans, t);
     const int gi = __builtin_amdgcn_readfirstlane(spans[lo].groom);
     const int s0 = (t - __builtin_amdgcn_readfirstlane(spans[lo].tile0)) * spt;
-    ftl_tile_impl::ftl_tile<CL::M, CL::G, CL::GU, NT, ftl_tile_impl::kWindAny, kLoadAhead>(grooms[gi], s0, sh);
+    ftl_tile_impl::ftl_tile<CL::M, CL::G, CL::GU, CP, ftl_tile_impl::kWindAny, kLoadAhead>(grooms[gi], s0, sh);
   }
 }
 
 }  // namespace
 
 hipError_t FTL_PASTE(ftl_launch_tiles_, FTL_CLASS_ID)(const FtlStep* grooms, const FtlSpan* spans, int nspans,
-                                                      int ntiles, int grid, hipStream_t stream, bool nt) {
+                                                      int ntiles, int grid, hipStream_t stream, FtlCache cp) {
   if (ntiles <= 0 || nspans <= 0) return hipSuccess;
-  if (nt)
-    hipLaunchKernelGGL(ftl_tiles_kernel<true>, dim3(grid), dim3(FTL_WAVE), 0, stream, grooms, spans, nspans, ntiles);
-  else
-    hipLaunchKernelGGL(ftl_tiles_kernel<false>, dim3(grid), dim3(FTL_WAVE), 0, stream, grooms, spans, nspans, ntiles);
+  FTL_WITH_CACHE(cp, hipLaunchKernelGGL(ftl_tiles_kernel<CP>, dim3(grid), dim3(FTL_WAVE), 0, stream, grooms, spans, nspans,
+                                        ntiles))
   return hipGetLastError();
 }
 
 int FTL_PASTE(ftl_tiles_occ_, FTL_CLASS_ID)() {
   int blocks = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, ftl_tiles_kernel<false>, FTL_WAVE, 0) != hipSuccess) {
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, ftl_tiles_kernel<kCacheDefault>, FTL_WAVE, 0) != hipSuccess) {
     (void)hipGetLastError();
     return 0;
   }

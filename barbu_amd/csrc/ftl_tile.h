@@ -171,13 +171,17 @@ typedef __amdgpu_buffer_rsrc_t BufferRsrc;
 __device__ __forceinline__ BufferRsrc buffer_of(const void* p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)bytes, 0x00027000);
 }
+template <bool STREAM>
 __device__ __forceinline__ float4 buffer_load4(BufferRsrc r, unsigned byte) {
-  const f4v t = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(r, (int)byte, 0, 0));
+  const f4v t = __builtin_bit_cast(f4v, __builtin_amdgcn_raw_buffer_load_b128(r, (int)byte, 0, STREAM ? 2 : 0));
   return make_float4(t.x, t.y, t.z, t.w);
 }
-template <bool NT>
+// The cache bits of the instruction: sc1 (16) writes through the XCD's L2, nt
+// (2) marks the line as not to be kept.
+template <FtlCache CP>
 __device__ __forceinline__ void buffer_store4(BufferRsrc r, unsigned byte, float4 v) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, f4v{v.x, v.y, v.z, v.w}), r, (int)byte, 0, NT ? 2 : 0);
+  constexpr int bits = CP == kCacheThrough ? 16 : CP == kCacheStream ? 2 : 0;
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, f4v{v.x, v.y, v.z, v.w}), r, (int)byte, 0, bits);
 }
 
 // Byte offset, within the tile, of the lane's point in row 0 of chunk c (row k
@@ -205,10 +209,8 @@ __device__ __forceinline__ unsigned row_offset(int N, int c, int lane) {
 constexpr int kFlushRows = FTL_FLUSH_ROWS;
 
 // Writes chunk c of the tile (C points per lane, staged in LDS) to dst in the
-// coalesced order of the load.  Called by the whole wave.  NT: the stores carry
-// the non-temporal hint (launches whose state is too large for the next step
-// to find any of it in the caches).
-template <int M, int G, bool GUARD, bool NT>
+// coalesced order of the load.  Called by the whole wave.
+template <int M, int G, bool GUARD, FtlCache CP>
 __device__ __forceinline__ void flush_chunk(BufferRsrc dst, int N, int c, const float4* __restrict__ stage, int lane) {
   constexpr int C = Tile<M, G, GUARD>::C;
   constexpr int RS = FTL_WAVE / C / G;
@@ -221,14 +223,14 @@ __device__ __forceinline__ void flush_chunk(BufferRsrc dst, int N, int c, const 
   tile_sync();
 #pragma unroll
   for (int k = 0; k < C; ++k) {
-    buffer_store4<NT>(dst, off + 16u * (unsigned)(k * RS * N), t0[k * FTL_WAVE]);
+    buffer_store4<CP>(dst, off + 16u * (unsigned)(k * RS * N), t0[k * FTL_WAVE]);
     if (k % kFlushRows == kFlushRows - 1) __builtin_amdgcn_sched_barrier(0);
   }
   tile_sync();
 }
 
 // The same for velocities, staged as three floats per point (park_slot).
-template <int M, int G, bool GUARD, bool NT>
+template <int M, int G, bool GUARD, FtlCache CP>
 __device__ __forceinline__ void flush_velocities(BufferRsrc dst, int N, int c, const float* stage, int lane) {
   constexpr int C = Tile<M, G, GUARD>::C;
   constexpr int RS = FTL_WAVE / C / G;
@@ -240,7 +242,7 @@ __device__ __forceinline__ void flush_velocities(BufferRsrc dst, int N, int c, c
 #pragma unroll
   for (int k = 0; k < C; ++k) {
     const float* t = t0 + k * (FTL_WAVE / C);
-    buffer_store4<NT>(dst, off + 16u * (unsigned)(k * RS * N),
+    buffer_store4<CP>(dst, off + 16u * (unsigned)(k * RS * N),
                       make_float4(t[0], t[FTL_WAVE + 1], t[2 * (FTL_WAVE + 1)], 0.0f));
     if (k % kFlushRows == kFlushRows - 1) __builtin_amdgcn_sched_barrier(0);
   }
@@ -284,7 +286,7 @@ __device__ __forceinline__ void collide_sweep(const Spheres& S, float3 (&p)[M], 
 // also forms the velocities, stages them and flushes every completed chunk;
 // the lane's last point is left to the caller (its velocity is the raw
 // correction and its collision comes after the sweep).
-template <int M, bool GUARD, bool FINAL, bool NT>
+template <int M, bool GUARD, bool FINAL, FtlCache CP>
 __device__ __forceinline__ void sweep(const FtlStep& A, const VelArgs& V, const Spheres& S, float3 (&p)[M],
                                       const LenLds& l, int nl,
                                       const float4* __restrict__ pp, float3& last_pre, float3& clast,
@@ -320,7 +322,7 @@ __device__ __forceinline__ void sweep(const FtlStep& A, const VelArgs& V, const 
         p[m] = pm;
         const float3 v = out_velocity(V, pp, m, pm, u);
         stage[slot<C>(lane, m % C)] = make_float4(v.x, v.y, v.z, 0.0f);
-        if (m % C == C - 1) flush_chunk<M, 1, GUARD, NT>(bvel, N, m / C, stage, lane);
+        if (m % C == C - 1) flush_chunk<M, 1, GUARD, CP>(bvel, N, m / C, stage, lane);
       }
       if (GUARD ? (j == nl - 1) : (j == M - 1)) {
         clast = c;
@@ -409,7 +411,7 @@ struct TileLds : TileLens<M, G == 1> {
 // lattice (first float4 of each node) in LDS.
 // WIND: whether the launch has wind, where the kernel knows.
 enum { kWindOff = 0, kWindOn = 1, kWindAny = 2 };
-template <int M, int G, bool GUARD, bool NT, int WIND, int PD_ = FTL_LOAD_AHEAD, int LW = 0>
+template <int M, int G, bool GUARD, FtlCache CP, int WIND, int PD_ = FTL_LOAD_AHEAD, int LW = 0>
 __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<M, G, GUARD>& sh,
                                          const float4* wl = nullptr) {
   float4* __restrict__ stage = sh.stage;
@@ -477,8 +479,8 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
     auto load_row = [&](int i) {
       const unsigned first = GUARD ? row_offset<M, G, GUARD, true>(N, i / C, lane) : off0 + 16u * (i / C * C);
       const unsigned off = first + 16u * (unsigned)(i % C * RS * N);
-      xr[i % (PD + 1)] = buffer_load4(bpos, off);
-      vr[i % (PD + 1)] = buffer_load4(bvel, off);
+      xr[i % (PD + 1)] = buffer_load4<CP == kCacheStream && !wind>(bpos, off);
+      vr[i % (PD + 1)] = buffer_load4<CP == kCacheStream && !wind>(bvel, off);
     };
 #pragma unroll
     for (int i = 0; i < PD; ++i) load_row(i);
@@ -588,8 +590,8 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
     float3 clast = f3(0.f, 0.f, 0.f);
     float3 u;
     for (int it = 0; it < K - 1; ++it)
-      sweep<M, GUARD, false, NT>(A, V, S, p, l, nl, pp, last_pre, clast, stage, bvel, N, lane, cm);
-    sweep<M, GUARD, true, NT>(A, V, S, p, l, nl, pp, last_pre, clast, stage, bvel, N, lane, cm);
+      sweep<M, GUARD, false, CP>(A, V, S, p, l, nl, pp, last_pre, clast, stage, bvel, N, lane, cm);
+    sweep<M, GUARD, true, CP>(A, V, S, p, l, nl, pp, last_pre, clast, stage, bvel, N, lane, cm);
     // The last point: velocity = raw correction, collisions deferred to here.
     u = clast;
 #pragma unroll
@@ -602,7 +604,7 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
         bad = !(isfinite(pm.x) && isfinite(pm.y) && isfinite(pm.z) && isfinite(v.x) && isfinite(v.y) &&
                 isfinite(v.z));
         stage[slot<C>(lane, j % C)] = make_float4(v.x, v.y, v.z, 0.0f);
-        flush_chunk<M, G, GUARD, NT>(bvel, N, j / C, stage, lane);
+        flush_chunk<M, G, GUARD, CP>(bvel, N, j / C, stage, lane);
       }
     }
   } else {
@@ -658,7 +660,7 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
       if (GUARD ? m == nl - 1 : m == M - 1)
         bad = !(isfinite(p[m].x) && isfinite(p[m].y) && isfinite(p[m].z) && isfinite(v.x) && isfinite(v.y) &&
                 isfinite(v.z));
-      if (m % C == C - 1) flush_velocities<M, G, GUARD, NT>(bvel, N, m / C, (float*)stage, lane);
+      if (m % C == C - 1) flush_velocities<M, G, GUARD, CP>(bvel, N, m / C, (float*)stage, lane);
     }
   }
   // positions, after every velocity (DFTL reads the step's input positions);
@@ -684,7 +686,7 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
       const float3 q = p[c * C + j];
       stage[slot<C>(sl, j)] = make_float4(q.x, q.y, q.z, w[j]);
     }
-    flush_chunk<M, G, GUARD, NT>(bpos, N, c, stage, lane);
+    flush_chunk<M, G, GUARD, CP>(bpos, N, c, stage, lane);
   }
   bad = bad && valid;
   const unsigned long long b = __ballot(bad);

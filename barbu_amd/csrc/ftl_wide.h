@@ -49,7 +49,7 @@ __device__ __forceinline__ float3 from_next_lane(float3 x) { return f3(dpp<0x101
 // Float4s of a form's LDS stage.
 constexpr int wide_stage(int m) { return m > 1 ? FTL_WAVE * m : 1; }
 
-template <int M, int G, bool NT>
+template <int M, int G, FtlCache CP>
 __device__ __forceinline__ void ftl_wide_tile(const FtlStep& A, int strand0, float4* stage) {
   constexpr int SPT = FTL_WAVE / G;
   int tid = (int)threadIdx.x;
@@ -71,13 +71,13 @@ __device__ __forceinline__ void ftl_wide_tile(const FtlStep& A, int strand0, flo
   float4 x[M], v[M];
 #pragma unroll
   for (int i = 0; i < M; ++i) {
-    x[i] = buffer_load4(bpos, own + 1024u * i);
-    v[i] = buffer_load4(bvel, own + 1024u * i);
+    x[i] = buffer_load4<CP == kCacheStream>(bpos, own + 1024u * i);
+    v[i] = buffer_load4<CP == kCacheStream>(bvel, own + 1024u * i);
   }
   // The strand's root, on every lane (the collider cull needs it there).
   float3 x0, p0;
   {
-    const float4 r = buffer_load4(bpos, 16u * (unsigned)(ls * N));
+    const float4 r = buffer_load4<false>(bpos, 16u * (unsigned)(ls * N));
     x0 = f3(r.x, r.y, r.z);
     const float3 src = A.rmode == kRootModel ? x0 : root_source(A, strand0 + min(ls, nst - 1));
     p0 = A.model_ident ? src : transform(A, src);
@@ -204,10 +204,10 @@ __device__ __forceinline__ void ftl_wide_tile(const FtlStep& A, int strand0, flo
         if (j < nl) stage[element_slot(ls * N + g * M + j)] = out[j];
       tile_sync();
 #pragma unroll
-      for (int i = 0; i < M; ++i) buffer_store4<NT>(b, own + 1024u * i, stage[element_slot(FTL_WAVE * i + lane)]);
+      for (int i = 0; i < M; ++i) buffer_store4<CP>(b, own + 1024u * i, stage[element_slot(FTL_WAVE * i + lane)]);
       tile_sync();
     } else {
-      buffer_store4<NT>(b, own, out[0]);
+      buffer_store4<CP>(b, own, out[0]);
     }
   };
   store_rows(bvel);

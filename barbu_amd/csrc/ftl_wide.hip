@@ -5,6 +5,7 @@
 #include <hip/hip_ext.h>
 
 #include "ftl_launch.h"
+#include "ftl_launch.h"
 #include "ftl_wide.h"
 
 #ifndef FTL_WIDE_LANES
@@ -20,7 +21,7 @@ using namespace ftl_wide_impl;
 
 #if FTL_WIDE_LANES > 0
 
-template <int M, int G, bool NT>
+template <int M, int G, FtlCache CP>
 __global__ __launch_bounds__(FTL_WAVE) void ftl_wide_kernel(FtlStep arg) {
   (void)arg;
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -29,10 +30,10 @@ __global__ __launch_bounds__(FTL_WAVE) void ftl_wide_kernel(FtlStep arg) {
   const FtlStep& A = arg;
 #endif
   __shared__ float4 sh[wide_stage(M)];
-  ftl_wide_tile<M, G, NT>(A, blockIdx.x * (FTL_WAVE / G), sh);
+  ftl_wide_tile<M, G, CP>(A, blockIdx.x * (FTL_WAVE / G), sh);
 }
 
-template <int M, int G, bool NT>
+template <int M, int G, FtlCache CP>
 __global__ __launch_bounds__(FTL_WAVE) void ftl_wide_tiles_kernel(const FtlStep* __restrict__ grooms,
                                                                   const FtlSpan* __restrict__ spans, int nspans) {
   __shared__ float4 sh[wide_stage(M)];
@@ -40,7 +41,7 @@ __global__ __launch_bounds__(FTL_WAVE) void ftl_wide_tiles_kernel(const FtlStep*
   const int s = span_of(spans, nspans, t);
   const int gi = __builtin_amdgcn_readfirstlane(spans[s].groom);
   const int s0 = (t - __builtin_amdgcn_readfirstlane(spans[s].tile0)) * (FTL_WAVE / G);
-  ftl_wide_tile<M, G, NT>(grooms[gi], s0, sh);
+  ftl_wide_tile<M, G, CP>(grooms[gi], s0, sh);
 }
 
 #define FTL_FORMS FTL_PASTE(FTL_WIDE_FORMS_, FTL_WIDE_LANES)
@@ -48,16 +49,13 @@ __global__ __launch_bounds__(FTL_WAVE) void ftl_wide_tiles_kernel(const FtlStep*
 }  // namespace
 
 hipError_t FTL_PASTE(ftl_launch_wide_, FTL_WIDE_LANES)(int m, const FtlStep& A, hipStream_t stream, hipEvent_t start,
-                                                       hipEvent_t stop, bool nt) {
+                                                       hipEvent_t stop, FtlCache cp) {
   constexpr int spt = FTL_WAVE / FTL_WIDE_LANES;
   const dim3 grid((A.nstrands + spt - 1) / spt), block(FTL_WAVE);
   switch (m) {
 #define FTL_WL(M, G)                                                                                      \
   case M:                                                                                                 \
-    if (nt)                                                                                               \
-      hipExtLaunchKernelGGL((ftl_wide_kernel<M, G, true>), grid, block, 0, stream, start, stop, 0, A);   \
-    else                                                                                                  \
-      hipExtLaunchKernelGGL((ftl_wide_kernel<M, G, false>), grid, block, 0, stream, start, stop, 0, A);  \
+    FTL_WITH_CACHE(cp, hipExtLaunchKernelGGL((ftl_wide_kernel<M, G, CP>), grid, block, 0, stream, start, stop, 0, A)) \
     return hipGetLastError();
     FTL_FORMS(FTL_WL)
 #undef FTL_WL
@@ -66,15 +64,12 @@ hipError_t FTL_PASTE(ftl_launch_wide_, FTL_WIDE_LANES)(int m, const FtlStep& A, 
 }
 
 hipError_t FTL_PASTE(ftl_launch_wide_tiles_, FTL_WIDE_LANES)(int m, const FtlStep* grooms, const FtlSpan* spans,
-                                                             int nspans, int ntiles, hipStream_t stream, bool nt) {
+                                                             int nspans, int ntiles, hipStream_t stream, FtlCache cp) {
   const dim3 grid(ntiles), block(FTL_WAVE);
   switch (m) {
 #define FTL_WT(M, G)                                                                                              \
   case M:                                                                                                         \
-    if (nt)                                                                                                       \
-      hipLaunchKernelGGL((ftl_wide_tiles_kernel<M, G, true>), grid, block, 0, stream, grooms, spans, nspans);    \
-    else                                                                                                          \
-      hipLaunchKernelGGL((ftl_wide_tiles_kernel<M, G, false>), grid, block, 0, stream, grooms, spans, nspans);   \
+    FTL_WITH_CACHE(cp, hipLaunchKernelGGL((ftl_wide_tiles_kernel<M, G, CP>), grid, block, 0, stream, grooms, spans, nspans)) \
     return hipGetLastError();
     FTL_FORMS(FTL_WT)
 #undef FTL_WT
@@ -100,7 +95,7 @@ __global__ __launch_bounds__(FTL_WAVE) void ftl_wide_all_kernel(const FtlStep* _
   switch (__builtin_amdgcn_readfirstlane(spans[s].cls)) {
 #define FTL_WA(M, G)                                                              \
   case ftl_wide_id(M, G):                                                         \
-    ftl_wide_tile<M, G, false>(grooms[gi], tile * (FTL_WAVE / G), sh);            \
+    ftl_wide_tile<M, G, kCacheThrough>(grooms[gi], tile * (FTL_WAVE / G), sh);    \
     break;
     FTL_WIDE_FORMS_4(FTL_WA) FTL_WIDE_FORMS_8(FTL_WA) FTL_WIDE_FORMS_16(FTL_WA)
 #undef FTL_WA
