@@ -20,11 +20,16 @@
 
 #include <cstring>
 
+#include "ftl_buffer.h"
 #include "ftl_internal.h"
+#include "ftl_launch.h"
 #include "ftl_render.h"
 
 namespace {
 
+using ftl_dev::buffer_of;
+using ftl_dev::buffer_store4;
+using ftl_dev::BufferRsrc;
 using ftl_dev::f3;
 
 struct ExpandArgs {
@@ -86,6 +91,37 @@ __device__ __forceinline__ float3 bary(const float4* __restrict__ rnd, int inst,
   return f3(sx, sy, 1.0f - (sx + sy));
 }
 
+// How a pass stores its output, which it writes once and does not read back
+// (us write-back, through and streaming):
+// * Written through the XCD's L2 (the lines do not wait dirty for the end of
+//   the kernel) where its stores cover whole lines, that is by pages and by
+//   batches: 43 MB 10.3, 8.8; 131 MB 24.2, 21.4; 917 MB of 3 x 2 x 16 164,
+//   160.5; 812 MB of 4 x 3 x 7 146, 139.  The per-vertex form's runs of 2 nsub
+//   vertices are whole 64-byte sectors when nsub is even (up to 256 MB: 4 x 3
+//   x 6, 224 MB, 37.0, 34.7; 6 x 2 x 10, 219 MB, 36.4, 34.2; above, 8 x 4 x 10,
+//   592 MB, 128, 136); otherwise the halves of a sector merge in the L2 only
+//   while written back (4 x 3 x 7, 306 MB, 62, 112), but for runs of 14 or more
+//   in outputs that the Infinity Cache holds easily (8 x 1 x 15, 140 MB, 24.2,
+//   22.5; 4 x 2 x 3, 61 MB, 13.9, 15.8).
+// * Streaming, by pages and batches, where a patch makes at most 100 vertices
+//   of its twelve guide points and the output exceeds 224 MB: such a pass reads
+//   enough that its stores push the guides out of the caches (2 x 1 x 13, 476
+//   MB, 116, 115, 93; 2 x 2 x 8, 585 MB, 144, 143, 100; 2 x 1 x 14, 296 MB, 62,
+//   65, 58; but 2 x 3 x 16 127, 123, 125).
+// * One-line pages between 128 and 224 MB gain by neither (2 x 1 x 13, 142 MB,
+//   29.0, 29.6, 27.8; 238 MB 50.5, 51.8, 49.8).
+FtlCache vertex_cache(const ExpandArgs& A) {
+  const long long bytes = (long long)A.nthreads * A.ninst * A.nlines * 16;
+  return A.nsub % 2 == 0 ? bytes <= (256ll << 20) ? kCacheThrough : kCacheDefault
+                         : A.nsub >= 7 && bytes <= (144ll << 20) ? kCacheThrough : kCacheDefault;
+}
+FtlCache run_cache(const ExpandArgs& A, bool page) {
+  const long long bytes = (long long)A.nthreads * A.ninst * A.nlines * 16;
+  if (bytes > (224ll << 20) && A.ninst * A.nlines * 2 * A.nsub <= 100) return kCacheStream;
+  return page && A.nlines == 1 && A.ninst <= 2 && bytes > (128ll << 20) ? kCacheDefault : kCacheThrough;
+}
+
+template <FtlCache CP>
 __global__ __launch_bounds__(256) void ftl_expand_kernel(ExpandArgs A) {
   // The weights of every (instance, line), once per workgroup, in LDS: read
   // from there, they cost the store loop no wait on the vector-memory counter
@@ -136,17 +172,21 @@ __global__ __launch_bounds__(256) void ftl_expand_kernel(ExpandArgs A) {
   }
   const float w = rel_pos(seg, u, (float)A.npoints);
 
-  // isoline (instance, triangle, segment, line) of the capture order
-  long long iso = ((long long)tri * A.nseg + seg) * A.nlines;
-  const long long inst_stride = (long long)A.ntris * A.nseg * A.nlines;
-  for (int inst = 0; inst < A.ninst; ++inst, iso += inst_stride) {
+  // isoline (instance, triangle, segment, line) of the capture order, from the
+  // workgroup's first patch on
+  const int first = (int)(blockIdx.x * blockDim.x) / nv, run = A.nlines * nv;
+  float4* __restrict__ out = A.out + (long long)first * run;
+  const long long inst_stride = (long long)A.ntris * A.nseg * run;
+  const unsigned at = 16u * (unsigned)((ts - first) * run + v);
+  for (int inst = 0; inst < A.ninst; ++inst, out += inst_stride) {
+    const BufferRsrc b = buffer_of(out, 0x7fffffffu);
     for (int line = 0; line < A.nlines; ++line) {
       const float4 c = wts[inst * A.nlines + line];
       // mat3x4(p0, p1, p2) * c
       const float4 o = make_float4(__builtin_fmaf(c.z, g[2].x, __builtin_fmaf(c.y, g[1].x, c.x * g[0].x)),
                                    __builtin_fmaf(c.z, g[2].y, __builtin_fmaf(c.y, g[1].y, c.x * g[0].y)),
                                    __builtin_fmaf(c.z, g[2].z, __builtin_fmaf(c.y, g[1].z, c.x * g[0].z)), w);
-      A.out[(iso + line) * nv + v] = o;
+      buffer_store4<CP>(b, at + 16u * (unsigned)(line * nv), o);
     }
   }
 }
@@ -183,64 +223,69 @@ __device__ __forceinline__ void expand_sync() {
 }
 
 // Blends and stores batch b (patches b * B ...) from its guides in G0 (LDS)
-// and the blend weights in wts (LDS).  GUARD: the pass's last batch, whose
-// patches may end early.  NC > 0: the blend count, at compile time.
-template <int NV, int NC, bool GUARD, int B>
+// and the blend weights in wts (LDS).  The stores are bounded by the pass's end:
+// the last batch's patches may end early.  NC > 0: the blend count, at compile
+// time.
+template <int NV, int NC, int B, FtlCache CP>
 __device__ __forceinline__ void expand_batch(const ExpandArgs& A, const float4* G0, const float4* wts, int b,
                                              int npatch, int lane) {
   const int nseg = A.nseg, nlines = A.nlines;
-  const long long inst_stride = (long long)A.ntris * nseg * nlines;
-  float4* __restrict__ out = A.out;
+  const long long inst_stride = (long long)npatch * nlines * NV;
+  float4* __restrict__ out = A.out + (long long)b * B * nlines * NV;
+  const unsigned bytes = 16u * (unsigned)(min(B, npatch - b * B) * nlines * NV);
   const float fsub = (float)A.nsub, fpts = (float)A.npoints, scale = A.scale;
 #pragma unroll
   for (int s = 0; s < B * NV / 64; ++s) {
     const int item = s * 64 + lane;
     const int i = item / NV, v = item % NV;
-    const int patch = b * B + i;
-    if (!GUARD || patch < npatch) {
-      const float4* G = G0 + i * kGuideF4;
-      const int tri = patch / nseg, seg = patch % nseg;
-      const float u = (float)((v >> 1) + (v & 1)) / fsub;
-      const Basis h = basis(u);
-      float3 g[3];
+    const float4* G = G0 + i * kGuideF4;
+    const int seg = (b * B + i) % nseg;
+    const float u = (float)((v >> 1) + (v & 1)) / fsub;
+    const Basis h = basis(u);
+    float3 g[3];
 #pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        const float4 p0 = G[4 * q + 0], p1 = G[4 * q + 1], q0 = G[4 * q + 2], q1 = G[4 * q + 3];
-        const float3 t0 = f3(q0.x * scale, q0.y * scale, q0.z * scale);
-        const float3 t1 = f3(q1.x * scale, q1.y * scale, q1.z * scale);
-        g[q] = f3(hmix(h, p0.x, p1.x, t0.x, t1.x), hmix(h, p0.y, p1.y, t0.y, t1.y), hmix(h, p0.z, p1.z, t0.z, t1.z));
+    for (int q = 0; q < 3; ++q) {
+      const float4 p0 = G[4 * q + 0], p1 = G[4 * q + 1], q0 = G[4 * q + 2], q1 = G[4 * q + 3];
+      const float3 t0 = f3(q0.x * scale, q0.y * scale, q0.z * scale);
+      const float3 t1 = f3(q1.x * scale, q1.y * scale, q1.z * scale);
+      g[q] = f3(hmix(h, p0.x, p1.x, t0.x, t1.x), hmix(h, p0.y, p1.y, t0.y, t1.y), hmix(h, p0.z, p1.z, t0.z, t1.z));
+    }
+    const float w = rel_pos(seg, u, fpts);
+    const unsigned at = 16u * (unsigned)(i * nlines * NV + v);
+    auto blend = [&](const float4 cw) {
+      return make_float4(__builtin_fmaf(cw.z, g[2].x, __builtin_fmaf(cw.y, g[1].x, cw.x * g[0].x)),
+                         __builtin_fmaf(cw.z, g[2].y, __builtin_fmaf(cw.y, g[1].y, cw.x * g[0].y)),
+                         __builtin_fmaf(cw.z, g[2].z, __builtin_fmaf(cw.y, g[1].z, cw.x * g[0].z)), w);
+    };
+    auto store = [&](int inst, int line, const float4 o) {
+      buffer_store4<CP>(buffer_of(out + inst * inst_stride, bytes), at + 16u * (unsigned)(line * NV), o);
+    };
+    int inst = 0, line = 0;  // (counted, not divided: a scalar base for each store's buffer)
+    auto next = [&] {
+      if (++line == nlines) {
+        line = 0;
+        ++inst;
       }
-      const float w = rel_pos(seg, u, fpts);
-      const long long iso = ((long long)tri * nseg + seg) * nlines;
-      auto blend = [&](const float4 cw) {
-        return make_float4(__builtin_fmaf(cw.z, g[2].x, __builtin_fmaf(cw.y, g[1].x, cw.x * g[0].x)),
-                           __builtin_fmaf(cw.z, g[2].y, __builtin_fmaf(cw.y, g[1].y, cw.x * g[0].y)),
-                           __builtin_fmaf(cw.z, g[2].z, __builtin_fmaf(cw.y, g[1].z, cw.x * g[0].z)), w);
-      };
-      if constexpr (NC > 0) {
+    };
+    if constexpr (NC > 0) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          const int inst = c / nlines, line = c % nlines;
-          out[(iso + inst * inst_stride + line) * NV + v] = blend(wts[c]);
-        }
-      } else {
-        // (instance, line) in the capture order, four blends at a time: their
-        // weights are read from LDS together, ahead of the four stores
-        const int nc = A.ninst * nlines;
-        int inst = 0, line = 0;
-        for (int c0 = 0; c0 < nc; c0 += 4) {
-          float4 cw[4];
+      for (int c = 0; c < NC; ++c) {
+        store(inst, line, blend(wts[c]));
+        next();
+      }
+    } else {
+      // (instance, line) in the capture order, four blends at a time: their
+      // weights are read from LDS together, ahead of the four stores
+      const int nc = A.ninst * nlines;
+      for (int c0 = 0; c0 < nc; c0 += 4) {
+        float4 cw[4];
 #pragma unroll
-          for (int k = 0; k < 4; ++k) cw[k] = wts[min(c0 + k, nc - 1)];
+        for (int k = 0; k < 4; ++k) cw[k] = wts[min(c0 + k, nc - 1)];
 #pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            if (c0 + k < nc) {
-              out[(iso + inst * inst_stride + line) * NV + v] = blend(cw[k]);
-              if (++line == nlines) {
-                line = 0;
-                ++inst;
-              }
-            }
+        for (int k = 0; k < 4; ++k) {
+          if (c0 + k < nc) {
+            store(inst, line, blend(cw[k]));
+            next();
           }
         }
       }
@@ -248,7 +293,7 @@ __device__ __forceinline__ void expand_batch(const ExpandArgs& A, const float4* 
   }
 }
 
-template <int NV, int NC, int B>
+template <int NV, int NC, int B, FtlCache CP>
 __global__ __launch_bounds__(64) void ftl_expand_batched_kernel(ExpandArgs A) {
   static_assert(NV % 2 == 0 && (B * NV) % 64 == 0 && B <= 64, "whole patches per wave-wide step");
   constexpr int kGuides = B * kGuideF4;
@@ -289,10 +334,7 @@ __global__ __launch_bounds__(64) void ftl_expand_batched_kernel(ExpandArgs A) {
 #pragma unroll
   for (int r = 0; r < kRuns; ++r) gd[guide_index(r)] = gv[r];
   expand_sync();
-  if ((b + 1) * B <= npatch)
-    expand_batch<NV, NC, false, B>(A, gd, wts, b, npatch, lane);
-  else
-    expand_batch<NV, NC, true, B>(A, gd, wts, b, npatch, lane);
+  expand_batch<NV, NC, B, CP>(A, gd, wts, b, npatch, lane);
 }
 
 // The same pass by pages of the output.  For one instance the capture of
@@ -317,7 +359,7 @@ constexpr int kPage = 256, kPageRows = kPage / 64;
 constexpr int page_patches(int run) { return (kPage - 1 + run - 1) / run + 1; }
 
 // ONE: one line per patch.
-template <bool ONE>
+template <bool ONE, FtlCache CP>
 __global__ __launch_bounds__(64) void ftl_expand_page_kernel(ExpandArgs A, long long total) {
   extern __shared__ float4 sm[];
   const int nlines = ONE ? 1 : A.nlines, nv = 2 * A.nsub;
@@ -382,8 +424,8 @@ __global__ __launch_bounds__(64) void ftl_expand_page_kernel(ExpandArgs A, long 
     }
     w[s] = rel_step(ju[i] + uu[v]);
   }
-  float4* __restrict__ out = A.out + base + lane;
-  const bool whole = base + kPage <= total;
+  float4* __restrict__ out = A.out + base;
+  const unsigned bytes = 16u * (unsigned)min((long long)kPage, total - base);
   for (int inst = 0; inst < A.ninst; ++inst, out += total) {
     float4 o[kPageRows];
 #pragma unroll
@@ -393,9 +435,9 @@ __global__ __launch_bounds__(64) void ftl_expand_page_kernel(ExpandArgs A, long 
                          __builtin_fmaf(c.z, g[s][2].y, __builtin_fmaf(c.y, g[s][1].y, c.x * g[s][0].y)),
                          __builtin_fmaf(c.z, g[s][2].z, __builtin_fmaf(c.y, g[s][1].z, c.x * g[s][0].z)), w[s]);
     }
+    const BufferRsrc b = buffer_of(out, bytes);
 #pragma unroll
-    for (int s = 0; s < kPageRows; ++s)
-      if (whole || base + 64 * s + lane < total) out[64 * s] = o[s];
+    for (int s = 0; s < kPageRows; ++s) buffer_store4<CP>(b, 16u * (unsigned)(64 * s + lane), o[s]);
   }
 }
 
@@ -422,10 +464,14 @@ bool launch_expand_page_if_faster(const ExpandArgs& A, int nc, hipStream_t strea
   const size_t lds = ((size_t)nc + nv + (size_t)np * kGuideF4 + np) * sizeof(float4) + (size_t)(np + nv) * sizeof(float);
   if (lds > 64 * 1024) return false;
   const dim3 grid((unsigned)((total + kPage - 1) / kPage)), block(64);
-  if (A.nlines == 1)
-    hipLaunchKernelGGL(ftl_expand_page_kernel<true>, grid, block, lds, stream, A, total);
-  else
-    hipLaunchKernelGGL(ftl_expand_page_kernel<false>, grid, block, lds, stream, A, total);
+  const FtlCache cp = run_cache(A, true);
+  if (A.nlines == 1) {
+    FTL_WITH_CACHE(cp, hipLaunchKernelGGL((ftl_expand_page_kernel<true, CP>), grid, block, lds, stream, A, total))
+  } else if (cp == kCacheStream) {
+    hipLaunchKernelGGL((ftl_expand_page_kernel<false, kCacheStream>), grid, block, lds, stream, A, total);
+  } else {
+    hipLaunchKernelGGL((ftl_expand_page_kernel<false, kCacheThrough>), grid, block, lds, stream, A, total);
+  }
   return true;
 }
 
@@ -439,11 +485,14 @@ void launch_expand_batched(const ExpandArgs& A, int nc, hipStream_t stream) {
   const size_t lds = (size_t)nc * sizeof(float4) + (size_t)B * kGuideF4 * sizeof(float4) + B * sizeof(int4);
   if constexpr (NSUB == 16) {
     if (nc == 6) {
-      hipLaunchKernelGGL((ftl_expand_batched_kernel<NV, 6, B>), dim3(nbatch), dim3(64), lds, stream, A);
+      hipLaunchKernelGGL((ftl_expand_batched_kernel<NV, 6, B, kCacheThrough>), dim3(nbatch), dim3(64), lds, stream, A);
       return;
     }
   }
-  hipLaunchKernelGGL((ftl_expand_batched_kernel<NV, 0, B>), dim3(nbatch), dim3(64), lds, stream, A);
+  if (run_cache(A, false) == kCacheStream)
+    hipLaunchKernelGGL((ftl_expand_batched_kernel<NV, 0, B, kCacheStream>), dim3(nbatch), dim3(64), lds, stream, A);
+  else
+    hipLaunchKernelGGL((ftl_expand_batched_kernel<NV, 0, B, kCacheThrough>), dim3(nbatch), dim3(64), lds, stream, A);
 }
 
 // Launches the batched pass where it measured faster than ftl_expand_kernel
@@ -633,7 +682,10 @@ extern "C" ftl_status ftl_expand_run(ftl_expand* e, const ftl_expand_params* p, 
   if (!launch_expand_batched_if_faster(A, p->nsubsegments, nc, (hipStream_t)stream) &&
       !launch_expand_page_if_faster(A, nc, (hipStream_t)stream)) {
     const int blocks = (int)((nthreads + 255) / 256);
-    hipLaunchKernelGGL(ftl_expand_kernel, dim3(blocks), dim3(256), lds, (hipStream_t)stream, A);
+    if (vertex_cache(A) == kCacheThrough)
+      hipLaunchKernelGGL(ftl_expand_kernel<kCacheThrough>, dim3(blocks), dim3(256), lds, (hipStream_t)stream, A);
+    else
+      hipLaunchKernelGGL(ftl_expand_kernel<kCacheDefault>, dim3(blocks), dim3(256), lds, (hipStream_t)stream, A);
   }
   if ((he = hipGetLastError()) != hipSuccess) return ftl_hip_fail(he, "ftl_expand_kernel launch");
   return FTL_OK;

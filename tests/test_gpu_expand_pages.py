@@ -36,3 +36,21 @@ def test_one_line(ctx, T, ninst, nsub):
 def test_large_outputs(ctx, ninst, nlines, nsub):
     per = 2 * ninst * nlines * nsub * 15
     check(ctx, 2000, 16, (384 << 20) // (16 * per) + 3, ninst, nlines, nsub)
+
+
+@pytest.mark.parametrize("above", [-1, 2])
+@pytest.mark.parametrize("mb,ninst,nlines,nsub", [(128, 2, 1, 13), (224, 1, 1, 15), (224, 2, 1, 8), (224, 1, 3, 16),
+                                                  (256, 2, 3, 6), (144, 3, 2, 9), (256, 4, 3, 8), (400, 3, 2, 7)])
+def test_cache_lines(ctx, mb, ninst, nlines, nsub, above):
+    """On both sides of the output sizes at which a form changes how its stores
+    use the caches: pages, batches and single vertices, with ends that fill no
+    page, batch or workgroup."""
+    per = 2 * ninst * nlines * nsub * 15
+    check(ctx, 2000, 16, (mb << 20) // (16 * per) + above, ninst, nlines, nsub)
+
+
+@pytest.mark.parametrize("T", [1, 2, 5, 13, 129])
+@pytest.mark.parametrize("ninst,nlines,nsub", [(1, 1, 1), (3, 2, 5), (2, 5, 2), (1, 1, 8), (3, 2, 16), (5, 2, 12), (8, 4, 64)])
+def test_ends(ctx, T, ninst, nlines, nsub):
+    """The last batch and the last workgroup hold fewer patches."""
+    check(ctx, 40, 4, T, ninst, nlines, nsub)
