@@ -200,34 +200,51 @@ __device__ __forceinline__ float pow_c(float x, float y) { return x == 0.0f ? 0.
 // Written out so the new position is produced in p's own registers (the
 // compiler otherwise builds it in temporaries and copies it back every point).
 // VALU instructions only; no memory access.
+#define FTL_POINT_ASM(p0, p1, p2, l0, l1, l2, sl)     \
+  "v_sub_f32 %[d0], %[" p0 "], %[" l0 "]\n\t"         \
+  "v_sub_f32 %[d1], %[" p1 "], %[" l1 "]\n\t"         \
+  "v_sub_f32 %[d2], %[" p2 "], %[" l2 "]\n\t"         \
+  "v_mul_f32 %[x], %[d0], %[d0]\n\t"                 \
+  "v_fmac_f32 %[x], %[d1], %[d1]\n\t"                \
+  "v_fmac_f32 %[x], %[d2], %[d2]\n\t"                \
+  "v_lshrrev_b32 %[y], 1, %[x]\n\t"                  \
+  "v_sub_u32 %[y], 0x5f3759df, %[y]\n\t"             \
+  "v_mul_f32 %[x], -0.5, %[x]\n\t"                   \
+  "v_mul_f32 %[t], %[y], %[y]\n\t"                   \
+  "v_fmaak_f32 %[t], %[x], %[t], 0x3fc00000\n\t"     \
+  "v_mul_f32 %[y], %[y], %[t]\n\t"                   \
+  "v_mul_f32 %[t], %[y], %[y]\n\t"                   \
+  "v_fmaak_f32 %[t], %[x], %[t], 0x3fc00000\n\t"     \
+  "v_mul_f32 %[y], %[y], %[t]\n\t"                   \
+  "v_mul_f32 %[t], %[y], %[y]\n\t"                   \
+  "v_fmaak_f32 %[t], %[x], %[t], 0x3fc00000\n\t"     \
+  "v_mul_f32 %[y], %[y], %[t]\n\t"                   \
+  "v_mul_f32 %[y], %[" sl "], %[y]\n\t"              \
+  "v_fma_f32 %[" p0 "], %[y], %[d0], %[" l0 "]\n\t"   \
+  "v_fma_f32 %[" p1 "], %[y], %[d1], %[" l1 "]\n\t"   \
+  "v_fma_f32 %[" p2 "], %[y], %[d2], %[" l2 "]\n\t"
+
 __device__ __forceinline__ void ftl_point(float3& p, const float3 lead, const float sl) {
-  float d0, d1, d2, x, y, t, s;
-  asm(
-      "v_sub_f32 %[d0], %[p0], %[l0]\n\t"
-      "v_sub_f32 %[d1], %[p1], %[l1]\n\t"
-      "v_sub_f32 %[d2], %[p2], %[l2]\n\t"
-      "v_mul_f32 %[x], %[d0], %[d0]\n\t"
-      "v_fmac_f32 %[x], %[d1], %[d1]\n\t"
-      "v_fmac_f32 %[x], %[d2], %[d2]\n\t"
-      "v_lshrrev_b32 %[y], 1, %[x]\n\t"
-      "v_sub_u32 %[y], 0x5f3759df, %[y]\n\t"
-      "v_mul_f32 %[x], -0.5, %[x]\n\t"
-      "v_mul_f32 %[t], %[y], %[y]\n\t"
-      "v_fmaak_f32 %[t], %[x], %[t], 0x3fc00000\n\t"
-      "v_mul_f32 %[y], %[y], %[t]\n\t"
-      "v_mul_f32 %[t], %[y], %[y]\n\t"
-      "v_fmaak_f32 %[t], %[x], %[t], 0x3fc00000\n\t"
-      "v_mul_f32 %[y], %[y], %[t]\n\t"
-      "v_mul_f32 %[t], %[y], %[y]\n\t"
-      "v_fmaak_f32 %[t], %[x], %[t], 0x3fc00000\n\t"
-      "v_mul_f32 %[y], %[y], %[t]\n\t"
-      "v_mul_f32 %[s], %[sl], %[y]\n\t"
-      "v_fma_f32 %[p0], %[s], %[d0], %[l0]\n\t"
-      "v_fma_f32 %[p1], %[s], %[d1], %[l1]\n\t"
-      "v_fma_f32 %[p2], %[s], %[d2], %[l2]"
+  float d0, d1, d2, x, y, t;
+  asm(FTL_POINT_ASM("p0", "p1", "p2", "l0", "l1", "l2", "sl")
       : [p0] "+v"(p.x), [p1] "+v"(p.y), [p2] "+v"(p.z), [d0] "=&v"(d0), [d1] "=&v"(d1), [d2] "=&v"(d2),
-        [x] "=&v"(x), [y] "=&v"(y), [t] "=&v"(t), [s] "=&v"(s)
+        [x] "=&v"(x), [y] "=&v"(y), [t] "=&v"(t)
       : [l0] "v"(lead.x), [l1] "v"(lead.y), [l2] "v"(lead.z), [sl] "v"(sl));
+}
+
+// Three consecutive points, each the next one's leader.  (Between two
+// statements that share registers the compiler places a wait state, which it
+// cannot see is unneeded.)
+__device__ __forceinline__ void ftl_points3(float3& p, float3& q, float3& r, const float3 lead, const float sp,
+                                            const float sq, const float sr) {
+  float d0, d1, d2, x, y, t;
+  asm(FTL_POINT_ASM("p0", "p1", "p2", "l0", "l1", "l2", "sp")
+      FTL_POINT_ASM("q0", "q1", "q2", "p0", "p1", "p2", "sq")
+      FTL_POINT_ASM("r0", "r1", "r2", "q0", "q1", "q2", "sr")
+      : [p0] "+&v"(p.x), [p1] "+&v"(p.y), [p2] "+&v"(p.z), [q0] "+&v"(q.x), [q1] "+&v"(q.y), [q2] "+&v"(q.z),
+        [r0] "+&v"(r.x), [r1] "+&v"(r.y), [r2] "+&v"(r.z), [d0] "=&v"(d0), [d1] "=&v"(d1), [d2] "=&v"(d2),
+        [x] "=&v"(x), [y] "=&v"(y), [t] "=&v"(t)
+      : [l0] "v"(lead.x), [l1] "v"(lead.y), [l2] "v"(lead.z), [sp] "v"(sp), [sq] "v"(sq), [sr] "v"(sr));
 }
 
 // Root transform: row c = fma(m_c0, x, fma(m_c1, y, fma(m_c2, z, t_c))).

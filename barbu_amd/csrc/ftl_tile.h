@@ -235,9 +235,20 @@ __device__ __forceinline__ void flush_velocities(BufferRsrc dst, int N, int c, c
 // several waves share a SIMD.  Each point still meets the colliders in order
 // with the same operations.  Point j takes part when on && j < jend && (j > 0
 // || on0).
+//
+// Lanes of more than four points take them in pairs: where strands lie against
+// a collider, every point of the wave is hit by some lane, and a hit is a serial
+// chain of 15 instructions.  A pair's chains run side by side on all lanes,
+// and only the three that write a point run under its hits' mask (kernel us
+// point by point and in pairs: 262k x 32, one collider 110.9, 107.5, two in
+// wind 131.0, 128.5; 50k x 64 at 16 iterations 84.0, 81.8).  Shorter lanes do
+// not: there the launch runs eight waves to a SIMD, which cover the chain
+// (1M x 4 59.0, 61.0), or one, where the longer code counts (4k x 16 9.1, 9.8).
 template <int M>
 __device__ __forceinline__ void collide_sweep(const Spheres& S, float3 (&p)[M], bool on, bool on0, int jend,
                                               int n) {
+  constexpr bool kPairs = M > 4 && M % 2 == 0;
+  if (kPairs && !on) return;
 #pragma unroll
   for (int k = 0; k < FTL_NCOL; ++k) {
     if (!more_colliders(n, k)) break;
@@ -245,15 +256,64 @@ __device__ __forceinline__ void collide_sweep(const Spheres& S, float3 (&p)[M], 
     // (with one or two points the copies cost more than they save)
     if constexpr (M > 2) asm volatile("" : "+v"(cx), "+v"(cy), "+v"(cz), "+v"(r2));
     const float3 c = f3(cx, cy, cz);
+    if constexpr (kPairs) {
 #pragma unroll
-    for (int j = 0; j < M; ++j) {
-      if (j >= jend) continue;
-      const float3 w = sub3(p[j], c);
-      const float dp = dot3(w, w);
-      if (on && (j > 0 || on0) && dp < r2) {
-        const float is = rsqrt_c(dp);
-        p[j] = fma3(S.r[k], mul3(w, is), c);
+      for (int j = 0; j < M; j += 2) {
+        float3 w[2];
+        float d[2];
+        unsigned long long hit[2];  // the lanes whose point is hit
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          w[i] = sub3(p[j + i], c);
+          d[i] = dot3(w[i], w[i]);
+          hit[i] = __ballot(d[i] < r2 && (j + i > 0 || on0) && j + i < jend);
+        }
+        if ((hit[0] | hit[1]) == 0) continue;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) w[i] = mul3(w[i], rsqrt_c(d[i]));
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          float3& q = p[j + i];
+          unsigned long long lanes;
+          asm("s_and_saveexec_b64 %[s], %[h]\n\t"
+              "v_fma_f32 %[x], %[r], %[wx], %[cx]\n\t"
+              "v_fma_f32 %[y], %[r], %[wy], %[cy]\n\t"
+              "v_fma_f32 %[z], %[r], %[wz], %[cz]\n\t"
+              "s_mov_b64 exec, %[s]"
+              : [x] "+v"(q.x), [y] "+v"(q.y), [z] "+v"(q.z), [s] "=&s"(lanes)
+              : [h] "s"(hit[i]), [r] "s"(S.r[k]), [wx] "v"(w[i].x), [wy] "v"(w[i].y), [wz] "v"(w[i].z), [cx] "v"(cx),
+                [cy] "v"(cy), [cz] "v"(cz)
+              : "scc");
+        }
       }
+    } else {
+#pragma unroll
+      for (int j = 0; j < M; ++j) {
+        if (j >= jend) continue;
+        const float3 w = sub3(p[j], c);
+        const float dp = dot3(w, w);
+        if (on && (j > 0 || on0) && dp < r2) {
+          const float is = rsqrt_c(dp);
+          p[j] = fma3(S.r[k], mul3(w, is), c);
+        }
+      }
+    }
+  }
+}
+
+// Points 1 .. M - 1 of a lane, each led by the one before it.  The points are
+// updated in their own registers under the lane mask (a select would be three
+// vector instructions with a scalar mask operand); a point's leader is the
+// previous point before that point's collision.  len(j): sigma * rest length.
+template <int M, typename Len>
+__device__ __forceinline__ void sweep_points(float3 (&p)[M], Len len) {
+#pragma unroll
+  for (int j = 1; j < M; j += 3) {
+    if (j + 2 < M) {
+      ftl_points3(p[j], p[j + 1], p[j + 2], p[j - 1], len(j), len(j + 1), len(j + 2));
+    } else {
+      ftl_point(p[j], p[j - 1], len(j));
+      if (j + 1 < M) ftl_point(p[j + 1], p[j], len(j + 1));
     }
   }
 }
@@ -274,6 +334,16 @@ __device__ __forceinline__ void sweep(const FtlStep& A, const VelArgs& V, const 
   float sg = A.sigma;
   asm volatile("" : "+v"(sg));
   const float dl = V.delta;
+  if (!FINAL) {
+    sweep_points<M>(p, [&](int j) { return sg * l.get(j); });
+#pragma unroll
+    for (int j = 1; j < M; ++j)
+      if (GUARD ? j == nl - 1 : j == M - 1) last_pre = p[j];
+    // Collisions of points 1 .. last (the root never collides; with GUARD the
+    // slots past the last point are not collided at all).
+    collide_sweep<M>(S, p, true, false, GUARD ? nl : M, cm);
+    return;
+  }
 #pragma unroll
   for (int j = 1; j < M; ++j) {
     // GUARD: slots j >= nl hold copies of the last point; they are swept like
@@ -282,36 +352,29 @@ __device__ __forceinline__ void sweep(const FtlStep& A, const VelArgs& V, const 
     const float3 q = p[j];
     ftl_point(p[j], p[j - 1], sg * l.get(j));
     const float3 pn = p[j];
-    if (FINAL) {
-      const float3 c = sub3(pn, q);
-      if (!GUARD || j < nl) {
-        // Point m = j-1 is final: u = delta * c_j.  The root keeps its own,
-        // p0 - x0 (:192), formed here from x0, which is still in memory.
-        const int m = j - 1;
-        float3 pm = p[m];
-        float3 u = mul3(c, dl);
-        if (m == 0) {
-          const float4 x0 = pp[0];
-          u = sub3(pm, f3(x0.x, x0.y, x0.z));
-        } else {
-          collide<true>(S, pm, u, cm);
-        }
-        p[m] = pm;
-        const float3 v = out_velocity(V, pp, m, pm, u);
-        stage[slot<C>(lane, m % C)] = make_float4(v.x, v.y, v.z, 0.0f);
-        if (m % C == C - 1) flush_chunk<M, 1, GUARD, CP>(bvel, N, m / C, stage, lane);
+    const float3 c = sub3(pn, q);
+    if (!GUARD || j < nl) {
+      // Point m = j-1 is final: u = delta * c_j.  The root keeps its own,
+      // p0 - x0 (:192), formed here from x0, which is still in memory.
+      const int m = j - 1;
+      float3 pm = p[m];
+      float3 u = mul3(c, dl);
+      if (m == 0) {
+        const float4 x0 = pp[0];
+        u = sub3(pm, f3(x0.x, x0.y, x0.z));
+      } else {
+        collide<true>(S, pm, u, cm);
       }
-      if (GUARD ? (j == nl - 1) : (j == M - 1)) {
-        clast = c;
-        last_pre = pn;
-      }
-    } else if (GUARD ? (j == nl - 1) : (j == M - 1)) {
+      p[m] = pm;
+      const float3 v = out_velocity(V, pp, m, pm, u);
+      stage[slot<C>(lane, m % C)] = make_float4(v.x, v.y, v.z, 0.0f);
+      if (m % C == C - 1) flush_chunk<M, 1, GUARD, CP>(bvel, N, m / C, stage, lane);
+    }
+    if (GUARD ? (j == nl - 1) : (j == M - 1)) {
+      clast = c;
       last_pre = pn;
     }
   }
-  // Collisions of points 1 .. last (the root never collides; with GUARD the
-  // slots past the last point are not collided at all).
-  if (!FINAL) collide_sweep<M>(S, p, true, false, GUARD ? nl : M, cm);
 }
 
 // The value of the previous lane of the same row of 16 lanes (DPP row_shr:1,
@@ -349,13 +412,9 @@ __device__ __forceinline__ void sweep_pipe(const Spheres& S, float3 (&p)[M], con
       }
     }
   }
-#pragma unroll
-  for (int j = 0; j < M; ++j) {
-    const bool upd = active && (j != 0 || g != 0);  // lane 0's slot 0 is the root
-    // The point is updated in its own registers under the lane mask (a select
-    // would be three vector instructions with a scalar mask operand); its
-    // leader is the previous point before that point's collision.
-    if (upd) ftl_point(p[j], j == 0 ? lead : p[j - 1], l.get(j));  // l holds sigma * rest length
+  if (active) {
+    if (g != 0) ftl_point(p[0], lead, l.get(0));  // (lane 0's slot 0 is the root)
+    sweep_points<M>(p, [&](int j) { return l.get(j); });  // l holds sigma * rest length
   }
   // (An inactive lane's value is read only by the next lane while that lane is
   // inactive too: fill and drain shift by one step per lane.)
