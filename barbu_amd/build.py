@@ -43,6 +43,9 @@ def _units():
                       "plain_%d.o" % k))
     for g in (2, 4, 8, 16, 0):  # the wide forms by lanes per strand; 0: all of them in one kernel
         units.append(("ftl_wide.hip", ["-DFTL_WIDE_LANES=%d" % g], "wide_%d.o" % g))
+    for c in (0, 1, 2):  # the kernel of mixed batches, by its use of the caches
+        units.append(("ftl_tiles_all.hip", ["-DFTL_CACHE=%d" % c, "-mllvm", "-pragma-unroll-threshold=200000"],
+                      "tiles_all_%d.o" % c))
     for src in ("ftl_misc.hip", "ftl_render.hip", "ftl_init.hip", "ftl_marschner.hip", "ftl_api.cpp", "ftl_batch_api.cpp", "ftl_autotune.cpp",
                 "ftl_scenario.cpp", "ftl_server.cpp"):
         units.append((src, [], os.path.splitext(src)[0] + ".o"))

@@ -60,8 +60,10 @@ static double class_ns_per_cp(const ftl_ctx* ctx, int cls, int K) {
 
 // Plans the tiles of a set of grooms as one span per groom: a batch whose
 // waves all fit the chip at once is one launch of the wide forms' common
-// kernel, each groom in the form of the batch's level; otherwise the grooms
-// are grouped by launch class or wide form (the one with the most expected
+// kernel, each groom in the form of the batch's level; a larger one of several
+// classes or wide forms is one launch of FTL_TILES_ALL, its costliest tiles
+// first; otherwise (one class, lanes set by hand, classes of two waves per
+// SIMD) the grooms are grouped by class or form (the one with the most expected
 // work first; within it, grooms with more iterations first).  Linear in the
 // number of grooms: the serving loop plans a batch per launch.
 ftl_status ftl_plan_tiles(ftl_ctx* ctx, ftl_groom* const* grooms, int n, std::vector<FtlSpan>& spans,
@@ -101,6 +103,16 @@ ftl_status ftl_plan_tiles(ftl_ctx* ctx, ftl_groom* const* grooms, int n, std::ve
     work[run] += class_ns_per_cp(ctx, cls, g->params.iterations) * (double)FTL_WAVE * km * nt;
     total_tiles += (size_t)nt;
     state_bytes += (size_t)g->nstrands * g->npoints * 2 * sizeof(float4);
+  }
+  // Several classes or forms that one kernel holds: that kernel (figures there).
+  if (automatic && level == 0) {
+    bool several = false, held = true;
+    for (const GroomPlan& gp : plan) {
+      several = several || gp.run != plan[0].run;
+      held = held && ftl_in_tiles_all(gp.cls);
+    }
+    if (several && held)
+      for (GroomPlan& gp : plan) gp.run = FTL_TILES_ALL;
   }
   // the class kernels of a batch run together: the batch's whole state decides
   const FtlCache cp = ftl_cache_for(state_bytes);

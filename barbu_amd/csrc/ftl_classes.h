@@ -95,3 +95,14 @@ constexpr int ftl_wide_id(int m, int g) { return 256 + 32 * m + g; }
 constexpr int ftl_wide_m(int id) { return (id - 256) / 32; }
 constexpr int ftl_wide_g(int id) { return (id - 256) % 32; }
 #define FTL_WIDE_ALL 128
+
+// The exact classes that run four or more waves per SIMD, the class of 2 and 3
+// points, and the forms of the other point counts in launches that fill the
+// chip, all in one kernel.
+#define FTL_TILES_ALL 129
+#define FTL_DEFAULT_CLASSES(X)                                                              \
+  X(0, 4, 1, false) X(1, 8, 1, false) X(2, 16, 1, false) X(4, 8, 2, false) X(5, 16, 2, false) \
+  X(7, 4, 4, false) X(8, 8, 4, false) X(9, 16, 4, false) X(10, 4, 1, true) X(15, 4, 2, false)
+#define FTL_DEFAULT_FORMS(X)                                            \
+  X(3, 2) X(4, 2) X(5, 2) X(6, 2) X(7, 2) X(8, 2)                       \
+  X(5, 4) X(6, 4) X(7, 4) X(8, 4) X(5, 8) X(6, 8) X(7, 8) X(8, 8)

@@ -48,9 +48,11 @@ int ftl_wide_form(int level, int npoints);
 // The plain step of one groom by a wide form.
 hipError_t ftl_launch_wide(int form, const FtlStep& A, hipStream_t stream, hipEvent_t start = nullptr,
                            hipEvent_t stop = nullptr);
+// Whether FTL_TILES_ALL holds a launch class or wide form.
+bool ftl_in_tiles_all(int cls);
 // Tile-list kernel of one class over the ntiles tiles of spans[0..nspans)
 // (every groom of that class, in tile order): workgroup b steps tiles b,
-// b + grid, ...  cls may be a wide form (ftl_wide_id) or FTL_WIDE_ALL, one
+// b + grid, ...  cls may be a wide form (ftl_wide_id), FTL_WIDE_ALL or FTL_TILES_ALL, one
 // workgroup per tile.
 hipError_t ftl_launch_tiles(int cls, const FtlStep* grooms, const FtlSpan* spans, int nspans, int ntiles, int grid,
                             hipStream_t stream, FtlCache cp);

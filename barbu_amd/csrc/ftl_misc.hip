@@ -215,6 +215,23 @@ FTL_WDECL(8)
 FTL_WDECL(16)
 #undef FTL_WDECL
 hipError_t ftl_launch_wide_all(const FtlStep*, const FtlSpan*, int, int, hipStream_t);
+#define FTL_ADECL(C) hipError_t ftl_launch_tiles_all_##C(const FtlStep*, const FtlSpan*, int, int, hipStream_t);
+FTL_ADECL(0)
+FTL_ADECL(1)
+FTL_ADECL(2)
+#undef FTL_ADECL
+
+bool ftl_in_tiles_all(int cls) {
+  switch (cls) {
+#define FTL_AC(id, M, G, GU) case id:
+#define FTL_AW(M, G) case ftl_wide_id(M, G):
+    FTL_DEFAULT_CLASSES(FTL_AC) FTL_DEFAULT_FORMS(FTL_AW)
+#undef FTL_AC
+#undef FTL_AW
+    return true;
+  }
+  return false;
+}
 
 // Lanes per strand of an npoints groom in a launch of this level.
 static int wide_lanes(int level, int npoints) {
@@ -284,6 +301,13 @@ hipError_t ftl_launch_tiles(int cls, const FtlStep* grooms, const FtlSpan* spans
   if (cls == FTL_WIDE_ALL) {
     if (ntiles <= 0 || nspans <= 0) return hipSuccess;
     return ftl_launch_wide_all(grooms, spans, nspans, ntiles, stream);
+  }
+  if (cls == FTL_TILES_ALL) {
+    if (ntiles <= 0 || nspans <= 0) return hipSuccess;
+    static_assert(kCacheDefault == 0 && kCacheThrough == 1 && kCacheStream == 2, "the units' names");
+    return (cp == kCacheDefault   ? ftl_launch_tiles_all_0
+            : cp == kCacheThrough ? ftl_launch_tiles_all_1
+                                  : ftl_launch_tiles_all_2)(grooms, spans, nspans, ntiles, stream);
   }
   if (cls >= ftl_wide_id(0, 0)) {
     if (ntiles <= 0 || nspans <= 0) return hipSuccess;

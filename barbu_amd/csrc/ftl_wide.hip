@@ -5,7 +5,6 @@
 #include <hip/hip_ext.h>
 
 #include "ftl_launch.h"
-#include "ftl_launch.h"
 #include "ftl_wide.h"
 
 #ifndef FTL_WIDE_LANES

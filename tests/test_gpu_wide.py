@@ -6,7 +6,8 @@ import numpy as np
 import pytest
 
 import barbu_amd as ba
-from tests.helpers import assert_bitexact
+from oracle import ftl_oracle as orc
+from tests.helpers import assert_bitexact, oracle_params_for
 from tests.test_gpu_parity import DT, _oracle_frame, _rigid, run_compare
 
 pytestmark = pytest.mark.gpu
@@ -99,3 +100,43 @@ def test_batch_levels(ctx, scale):
             assert_bitexact(p, s["pos"], "groom %d frame %d positions" % (i, k))
             assert_bitexact(v, s["vel"], "groom %d frame %d velocities" % (i, k))
     b.close()
+
+
+@pytest.mark.parametrize("wind,dftl,iterations", [(0, 0, 2), (1, 0, 1), (0, 1, 3)])
+def test_mixed_batch(ctx, wind, dftl, iterations):
+    """A batch past the last level whose grooms need every class and form: one
+    kernel, whichever of them a groom's point count names, partial tiles in
+    all.  Stepped as a batch object, at once, and by class."""
+    grooms, states = [], []
+    params = ba.make_params(force_scale=1.0, damping=0.9, length_scale=1.0, iterations=iterations, velocity_mode=dftl,
+                            max_velocity=2.0, wind_amplitude=2.0 * wind, wind_frequency=2.0, wind_seed=5)
+    for i, n in enumerate([2, 3, 4, 5, 6, 8, 9, 11, 13, 15, 16, 17, 20, 24, 25, 32, 33, 40, 41, 48, 49, 56, 57, 63, 64]):
+        pos, vel, roots = scene(3000 + 37 * i, n, 300 + i)
+        g = ba.Groom(ctx, pos, vel, rest_roots=roots)
+        g.set_params(params)
+        g.set_root_mode(ba.FTL_ROOT_REST)
+        g.set_colliders(np.float32(SPHERES))
+        g.set_root_transform(_rigid(0, i))
+        grooms.append(g)
+        states.append((pos.copy(), vel.copy(), roots))
+    table = ba.wind_table(params) if wind else None
+    b = ba.Batch(ctx, grooms)
+    for k in range(3):
+        if k == 0:
+            b.launch([DT] * len(grooms))
+        elif k == 1:
+            ba.batch_step(ctx, grooms, [DT] * len(grooms))
+        else:  # by class again: some grooms' lanes are set
+            for g in grooms[::5]:
+                g.set_lanes(1)
+            ba.batch_step(ctx, grooms, [DT] * len(grooms))
+        for i, (g, (pos, vel, roots)) in enumerate(zip(grooms, states)):
+            op = oracle_params_for(params, pos.shape[1], DT, spheres=SPHERES, model=_rigid(0, i),
+                                   root_mode=ba.FTL_ROOT_REST, wind=table)
+            orc.step_f32(op, pos, vel, roots)
+            p, v = g.download()
+            assert_bitexact(p, pos, "groom %d step %d positions" % (i, k))
+            assert_bitexact(v, vel, "groom %d step %d velocities" % (i, k))
+    b.close()
+    for g in grooms:
+        g.close()
