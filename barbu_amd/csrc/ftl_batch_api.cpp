@@ -1,20 +1,19 @@
 // Batched FTL steps: many grooms, uneven strand and point counts, stepped by
-// one graph launch per frame (or, when they make one kernel, by that kernel
-// after the upload).  There is no counterpart in the reference, which
-// dispatches one workgroup per strand of its single groom (src/fx/hair.cc:112).
+// one kernel per frame after the upload of their descriptors (or, when they
+// need a kernel per launch class, by one graph launch).  There is no
+// counterpart in the reference, which dispatches one workgroup per strand of
+// its single groom (src/fx/hair.cc:112).
 //
 // A batch is planned once: each groom is cut into 64-lane tiles of its launch
-// class (points per lane x lanes per strand), and the grooms are grouped by
-// class, each a span of consecutive tiles of its class's launch (one record
-// per groom: the kernel maps a tile to its groom by a search over the
-// spans).  Every class has its own tile-list kernel, compiled with the register
-// budget of that class (one kernel for all classes would carry the register
-// count of the heaviest one); a small batch runs the wide forms' common kernel
-// (ftl_plan_tiles).  A frame is [upload the per-groom descriptors
-// from pinned memory -> one tile-list kernel per class present, as parallel
-// branches], captured once into a HIP graph: one graph launch steps every
-// groom.  Two graphs with their own pinned descriptor buffers alternate, so
-// the host prepares frame k+1 while frame k runs.
+// class or wide form (points per lane x lanes per strand), a span of
+// consecutive tiles of the launch (one record per groom: the kernel maps a
+// tile to its groom by a search over the spans).  ftl_plan_tiles says which
+// kernel takes the spans.  A batch of several kernels is [upload the
+// per-groom descriptors from pinned memory -> one tile-list kernel per class
+// present, as parallel branches], captured once into a HIP graph (a batch of
+// one kernel has its graph too, for launches on a stream that is being
+// captured).  Two descriptor buffers (and graphs) alternate, so the host prepares frame k+1
+// while frame k runs.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -375,7 +374,6 @@ extern "C" ftl_status ftl_batch_create(ftl_ctx* ctx, ftl_groom* const* grooms, i
     std::memset(b->h_steps[k], 0, sb);
     if ((e = hipEventCreateWithFlags(&b->done[k], hipEventDisableTiming)) != hipSuccess)
       return bail(ftl_hip_fail(e, "hipEventCreate"));
-    if (runs.size() == 1) continue;  // launched directly: see ftl_batch_launch
     if ((e = hipStreamBeginCapture(b->cap, hipStreamCaptureModeThreadLocal)) != hipSuccess)
       return bail(ftl_hip_fail(e, "hipStreamBeginCapture"));
     hipError_t e1 = FTL_KERNEL_UPLOAD ? ftl_launch_upload(b->h_steps[k], b->d_steps[k], sb, b->cap)
@@ -435,7 +433,14 @@ extern "C" ftl_status ftl_batch_launch(ftl_batch* b, const float* dt, void* stre
     ftl_status st = ftl_make_step(b->grooms[i], dt[i], &b->h_steps[k][i]);
     if (st != FTL_OK) return st;
   }
-  if (b->runs.size() == 1) {
+  // A launch recorded into a capture of the caller's would read the batch's
+  // buffers at every replay, whatever has become of them: there the graph is
+  // launched, which the runtime runs at once.
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  const bool capturing =
+      hipStreamIsCapturing((hipStream_t)stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
+  if (capturing) (void)hipGetLastError();
+  if (b->runs.size() == 1 && !capturing) {
     // One kernel after the upload: two launches on the caller's stream follow
     // each other closer than the nodes of a graph do (a frame of 24 small
     // grooms: 27.6 us, as a graph 34.7).

@@ -2,10 +2,13 @@
 launches at each level, point counts around the edges of the lanes' shares,
 partial tiles, and the ragged point counts of launches that fill the chip.
 They perform the oracle's operations in the oracle's order: bit for bit."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import barbu_amd as ba
+from barbu_amd import _hip as hipm
 from oracle import ftl_oracle as orc
 from tests.helpers import assert_bitexact, oracle_params_for
 from tests.test_gpu_parity import DT, _oracle_frame, _rigid, run_compare
@@ -137,6 +140,70 @@ def test_mixed_batch(ctx, wind, dftl, iterations):
             p, v = g.download()
             assert_bitexact(p, pos, "groom %d step %d positions" % (i, k))
             assert_bitexact(v, vel, "groom %d step %d velocities" % (i, k))
+    b.close()
+    for g in grooms:
+        g.close()
+
+
+@pytest.mark.parametrize("ngrooms", [63, 64, 65, 129, 4097])
+@pytest.mark.parametrize("mixed", [0, 1])
+def test_many_spans(ctx, ngrooms, mixed):
+    """The search for a tile's groom over one round of 64 spans, two, and three:
+    every groom is stepped exactly once."""
+    grooms, states = [], []
+    params = ba.make_params(force_scale=1.0, damping=0.9, length_scale=1.0, iterations=1)
+    big = 70000 if mixed else 3  # past the last level: by class, or the kernel of several
+    for i in range(ngrooms):
+        s, n = (big, 32) if i == ngrooms // 2 else (1 + (7 * i) % 11, (4, 8, 20)[i % 3])
+        pos, vel, roots = scene(s, n, i % 50)
+        g = ba.Groom(ctx, pos, vel, rest_roots=roots)
+        g.set_params(params)
+        g.set_root_mode(ba.FTL_ROOT_REST)
+        g.set_colliders(np.float32(SPHERES))
+        grooms.append(g)
+        states.append(dict(pos=pos.copy(), vel=vel.copy(), roots=roots, params=params, spheres=np.float32(SPHERES), N=n))
+    ba.batch_step(ctx, grooms, [DT] * ngrooms)
+    _oracle_frame(states, [DT] * ngrooms, [None] * ngrooms)
+    for i, (g, s) in enumerate(zip(grooms, states)):
+        p, v = g.download()
+        assert_bitexact(p, s["pos"], "groom %d positions" % i)
+        assert_bitexact(v, s["vel"], "groom %d velocities" % i)
+        g.close()
+
+
+@pytest.mark.parametrize("lanes", [0, 1])
+def test_batch_launch_while_capturing(ctx, lanes):
+    """A frame launched on a stream that is being captured runs at once and
+    leaves nothing in the caller's graph, with one kernel (lanes 0) as with
+    several."""
+    grooms, states = [], []
+    for i, n in enumerate((8, 16)):
+        pos, vel, roots = scene(100 + i, n, i)
+        params = ba.make_params(force_scale=1.0, damping=0.9, length_scale=1.0)
+        g = ba.Groom(ctx, pos, vel, rest_roots=roots)
+        g.set_params(params)
+        g.set_root_mode(ba.FTL_ROOT_REST)
+        g.set_colliders(np.float32(SPHERES))
+        g.set_lanes(lanes)
+        grooms.append(g)
+        states.append(dict(pos=pos.copy(), vel=vel.copy(), roots=roots, params=params, spheres=np.float32(SPHERES), N=n))
+    b = ba.Batch(ctx, grooms)
+    b.launch([DT] * 2)
+    stream, graph, nodes = hipm.Stream(), C.c_void_p(), C.c_size_t(99)
+    hipm.device_synchronize()
+    assert hipm.hip().hipStreamBeginCapture(stream.h, 1) == 0  # hipStreamCaptureModeThreadLocal
+    b.launch([DT] * 2, stream.h)
+    assert hipm.hip().hipStreamEndCapture(stream.h, C.byref(graph)) == 0
+    assert hipm.hip().hipGraphGetNodes(graph, None, C.byref(nodes)) == 0 and nodes.value == 0
+    assert hipm.hip().hipGraphDestroy(graph) == 0
+    hipm.device_synchronize()
+    b.launch([DT] * 2)
+    for _ in range(3):
+        _oracle_frame(states, [DT] * 2, [None] * 2)
+    for g, s in zip(grooms, states):
+        p, v = g.download()
+        assert_bitexact(p, s["pos"], "positions")
+        assert_bitexact(v, s["vel"], "velocities")
     b.close()
     for g in grooms:
         g.close()
