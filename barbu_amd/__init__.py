@@ -302,7 +302,7 @@ class Skin:
 
 
 class Batch:
-    """A fixed set of grooms stepped as one graph-captured frame (ftl_batch_*)."""
+    """A fixed set of grooms stepped as one frame (ftl_batch_*)."""
 
     def __init__(self, ctx, grooms):
         self.grooms = list(grooms)
@@ -332,7 +332,7 @@ class Batch:
 
 
 def batch_step(ctx, grooms, dt, stream=None):
-    """One batched step over grooms (ftl_batch_step): a tile-list kernel per launch class."""
+    """One batched step over grooms (ftl_batch_step)."""
     arr = (C.c_void_p * len(grooms))(*[g.handle.value for g in grooms])
     dt = np.ascontiguousarray(np.broadcast_to(np.asarray(dt, np.float32), (len(grooms),)))
     check(lib().ftl_batch_step(ctx.handle, arr, len(grooms), _ptr(dt), stream), "ftl_batch_step")

@@ -9,8 +9,8 @@
 //      creatures are pending, it takes them in arrival order (one per
 //      creature, up to the per-batch traffic cap), applies each request's
 //      inputs to its groom and launches one batched step on the slot's
-//      streams (tile plan -> pinned descriptors -> upload kernel -> one
-//      tile-list kernel per launch class, classes side by side).
+//      streams (tile plan -> pinned descriptors -> upload kernel -> the
+//      tile-list kernel, or one per launch class side by side).
 // Slots overlap on the device, so requests that arrive while a batch runs
 // start as soon as a slot frees, not when the device drains.
 #include <hip/hip_runtime.h>

@@ -274,8 +274,8 @@ ftl_status ftl_groom_root_frames(ftl_groom* g, float* roots, float* normals);
 /* -- batched steps --------------------------------------------------------- */
 
 /* Steps n grooms of one context as one batch: the grooms are cut into 64-lane
-   tiles, and one kernel per launch class present steps the tiles of its
-   grooms (the classes run side by side).  dt: one value per groom.  For repeated frames over the same
+   tiles, which one kernel steps (where grooms have their lanes set, one kernel
+   per launch class present).  dt: one value per groom.  For repeated frames over the same
    grooms, ftl_batch_create / ftl_batch_launch avoid re-planning. */
 ftl_status ftl_batch_step(ftl_ctx* ctx, ftl_groom* const* grooms, int n, const float* dt,
                           void* stream);
@@ -298,10 +298,10 @@ ftl_status ftl_batch_step(ftl_ctx* ctx, ftl_groom* const* grooms, int n, const f
    be read by anything else. */
 ftl_status ftl_batch_step_noalloc(ftl_ctx* ctx, ftl_groom* const* grooms, int n, const float* dt, void* stream);
 
-/* A fixed set of grooms stepped as one frame, planned once: a HIP graph
-   (parameter upload + one kernel per launch class) replayed by
-   ftl_batch_launch, or, when one kernel steps them all, the upload and that
-   kernel. */
+/* A fixed set of grooms stepped as one frame, planned once: ftl_batch_launch
+   uploads the parameters and launches the kernel that steps them all, or,
+   where they need a kernel per launch class, replays a HIP graph of the
+   upload and those. */
 ftl_status ftl_batch_create(ftl_ctx* ctx, ftl_groom* const* grooms, int n, ftl_batch** out);
 void ftl_batch_destroy(ftl_batch* b);
 /* One frame: per-groom dt (n values).  Colliders, transforms, params and time
