@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <mutex>
 #include <vector>
@@ -53,6 +54,17 @@ struct ftl_skin {
   void* d_nout = nullptr;
   std::vector<float> h_dq, h_mats;
   bool dirty = false, mats_dirty = false;
+  // Pinned copies of the bones (dual quaternions, then matrices) that upload
+  // kernels read, in turn; uploaded[k] follows the last kernel that read stage[k].
+  char* stage[2] = {};
+  hipEvent_t uploaded[2] = {};
+  int turn = 0;
+  // The one stream on which the vertices have been skinned and grooms stepped on
+  // them, kNoStream before the first; mixed: there were several, or one that
+  // cannot be told (a batch, a server, a capture, per-thread streams).
+  static inline void* const kNoStream = (void*)~(uintptr_t)0;
+  std::atomic<void*> user{kNoStream};
+  std::atomic<bool> mixed{false};
   // grooms bound to this skin (ctx->mu): destroying the skin unbinds them
   std::vector<ftl_groom*> bound;
 };
@@ -109,7 +121,9 @@ ftl_status ftl_check_device_range(const void* p, size_t bytes, const char* what)
 void ftl_dev_free(ftl_ctx* ctx, void* p, size_t bytes);
 // Fills the kernel descriptor of one step of g.
 // may_alloc false: fail rather than allocate the groom's wind lattice.
-ftl_status ftl_make_step(ftl_groom* g, float dt, FtlStep* A, bool may_alloc = true);
+// stream: the plain step's, else null (a skin whose groom is stepped by other
+// means is `mixed`).
+ftl_status ftl_make_step(ftl_groom* g, float dt, FtlStep* A, bool may_alloc = true, void* const* stream = nullptr);
 // Per-device set-up of the no-allocation batched step (its scratch address);
 // called by ftl_init with the device current.
 ftl_status ftl_noalloc_setup(int device);

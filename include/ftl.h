@@ -246,7 +246,9 @@ ftl_status ftl_skin_set_joint_matrices(ftl_skin* s, const float* global_pose, co
    joint matrices (:128).  Not renormalised, as in the reference. */
 ftl_status ftl_skin_set_rest_normals(ftl_skin* s, const float* normals);
 /* Skins every vertex (and normal) on `stream` (inc_skinning.glsl:22-31 and
-   the mode's subroutine). */
+   the mode's subroutine).  Asynchronous while the skin's updates and its
+   grooms' plain steps use one stream; once another one, a batch, a server or
+   a capture has used it, new bones wait for `stream` and are copied. */
 ftl_status ftl_skin_update(ftl_skin* s, void* stream);
 /* Synchronous copy of the skinned vertices (float4 [nverts]). */
 ftl_status ftl_skin_download(ftl_skin* s, float* verts);
