@@ -945,6 +945,9 @@ extern "C" ftl_status ftl_skin_update(ftl_skin* s, void* stream) {
     s->dirty = s->mats_dirty = false;
   } else if (s->dirty || s->mats_dirty) {
     // Synchronous copies: the bones are tiny and the host arrays are reused.
+    // (An upload of the time when one stream used the skin may still be on its way.)
+    for (hipEvent_t ev : s->uploaded)
+      if (ev && (e = hipEventSynchronize(ev)) != hipSuccess) return ftl_hip_fail(e, "hipEventSynchronize");
     if ((e = hipStreamSynchronize((hipStream_t)stream)) != hipSuccess) return ftl_hip_fail(e, "hipStreamSynchronize");
     if (s->dirty && (e = hipMemcpy(s->d_dq, s->h_dq.data(), (size_t)s->nbones * 32, hipMemcpyHostToDevice)) !=
                         hipSuccess)
