@@ -736,6 +736,9 @@ extern "C" ftl_status ftl_skin_create(ftl_ctx* ctx, const ftl_skin_desc* d, ftl_
   }
   ok = ok && hipMemcpy(s->d_dq, s->h_dq.data(), bb, hipMemcpyHostToDevice) == hipSuccess &&
        hipMemcpy(s->d_mats, s->h_mats.data(), mb, hipMemcpyHostToDevice) == hipSuccess;
+  for (int k = 0; k < 2; ++k)
+    ok = ok && hipHostMalloc((void**)&s->stage[k], bb + mb, hipHostMallocCoherent) == hipSuccess &&
+         hipEventCreateWithFlags(&s->uploaded[k], hipEventDisableTiming) == hipSuccess;
   {
     std::lock_guard<std::mutex> lk(ctx->mu);
     ctx->live_objects++;
@@ -922,14 +925,8 @@ extern "C" ftl_status ftl_skin_update(ftl_skin* s, void* stream) {
     // -> 21.8 us a frame, 2M of 32 807 -> 788.)
     const int k = s->turn;
     const size_t bb = (size_t)s->nbones * 32, mb = (size_t)s->nbones * 48;
-    if (!s->stage[k] && (e = hipHostMalloc((void**)&s->stage[k], bb + mb, hipHostMallocCoherent)) != hipSuccess)
-      return ftl_hip_fail(e, "hipHostMalloc bones");
-    if (!s->uploaded[k]) {
-      if ((e = hipEventCreateWithFlags(&s->uploaded[k], hipEventDisableTiming)) != hipSuccess)
-        return ftl_hip_fail(e, "hipEventCreate");
-    } else if ((e = hipEventSynchronize(s->uploaded[k])) != hipSuccess) {
-      return ftl_hip_fail(e, "hipEventSynchronize");
-    }
+    // (the stage was last read by the update before the previous one)
+    if ((e = hipEventSynchronize(s->uploaded[k])) != hipSuccess) return ftl_hip_fail(e, "hipEventSynchronize");
     if (s->dirty) {
       std::memcpy(s->stage[k], s->h_dq.data(), bb);
       if ((e = ftl_launch_upload(s->stage[k], s->d_dq, bb, (hipStream_t)stream)) != hipSuccess)
