@@ -95,8 +95,7 @@ __device__ __forceinline__ float3 bary(const float4* __restrict__ rnd, int inst,
 // (us write-back, through and streaming):
 // * Written through the XCD's L2 (the lines do not wait dirty for the end of
 //   the kernel) where its stores cover whole lines, that is by pages and by
-//   batches: 43 MB 10.3, 8.8; 131 MB 24.2, 21.4; 917 MB of 3 x 2 x 16 164,
-//   160.5; 812 MB of 4 x 3 x 7 146, 139.  The per-vertex form's runs of 2 nsub
+//   batches: 43 MB 10.3, 8.8; 131 MB 24.2, 21.4; 812 MB of 4 x 3 x 7 146, 139.  The per-vertex form's runs of 2 nsub
 //   vertices are whole 64-byte sectors when nsub is even (up to 256 MB: 4 x 3
 //   x 6, 224 MB, 37.0, 34.7; 6 x 2 x 10, 219 MB, 36.4, 34.2; above, 8 x 4 x 10,
 //   592 MB, 128, 136); otherwise the halves of a sector merge in the L2 only
@@ -226,7 +225,7 @@ __device__ __forceinline__ void expand_sync() {
 // and the blend weights in wts (LDS).  The stores are bounded by the pass's end:
 // the last batch's patches may end early.  NC > 0: the blend count, at compile
 // time.
-template <int NV, int NC, int B, FtlCache CP>
+template <int NV, int NC, int B, FtlCache CP, bool GUARD = false>
 __device__ __forceinline__ void expand_batch(const ExpandArgs& A, const float4* G0, const float4* wts, int b,
                                              int npatch, int lane) {
   const int nseg = A.nseg, nlines = A.nlines;
@@ -238,8 +237,10 @@ __device__ __forceinline__ void expand_batch(const ExpandArgs& A, const float4* 
   for (int s = 0; s < B * NV / 64; ++s) {
     const int item = s * 64 + lane;
     const int i = item / NV, v = item % NV;
+    const int patch = b * B + i;
+    if (GUARD && patch >= npatch) continue;
     const float4* G = G0 + i * kGuideF4;
-    const int seg = (b * B + i) % nseg;
+    const int seg = patch % nseg;
     const float u = (float)((v >> 1) + (v & 1)) / fsub;
     const Basis h = basis(u);
     float3 g[3];
@@ -267,7 +268,14 @@ __device__ __forceinline__ void expand_batch(const ExpandArgs& A, const float4* 
         ++inst;
       }
     };
-    if constexpr (NC > 0) {
+    if constexpr (CP == kCacheDefault) {
+      static_assert(NC > 0, "written back with the blend count at compile time only");
+      const long long iso = (long long)patch * nlines;
+      const long long iso_stride = (long long)A.ntris * nseg * nlines;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        A.out[(iso + (c / nlines) * iso_stride + c % nlines) * NV + v] = blend(wts[c]);
+    } else if constexpr (NC > 0) {
 #pragma unroll
       for (int c = 0; c < NC; ++c) {
         store(inst, line, blend(wts[c]));
@@ -334,7 +342,10 @@ __global__ __launch_bounds__(64) void ftl_expand_batched_kernel(ExpandArgs A) {
 #pragma unroll
   for (int r = 0; r < kRuns; ++r) gd[guide_index(r)] = gv[r];
   expand_sync();
-  expand_batch<NV, NC, B, CP>(A, gd, wts, b, npatch, lane);
+  if (CP == kCacheDefault && (b + 1) * B > npatch)
+    expand_batch<NV, NC, B, CP, CP == kCacheDefault>(A, gd, wts, b, npatch, lane);
+  else
+    expand_batch<NV, NC, B, CP>(A, gd, wts, b, npatch, lane);
 }
 
 // The same pass by pages of the output.  For one instance the capture of
@@ -485,7 +496,12 @@ void launch_expand_batched(const ExpandArgs& A, int nc, hipStream_t stream) {
   const size_t lds = (size_t)nc * sizeof(float4) + (size_t)B * kGuideF4 * sizeof(float4) + B * sizeof(int4);
   if constexpr (NSUB == 16) {
     if (nc == 6) {
-      hipLaunchKernelGGL((ftl_expand_batched_kernel<NV, 6, B, kCacheThrough>), dim3(nbatch), dim3(64), lds, stream, A);
+      // Above 384 MB plain stores to plain addresses beat those through a buffer
+      // (917 MB 154.5 us; through 161.7, written back by a buffer 166.5).
+      if ((long long)A.nthreads * nc * 16 > (384ll << 20))
+        hipLaunchKernelGGL((ftl_expand_batched_kernel<NV, 6, B, kCacheDefault>), dim3(nbatch), dim3(64), lds, stream, A);
+      else
+        hipLaunchKernelGGL((ftl_expand_batched_kernel<NV, 6, B, kCacheThrough>), dim3(nbatch), dim3(64), lds, stream, A);
       return;
     }
   }

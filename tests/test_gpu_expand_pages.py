@@ -40,7 +40,7 @@ def test_large_outputs(ctx, ninst, nlines, nsub):
 
 @pytest.mark.parametrize("above", [-1, 2])
 @pytest.mark.parametrize("mb,ninst,nlines,nsub", [(128, 2, 1, 13), (224, 1, 1, 15), (224, 2, 1, 8), (224, 1, 3, 16),
-                                                  (256, 2, 3, 6), (144, 3, 2, 9), (256, 4, 3, 8), (400, 3, 2, 7)])
+                                                  (256, 2, 3, 6), (144, 3, 2, 9), (256, 4, 3, 8), (400, 3, 2, 7), (384, 3, 2, 16)])
 def test_cache_lines(ctx, mb, ninst, nlines, nsub, above):
     """On both sides of the output sizes at which a form changes how its stores
     use the caches: pages, batches and single vertices, with ends that fill no
