@@ -1,6 +1,6 @@
 // Batched FTL steps: many grooms, uneven strand and point counts, stepped by
-// one kernel per frame after the upload of their descriptors (or, when they
-// need a kernel per launch class, by one graph launch).  There is no
+// one kernel per frame after the upload of their descriptors (or by a kernel
+// per launch class, side by side, when they need that).  There is no
 // counterpart in the reference, which dispatches one workgroup per strand of
 // its single groom (src/fx/hair.cc:112).
 //
@@ -8,12 +8,16 @@
 // class or wide form (points per lane x lanes per strand), a span of
 // consecutive tiles of the launch (one record per groom: the kernel maps a
 // tile to its groom by a search over the spans).  ftl_plan_tiles says which
-// kernel takes the spans.  A batch of several kernels is [upload the
-// per-groom descriptors from pinned memory -> one tile-list kernel per class
-// present, as parallel branches], captured once into a HIP graph (a batch of
-// one kernel has its graph too, for launches on a stream that is being
-// captured).  Two descriptor buffers (and graphs) alternate, so the host prepares frame k+1
-// while frame k runs.
+// kernel takes the spans.  A frame is [upload the per-groom descriptors from
+// pinned memory -> the kernel, or one tile-list kernel per class present on
+// streams forked from the caller's and joined back to it].  The same, class
+// after class, is captured once into a HIP graph for launches on a stream that
+// is being captured.  Two descriptor buffers (and graphs) alternate, so the
+// host prepares frame k+1 while frame k runs.
+//
+// (The graph has one last node.  With the classes as parallel branches, and so
+// a last node each, a graph launched behind another on one stream started
+// before the branches of the first had ended: frames of one groom overlapped.)
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -151,9 +155,9 @@ ftl_status ftl_plan_tiles(ftl_ctx* ctx, ftl_groom* const* grooms, int n, std::ve
   return FTL_OK;
 }
 
-// Enqueues one tile-list kernel per class on s.  With side streams (graph
-// capture, serving slots) the classes after the first are forked onto them
-// and joined back, so they run side by side (parallel graph branches).
+// Enqueues one tile-list kernel per class on s.  With side streams the classes
+// after the first are forked onto them and joined back, so they run side by
+// side.
 hipError_t ftl_enqueue_runs(const std::vector<ClassRun>& runs, const FtlStep* d_steps, const FtlSpan* d_spans,
                             hipStream_t s, const std::vector<hipStream_t>* side, const std::vector<hipEvent_t>* side_ev,
                             hipEvent_t fork) {
@@ -379,7 +383,7 @@ extern "C" ftl_status ftl_batch_create(ftl_ctx* ctx, ftl_groom* const* grooms, i
     hipError_t e1 = FTL_KERNEL_UPLOAD ? ftl_launch_upload(b->h_steps[k], b->d_steps[k], sb, b->cap)
                                       : hipMemcpyAsync(b->d_steps[k], b->h_steps[k], sb, hipMemcpyHostToDevice, b->cap);
     hipError_t e2 = e1 == hipSuccess
-                        ? ftl_enqueue_runs(b->runs, b->d_steps[k], b->d_spans, b->cap, &b->side, &b->side_ev, b->fork)
+                        ? ftl_enqueue_runs(b->runs, b->d_steps[k], b->d_spans, b->cap, nullptr, nullptr, nullptr)
                         : hipSuccess;
     hipError_t e3 = hipStreamEndCapture(b->cap, &b->graph[k]);
     if (e1 != hipSuccess) return bail(ftl_hip_fail(e1, "capture: descriptor upload"));
@@ -440,15 +444,15 @@ extern "C" ftl_status ftl_batch_launch(ftl_batch* b, const float* dt, void* stre
   const bool capturing =
       hipStreamIsCapturing((hipStream_t)stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
   if (capturing) (void)hipGetLastError();
-  if (b->runs.size() == 1 && !capturing) {
-    // One kernel after the upload: two launches on the caller's stream follow
-    // each other closer than the nodes of a graph do (a frame of 24 small
-    // grooms: 27.6 us, as a graph 34.7).
+  if (!capturing) {
+    // Launches on the caller's stream follow each other closer than the nodes
+    // of a graph do (a frame of 24 small grooms, one kernel: 27.6 us, as a graph
+    // 34.7).
     const size_t sb = b->grooms.size() * sizeof(FtlStep);
     if ((e = ftl_launch_upload(b->h_steps[k], b->d_steps[k], sb, (hipStream_t)stream)) != hipSuccess)
       return ftl_hip_fail(e, "descriptor upload");
-    if ((e = ftl_enqueue_runs(b->runs, b->d_steps[k], b->d_spans, (hipStream_t)stream, nullptr, nullptr, nullptr)) !=
-        hipSuccess)
+    if ((e = ftl_enqueue_runs(b->runs, b->d_steps[k], b->d_spans, (hipStream_t)stream, &b->side, &b->side_ev,
+                              b->fork)) != hipSuccess)
       return ftl_hip_fail(e, "batched step launch");
   } else if ((e = hipGraphLaunch(b->exec[k], (hipStream_t)stream)) != hipSuccess) {
     return ftl_hip_fail(e, "hipGraphLaunch");

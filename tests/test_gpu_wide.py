@@ -207,3 +207,55 @@ def test_batch_launch_while_capturing(ctx, lanes):
     b.close()
     for g in grooms:
         g.close()
+
+
+def _queued_batch(ctx, lanes, points, nstrands=6000):
+    """Grooms with enough work that frames queue up behind each other; their
+    batch, states for the oracle, and a function that launches one frame with
+    new root transforms."""
+    grooms, states, frames = [], [], []
+    for i, n in enumerate(points):
+        pos, vel, roots = scene(nstrands + i, n, i)
+        params = ba.make_params(force_scale=1.0, damping=0.9, length_scale=1.0, iterations=32)
+        g = ba.Groom(ctx, pos, vel, rest_roots=roots)
+        g.set_params(params)
+        g.set_root_mode(ba.FTL_ROOT_REST)
+        g.set_colliders(np.float32(SPHERES))
+        g.set_lanes(lanes)
+        grooms.append(g)
+        states.append(dict(pos=pos.copy(), vel=vel.copy(), roots=roots, params=params, spheres=np.float32(SPHERES), N=n))
+    b = ba.Batch(ctx, grooms)
+
+    def frame(stream):
+        models = [_rigid(len(frames), i) for i in range(len(grooms))]
+        frames.append(models)
+        for g, m in zip(grooms, models):
+            g.set_root_transform(m)
+        b.launch([DT] * len(grooms), stream)
+
+    def finish():
+        hipm.device_synchronize()
+        for models in frames:
+            _oracle_frame(states, [DT] * len(grooms), models)
+        for i, (g, s) in enumerate(zip(grooms, states)):
+            p, v = g.download()
+            assert_bitexact(p, s["pos"], "groom %d positions" % i)
+            assert_bitexact(v, s["vel"], "groom %d velocities" % i)
+        b.close()
+        for g in grooms:
+            g.close()
+
+    return frame, finish
+
+
+@pytest.mark.parametrize("lanes,points", [(0, (16, 32)), (1, (16, 32)), (1, (4, 8, 16, 32))])
+@pytest.mark.parametrize("null_stream", [0, 1])
+def test_batch_frames_follow_each_other(ctx, lanes, points, null_stream):
+    """Frames launched one behind the other without a wait between them: each
+    kernel of a frame follows all of the frame before (lanes 1: a kernel per
+    class)."""
+    frame, finish = _queued_batch(ctx, lanes, points)
+    stream = None if null_stream else hipm.Stream().h
+    for _ in range(7):
+        frame(stream)
+    finish()
