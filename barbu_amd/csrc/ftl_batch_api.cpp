@@ -44,6 +44,9 @@ struct ftl_batch {
   hipGraph_t graph[2] = {nullptr, nullptr};
   hipGraphExec_t exec[2] = {nullptr, nullptr};
   hipEvent_t done[2] = {nullptr, nullptr};
+  // Graphs of one node that records done[k], for frames on a capturing stream.
+  hipGraph_t mark[2] = {nullptr, nullptr};
+  hipGraphExec_t mark_exec[2] = {nullptr, nullptr};
   int cur = 0;
 };
 
@@ -312,6 +315,8 @@ static void batch_release(ftl_batch* b) {
   for (int k = 0; k < 2; ++k) {
     if (b->exec[k]) (void)hipGraphExecDestroy(b->exec[k]);
     if (b->graph[k]) (void)hipGraphDestroy(b->graph[k]);
+    if (b->mark_exec[k]) (void)hipGraphExecDestroy(b->mark_exec[k]);
+    if (b->mark[k]) (void)hipGraphDestroy(b->mark[k]);
     if (b->done[k]) (void)hipEventDestroy(b->done[k]);
     if (b->h_steps[k]) (void)hipHostFree(b->h_steps[k]);
     ftl_dev_free(ctx, b->d_steps[k], b->grooms.size() * sizeof(FtlStep));
@@ -391,6 +396,11 @@ extern "C" ftl_status ftl_batch_create(ftl_ctx* ctx, ftl_groom* const* grooms, i
     if (e3 != hipSuccess) return bail(ftl_hip_fail(e3, "hipStreamEndCapture"));
     if ((e = hipGraphInstantiate(&b->exec[k], b->graph[k], nullptr, nullptr, 0)) != hipSuccess)
       return bail(ftl_hip_fail(e, "hipGraphInstantiate"));
+    hipGraphNode_t node;
+    if ((e = hipGraphCreate(&b->mark[k], 0)) != hipSuccess ||
+        (e = hipGraphAddEventRecordNode(&node, b->mark[k], nullptr, 0, b->done[k])) != hipSuccess ||
+        (e = hipGraphInstantiate(&b->mark_exec[k], b->mark[k], nullptr, nullptr, 0)) != hipSuccess)
+      return bail(ftl_hip_fail(e, "graph of the frame's end"));
   }
   {
     std::lock_guard<std::mutex> lk(ctx->mu);
@@ -439,7 +449,9 @@ extern "C" ftl_status ftl_batch_launch(ftl_batch* b, const float* dt, void* stre
   }
   // A launch recorded into a capture of the caller's would read the batch's
   // buffers at every replay, whatever has become of them: there the graph is
-  // launched, which the runtime runs at once.
+  // launched, which the runtime runs at once, and so is the graph that records
+  // done[k] behind it: recorded on the stream itself, the event would become
+  // part of the capture and say nothing of the frame that ran.
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   const bool capturing =
       hipStreamIsCapturing((hipStream_t)stream, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
@@ -457,7 +469,12 @@ extern "C" ftl_status ftl_batch_launch(ftl_batch* b, const float* dt, void* stre
   } else if ((e = hipGraphLaunch(b->exec[k], (hipStream_t)stream)) != hipSuccess) {
     return ftl_hip_fail(e, "hipGraphLaunch");
   }
-  if ((e = hipEventRecord(b->done[k], (hipStream_t)stream)) != hipSuccess) return ftl_hip_fail(e, "hipEventRecord");
+  if (capturing) {
+    if ((e = hipGraphLaunch(b->mark_exec[k], (hipStream_t)stream)) != hipSuccess)
+      return ftl_hip_fail(e, "hipGraphLaunch of the frame's end");
+  } else if ((e = hipEventRecord(b->done[k], (hipStream_t)stream)) != hipSuccess) {
+    return ftl_hip_fail(e, "hipEventRecord");
+  }
   b->cur ^= 1;
   return FTL_OK;
 }

@@ -259,3 +259,23 @@ def test_batch_frames_follow_each_other(ctx, lanes, points, null_stream):
     for _ in range(7):
         frame(stream)
     finish()
+
+
+@pytest.mark.parametrize("lanes", [0, 1])
+def test_batch_frames_around_a_capture(ctx, lanes):
+    """Frames inside and after a capture, none of them waited for: each one's
+    descriptors stay as they are until it has read them.  (The frames in the
+    capture come back to a buffer that one of them used.)"""
+    frame, finish = _queued_batch(ctx, lanes, (16, 32))
+    stream, graph, nodes = hipm.Stream(), C.c_void_p(), C.c_size_t(99)
+    frame(None)
+    hipm.device_synchronize()
+    assert hipm.hip().hipStreamBeginCapture(stream.h, 1) == 0  # hipStreamCaptureModeThreadLocal
+    for _ in range(4):
+        frame(stream.h)
+    assert hipm.hip().hipStreamEndCapture(stream.h, C.byref(graph)) == 0
+    assert hipm.hip().hipGraphGetNodes(graph, None, C.byref(nodes)) == 0 and nodes.value == 0
+    assert hipm.hip().hipGraphDestroy(graph) == 0
+    for _ in range(4):
+        frame(stream.h)
+    finish()
