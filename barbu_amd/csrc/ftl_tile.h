@@ -504,6 +504,15 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
   // it row by row.
   auto load_phase = [&](auto wind_on) {
     constexpr bool wind = decltype(wind_on)::value;
+    // (The compiler otherwise joins what the copies have in common at their
+    // heads and keeps it alive through both: the 8-point forms of one lane took
+    // 92 to 96 VGPRs, or spilled, against 79 to 90.  Us a step of one lane a
+    // strand, joined and apart: 524k strands of 8 points 67.7, 66.2 with wind,
+    // 58.0, 52.7 without; 600k of 7 90.4, 88.8 with wind, 73.3, 70.0 without.)
+    if constexpr (wind)
+      asm volatile("; with wind" ::: "memory");
+    else
+      asm volatile("; without wind" ::: "memory");
     constexpr int RS = FTL_WAVE / C / G;
     // (the global gathers' taps leave the registers for two rows)
     constexpr int PD = wind && LW == 0 && PD_ > 2 ? 2 : PD_ < M ? PD_ : M;
