@@ -27,8 +27,10 @@ int ftl_class_guarded(int cls);
 //     stores keep their lines (1 GB of 32 points: default 435, stores alone
 //     405, with the loads 391; 922 MB of 24 points, three grooms in turn, 347
 //     -> 323).  The launch classes' loads stay cached with wind (405 against
-//     413); the wide forms' do not (-1 to +1.5%, and a test of the wind ahead
-//     of their loads costs as much).
+//     413) and where lines are shared (ftl_tile); the wide forms' do not (-1 to
+//     +1.5%, and a test of the wind ahead of their loads costs as much).
+// The guarded classes of 5 to 16 points on one lane use the default at every
+// size (ftl_plain.hip).
 FtlCache ftl_cache_for(size_t state_bytes);
 #define FTL_WITH_CACHE(cp, ...)                                                      \
   switch (cp) {                                                                      \

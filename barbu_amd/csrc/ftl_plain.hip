@@ -64,6 +64,16 @@ constexpr size_t kWindGroupLds =
 constexpr int kWindGroupsPerCu = (kWavesPerEu == 2 ? 8 : 16) / kWindWaves;
 constexpr bool kWindLds = (kWavesPerEu == 4 || kWavesPerEu == 2) && kWindGroupsPerCu * kWindGroupLds <= 160 * 1024;
 
+// How the class uses the caches.  A lane of a guarded class of 8 or 16 points
+// holds a strand that is no whole lines, and stores part of a line at a time:
+// written through or streamed, the parts do not merge in the L2 (us a step,
+// default against ftl_cache_for's choice: 33 MB of 7 points at 2 iterations 14.3,
+// 19.2, with wind 18.6, 23.7; 134 MB with wind 76.6, 88.8; 440 MB 222, 340; 440 MB
+// of 11 points 296, 576).
+constexpr FtlCache class_cache(FtlCache cp) {
+  return CL::GU && CL::G == 1 && CL::M > 4 && CL::M <= 16 ? kCacheDefault : cp;
+}
+
 // A class with the LDS form never runs its plain kernel with wind.
 constexpr int kPlainWind = kWindLds && FTL_WIND_LDS ? ftl_tile_impl::kWindOff : ftl_tile_impl::kWindAny;
 
@@ -124,10 +134,10 @@ hipError_t FTL_PASTE(ftl_launch_plain_, FTL_CLASS_ID)(const FtlStep& A, hipStrea
   if (nblocks <= 0) return hipSuccess;
   if (kWindLds && FTL_WIND_LDS && A.wind_grid) {
     const dim3 grid((nblocks + kWindWaves - 1) / kWindWaves), block(FTL_WAVE * kWindWaves);
-    FTL_WITH_CACHE(cp, hipExtLaunchKernelGGL(ftl_plain_wind_kernel<CP>, grid, block, 0, stream, start, stop, 0, A))
+    FTL_WITH_CACHE(cp, hipExtLaunchKernelGGL(ftl_plain_wind_kernel<class_cache(CP)>, grid, block, 0, stream, start, stop, 0, A))
     return hipGetLastError();
   }
-  FTL_WITH_CACHE(cp, hipExtLaunchKernelGGL(ftl_plain_kernel<CP>, dim3(nblocks), dim3(FTL_WAVE), 0, stream, start, stop, 0, A))
+  FTL_WITH_CACHE(cp, hipExtLaunchKernelGGL(ftl_plain_kernel<class_cache(CP)>, dim3(nblocks), dim3(FTL_WAVE), 0, stream, start, stop, 0, A))
   return hipGetLastError();
 }
 
@@ -162,7 +172,7 @@ void ftl_tiles_kernel(const FtlStep* __restrict__ grooms, const FtlSpan* __restr
 hipError_t FTL_PASTE(ftl_launch_tiles_, FTL_CLASS_ID)(const FtlStep* grooms, const FtlSpan* spans, int nspans,
                                                       int ntiles, int grid, hipStream_t stream, FtlCache cp) {
   if (ntiles <= 0 || nspans <= 0) return hipSuccess;
-  FTL_WITH_CACHE(cp, hipLaunchKernelGGL(ftl_tiles_kernel<CP>, dim3(grid), dim3(FTL_WAVE), 0, stream, grooms, spans, nspans,
+  FTL_WITH_CACHE(cp, hipLaunchKernelGGL(ftl_tiles_kernel<class_cache(CP)>, dim3(grid), dim3(FTL_WAVE), 0, stream, grooms, spans, nspans,
                                         ntiles))
   return hipGetLastError();
 }

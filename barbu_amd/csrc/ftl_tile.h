@@ -514,6 +514,13 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
     else
       asm volatile("; without wind" ::: "memory");
     constexpr int RS = FTL_WAVE / C / G;
+    // Streaming loads (ftl_cache_for) keep no line, so a line that two rows read
+    // comes twice: not for strands that are no whole lines, nor for the 4-point
+    // form, which they slow as well.  (Us a step above 384 MB, with and without
+    // them: 546 MB of 4 points 246, 215; of 7, one lane, 477, 304; of 20, two
+    // lanes, 389, 274; of 31, two lanes, 440 MB 466, 324; but of 40 and 48 on one
+    // lane they gain 4 to 15%.)
+    constexpr bool kStream = CP == kCacheStream && !wind && (GUARD ? M >= 48 : M * G > 4);
     // (the global gathers' taps leave the registers for two rows)
     constexpr int PD = wind && LW == 0 && PD_ > 2 ? 2 : PD_ < M ? PD_ : M;
     float4 xr[PD + 1], vr[PD + 1];
@@ -524,8 +531,8 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
     auto load_row = [&](int i) {
       const unsigned first = GUARD ? row_offset<M, G, GUARD, true>(N, i / C, lane) : off0 + 16u * (i / C * C);
       const unsigned off = first + 16u * (unsigned)(i % C * RS * N);
-      xr[i % (PD + 1)] = buffer_load4<CP == kCacheStream && !wind>(bpos, off);
-      vr[i % (PD + 1)] = buffer_load4<CP == kCacheStream && !wind>(bvel, off);
+      xr[i % (PD + 1)] = buffer_load4<kStream>(bpos, off);
+      vr[i % (PD + 1)] = buffer_load4<kStream>(bvel, off);
     };
 #pragma unroll
     for (int i = 0; i < PD; ++i) load_row(i);

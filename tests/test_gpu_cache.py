@@ -49,3 +49,14 @@ def test_batch(ctx, mb):
     batch.close()
     for g in grooms:
         g.close()
+
+
+@pytest.mark.parametrize("mb", [100, 390])
+@pytest.mark.parametrize("npoints,lanes,wind", [(7, 1, 0), (11, 1, 1), (3, 0, 0), (20, 2, 0), (48, 1, 0), (40, 4, 0)])
+def test_guarded_classes(ctx, mb, npoints, lanes, wind):
+    """Strands that are no whole lines, by the launch classes."""
+    nstrands = (mb << 20) // (32 * npoints) + 1
+    pos, vel, _ = ba.sphere_groom(nstrands, npoints, radius=1.0, length=0.3, seed=npoints)
+    params = ba.make_params(force_scale=1.0, damping=0.9, length_scale=1.0, iterations=1, wind_amplitude=2.0 * wind,
+                            wind_frequency=2.0, wind_seed=5)
+    run_compare(ctx, pos, vel, params, SPHERES, 1, lanes=lanes, label="N=%d lanes %d %d MB" % (npoints, lanes, mb))

@@ -80,3 +80,11 @@ def test_class_waves_per_simd(units, cls, waves):
         groups = 160 * 1024 // max(1, k[".group_segment_fixed_size"])
         by_lds = groups * k[".max_flat_workgroup_size"] // 64 // 4
         assert 512 // regs >= min(waves, by_lds), (k[".name"], k[".vgpr_count"])
+
+
+@pytest.mark.parametrize("cls", [11, 12])
+def test_guarded_one_lane_classes_write_back(units, cls):
+    """The guarded classes of 5 to 16 points on one lane exist with the default
+    use of the caches only (FtlCache 0): partial lines merge in the L2."""
+    uses = {m for k in units[cls] for m in re.findall(r"FtlCache(\d)", k[".name"])}
+    assert uses == {"0"}
