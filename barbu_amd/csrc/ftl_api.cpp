@@ -594,7 +594,10 @@ static ftl_status groom_step(ftl_groom* g, float dt, void* stream, hipEvent_t st
   if (st != FTL_OK) return st;
   // lanes left to the library: by the size of the launch
   const int form =
-      g->lanes == 0 ? ftl_wide_form(ftl_wide_level(g->ctx->ncu, &g->nstrands, &g->npoints, 1), g->npoints) : -1;
+      g->lanes == 0 ? ftl_wide_form(ftl_wide_level(g->ctx->ncu, &g->nstrands, &g->npoints, 1), g->npoints, true,
+                                    ftl_cache_for((size_t)g->nstrands * g->npoints * 2 * sizeof(float4)),
+                                    A.wind_grid != 0)
+                    : -1;
   const int cls = form >= 0 ? -1 : ftl_class_for(g->ctx, g->npoints, g->lanes, FTL_MAX_POINTS, A.wind_grid != 0);
   if (form < 0 && cls < 0) return ftl_fail(FTL_ERR_UNSUPPORTED, "no launch class for npoints=%d", g->npoints);
   hipError_t e;

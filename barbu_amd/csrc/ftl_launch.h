@@ -46,7 +46,8 @@ hipError_t ftl_launch_plain(int cls, const FtlStep& A, hipStream_t stream, hipEv
 int ftl_wide_level(int ncu, const int* nstrands, const int* npoints, int n);
 // The form of a groom in a launch of that level; at level 0, the form of the
 // point counts no exact launch class holds, or -1 (a launch class is faster).
-int ftl_wide_form(int level, int npoints);
+// plain: in a plain step, with its use of the caches and whether it has wind.
+int ftl_wide_form(int level, int npoints, bool plain = false, FtlCache cp = kCacheDefault, bool wind = false);
 // The plain step of one groom by a wide form.
 hipError_t ftl_launch_wide(int form, const FtlStep& A, hipStream_t stream, hipEvent_t start = nullptr,
                            hipEvent_t stop = nullptr);

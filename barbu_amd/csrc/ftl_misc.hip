@@ -270,13 +270,22 @@ int ftl_wide_level(int ncu, const int* nstrands, const int* npoints, int n) {
 // a guarded class's lanes; a wide form pads none of its loads and stores, and
 // at most its last lanes' sweeps (us at 262,144 strands, guarded class against
 // wide form: 6 points 29.8, 25.9; 9 points 51.6, 35.7; 20 points 81.6, 65.2;
-// 40 points 199, 160; 48 points 215, 192; 63 points 393, 276).
-int ftl_wide_form(int level, int npoints) {
+// 40 points 199, 160; 48 points 215, 192; 63 points 393, 276).  A plain step of
+// 13 to 15 points keeps its guarded class, which pads the least there, in wind,
+// which that takes from LDS (us, class against wide form: 314 MB of 14 points
+// 134, 155, at 2 iterations 111, 148; 137 MB of 15 points at 4 iterations 27%
+// less), and above 384 MB (440 MB of 14 points without wind at 4 and 8
+// iterations 135, 157 and 137, 156; with two colliders 144, 157 and 170, 164).
+// Below, without wind, the form is as fast or faster (40 MB 25.6, 24.5), and so
+// it is in batches, where both gather the wind from global memory (76, 71;
+// without wind 60, 60).
+int ftl_wide_form(int level, int npoints, bool plain, FtlCache cp, bool wind) {
   int g;
   if (level > 0) {
     g = wide_lanes(level, npoints);
   } else {
     if (npoints < 5 || npoints == 8 || npoints == 16 || npoints == 32 || npoints == 64) return -1;
+    if (plain && npoints >= 13 && npoints <= 15 && (wind || cp == kCacheStream)) return -1;
     g = npoints <= 16 ? 2 : npoints <= 32 ? 4 : 8;
   }
   return ftl_wide_id((npoints + g - 1) / g, g);

@@ -46,6 +46,19 @@ def test_levels(ctx, npoints, nstrands):
     run_compare(ctx, pos, vel, params, SPHERES, 1, label="N=%d S=%d" % (npoints, nstrands))
 
 
+@pytest.mark.parametrize("npoints", [12, 13, 14, 15, 17])
+@pytest.mark.parametrize("nstrands", [32767, 32769, 70001])
+@pytest.mark.parametrize("wind,dftl", [(0, 0), (1, 0), (1, 1)])
+def test_launches_of_13_to_15_points(ctx, npoints, nstrands, wind, dftl):
+    """On both sides of the last level and of the point counts whose plain step
+    keeps its launch class in launches that fill the chip."""
+    pos, vel, roots = scene(nstrands, npoints, npoints)
+    params = ba.make_params(force_scale=1.0, damping=0.9, length_scale=1.1, iterations=2, velocity_mode=dftl,
+                            max_velocity=2.0, wind_amplitude=2.0 * wind, wind_frequency=2.0, wind_seed=5)
+    run_compare(ctx, pos, vel, params, SPHERES, 2, roots=roots, root_mode=ba.FTL_ROOT_REST,
+                models=lambda k: _rigid(0, 0.1 * k), label="N=%d S=%d" % (npoints, nstrands))
+
+
 @pytest.mark.parametrize("npoints", [7, 20])
 def test_streaming_stores(ctx, npoints):
     """A ragged groom above the state size from which stores are hinted."""
