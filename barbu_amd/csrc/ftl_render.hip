@@ -92,32 +92,49 @@ __device__ __forceinline__ float3 bary(const float4* __restrict__ rnd, int inst,
 }
 
 // How a pass stores its output, which it writes once and does not read back
-// (us write-back, through and streaming):
-// * Written through the XCD's L2 (the lines do not wait dirty for the end of
-//   the kernel) where its stores cover whole lines, that is by pages and by
-//   batches: 43 MB 10.3, 8.8; 131 MB 24.2, 21.4; 812 MB of 4 x 3 x 7 146, 139.  The per-vertex form's runs of 2 nsub
-//   vertices are whole 64-byte sectors when nsub is even (up to 256 MB: 4 x 3
-//   x 6, 224 MB, 37.0, 34.7; 6 x 2 x 10, 219 MB, 36.4, 34.2; above, 8 x 4 x 10,
-//   592 MB, 128, 136); otherwise the halves of a sector merge in the L2 only
-//   while written back (4 x 3 x 7, 306 MB, 62, 112), but for runs of 14 or more
-//   in outputs that the Infinity Cache holds easily (8 x 1 x 15, 140 MB, 24.2,
-//   22.5; 4 x 2 x 3, 61 MB, 13.9, 15.8).
-// * Streaming, by pages and batches, where a patch makes at most 100 vertices
-//   of its twelve guide points and the output exceeds 224 MB: such a pass reads
-//   enough that its stores push the guides out of the caches (2 x 1 x 13, 476
-//   MB, 116, 115, 93; 2 x 2 x 8, 585 MB, 144, 143, 100; 2 x 1 x 14, 296 MB, 62,
-//   65, 58; but 2 x 3 x 16 127, 123, 125).
-// * One-line pages between 128 and 224 MB gain by neither (2 x 1 x 13, 142 MB,
-//   29.0, 29.6, 27.8; 238 MB 50.5, 51.8, 49.8).
+// (us written back by plain stores to plain addresses, through the XCD's L2,
+// and streaming):
+// * Through (the lines do not wait dirty for the end of the kernel) where its
+//   stores cover whole lines, that is by pages and by batches: 43 MB 10.3, 8.8;
+//   208 MB of 2 x 1 x 32 37.0, 33.4; 470 MB of 2 x 1 x 40 86, 83; 812 MB of
+//   4 x 3 x 7 146, 139; 292 MB of 3 x 2 x 16 46.7, 42.5; 568 MB of 2 x 4 x 12
+//   109.3, 106.9; 596 MB of 4 x 2 x 16 109.4, 105.5.  Six blends of sixteen
+//   subsegments, whose plain stores are addressed at compile time, write back
+//   above 384 MB (366 MB of 3 x 2 x 16 64, 61.7; 412 to 700 MB 3% less than
+//   through; 0.73 to 1.9 GB 5% less).
+// * The per-vertex form's runs of 2 nsub vertices are whole 64-byte sectors when
+//   nsub is even (up to 256 MB: 4 x 3 x 6, 224 MB, 37.0, 34.7; 6 x 2 x 10, 219
+//   MB, 36.4, 34.2; above, 8 x 4 x 10, 592 MB, 128, 136); otherwise the halves
+//   of a sector merge in the L2 only while written back (4 x 3 x 7, 306 MB, 62,
+//   112), but for runs of 14 or more in outputs that the Infinity Cache holds
+//   easily (8 x 1 x 15, 140 MB, 24.2, 22.5; 4 x 2 x 3, 61 MB, 13.9, 15.8).
+//   Written back through a buffer the same stores ran up to 20% slower (399 MB
+//   of 4 x 4 x 8 58, 70).
+// * Streaming, where a patch makes few vertices of its twelve guide points: such
+//   a pass reads enough that its stores push the guides out of the caches.  By
+//   batches, up to 64 vertices above 256 MB (324 MB of 1 x 4 x 8 64, 59, 53; 533
+//   MB of 2 x 2 x 8 123, 119, 87) and up to 96 above 384 MB in batches of four
+//   patches (617 MB of 3 x 1 x 16 121, 118, 102; 651 MB of 6 x 1 x 8 124, 121,
+//   113; but in batches of eight 685 MB of 4 x 1 x 12 124, 122, 129, and below
+//   273 MB of 4 x 1 x 12 45.5, 40.4, 52.4).  By pages up to 100, above 224 MB
+//   (2 x 1 x 13, 476 MB, 116, 115, 93; 2 x 1 x 14, 296 MB, 62, 65, 58; but 2 x 3
+//   x 16 127, 123, 125).
+long long output_bytes(const ExpandArgs& A) { return (long long)A.nthreads * A.ninst * A.nlines * 16; }
 FtlCache vertex_cache(const ExpandArgs& A) {
-  const long long bytes = (long long)A.nthreads * A.ninst * A.nlines * 16;
+  const long long bytes = output_bytes(A);
   return A.nsub % 2 == 0 ? bytes <= (256ll << 20) ? kCacheThrough : kCacheDefault
                          : A.nsub >= 7 && bytes <= (144ll << 20) ? kCacheThrough : kCacheDefault;
 }
-FtlCache run_cache(const ExpandArgs& A, bool page) {
-  const long long bytes = (long long)A.nthreads * A.ninst * A.nlines * 16;
-  if (bytes > (224ll << 20) && A.ninst * A.nlines * 2 * A.nsub <= 100) return kCacheStream;
-  return page && A.nlines == 1 && A.ninst <= 2 && bytes > (128ll << 20) ? kCacheDefault : kCacheThrough;
+FtlCache batch_cache(const ExpandArgs& A) {
+  const long long bytes = output_bytes(A);
+  const int vertices = A.ninst * A.nlines * 2 * A.nsub;
+  if (vertices == 192 && A.nsub == 16) return bytes <= (384ll << 20) ? kCacheThrough : kCacheDefault;
+  return (vertices <= 64 && bytes > (256ll << 20)) || (vertices <= 96 && A.nsub != 12 && bytes > (384ll << 20))
+             ? kCacheStream
+             : kCacheThrough;
+}
+FtlCache page_cache(const ExpandArgs& A) {
+  return output_bytes(A) > (224ll << 20) && A.ninst * A.nlines * 2 * A.nsub <= 100 ? kCacheStream : kCacheThrough;
 }
 
 template <FtlCache CP>
@@ -171,21 +188,28 @@ __global__ __launch_bounds__(256) void ftl_expand_kernel(ExpandArgs A) {
   }
   const float w = rel_pos(seg, u, (float)A.npoints);
 
-  // isoline (instance, triangle, segment, line) of the capture order, from the
-  // workgroup's first patch on
-  const int first = (int)(blockIdx.x * blockDim.x) / nv, run = A.nlines * nv;
-  float4* __restrict__ out = A.out + (long long)first * run;
-  const long long inst_stride = (long long)A.ntris * A.nseg * run;
-  const unsigned at = 16u * (unsigned)((ts - first) * run + v);
-  for (int inst = 0; inst < A.ninst; ++inst, out += inst_stride) {
-    const BufferRsrc b = buffer_of(out, 0x7fffffffu);
-    for (int line = 0; line < A.nlines; ++line) {
-      const float4 c = wts[inst * A.nlines + line];
-      // mat3x4(p0, p1, p2) * c
-      const float4 o = make_float4(__builtin_fmaf(c.z, g[2].x, __builtin_fmaf(c.y, g[1].x, c.x * g[0].x)),
-                                   __builtin_fmaf(c.z, g[2].y, __builtin_fmaf(c.y, g[1].y, c.x * g[0].y)),
-                                   __builtin_fmaf(c.z, g[2].z, __builtin_fmaf(c.y, g[1].z, c.x * g[0].z)), w);
-      buffer_store4<CP>(b, at + 16u * (unsigned)(line * nv), o);
+  auto blend = [&](const float4 c) {
+    // mat3x4(p0, p1, p2) * c
+    return make_float4(__builtin_fmaf(c.z, g[2].x, __builtin_fmaf(c.y, g[1].x, c.x * g[0].x)),
+                       __builtin_fmaf(c.z, g[2].y, __builtin_fmaf(c.y, g[1].y, c.x * g[0].y)),
+                       __builtin_fmaf(c.z, g[2].z, __builtin_fmaf(c.y, g[1].z, c.x * g[0].z)), w);
+  };
+  if constexpr (CP == kCacheDefault) {
+    // isoline (instance, triangle, segment, line) of the capture order
+    long long iso = (long long)ts * A.nlines;
+    const long long inst_stride = (long long)A.ntris * A.nseg * A.nlines;
+    for (int inst = 0; inst < A.ninst; ++inst, iso += inst_stride)
+      for (int line = 0; line < A.nlines; ++line) A.out[(iso + line) * nv + v] = blend(wts[inst * A.nlines + line]);
+  } else {
+    // the same, from the workgroup's first patch on
+    const int first = (int)(blockIdx.x * blockDim.x) / nv, run = A.nlines * nv;
+    float4* __restrict__ out = A.out + (long long)first * run;
+    const long long inst_stride = (long long)A.ntris * A.nseg * run;
+    const unsigned at = 16u * (unsigned)((ts - first) * run + v);
+    for (int inst = 0; inst < A.ninst; ++inst, out += inst_stride) {
+      const BufferRsrc b = buffer_of(out, 0x7fffffffu);
+      for (int line = 0; line < A.nlines; ++line)
+        buffer_store4<CP>(b, at + 16u * (unsigned)(line * nv), blend(wts[inst * A.nlines + line]));
     }
   }
 }
@@ -475,14 +499,11 @@ bool launch_expand_page_if_faster(const ExpandArgs& A, int nc, hipStream_t strea
   const size_t lds = ((size_t)nc + nv + (size_t)np * kGuideF4 + np) * sizeof(float4) + (size_t)(np + nv) * sizeof(float);
   if (lds > 64 * 1024) return false;
   const dim3 grid((unsigned)((total + kPage - 1) / kPage)), block(64);
-  const FtlCache cp = run_cache(A, true);
-  if (A.nlines == 1) {
-    FTL_WITH_CACHE(cp, hipLaunchKernelGGL((ftl_expand_page_kernel<true, CP>), grid, block, lds, stream, A, total))
-  } else if (cp == kCacheStream) {
-    hipLaunchKernelGGL((ftl_expand_page_kernel<false, kCacheStream>), grid, block, lds, stream, A, total);
-  } else {
-    hipLaunchKernelGGL((ftl_expand_page_kernel<false, kCacheThrough>), grid, block, lds, stream, A, total);
-  }
+  const bool one = A.nlines == 1, streaming = page_cache(A) == kCacheStream;
+  auto kernel = one ? (streaming ? ftl_expand_page_kernel<true, kCacheStream> : ftl_expand_page_kernel<true, kCacheThrough>)
+                    : (streaming ? ftl_expand_page_kernel<false, kCacheStream>
+                                 : ftl_expand_page_kernel<false, kCacheThrough>);
+  hipLaunchKernelGGL(kernel, grid, block, lds, stream, A, total);
   return true;
 }
 
@@ -494,21 +515,18 @@ void launch_expand_batched(const ExpandArgs& A, int nc, hipStream_t stream) {
   const int npatch = A.ntris * A.nseg;
   const int nbatch = (npatch + B - 1) / B;
   const size_t lds = (size_t)nc * sizeof(float4) + (size_t)B * kGuideF4 * sizeof(float4) + B * sizeof(int4);
+  const FtlCache cp = batch_cache(A);
   if constexpr (NSUB == 16) {
     if (nc == 6) {
-      // Above 384 MB plain stores to plain addresses beat those through a buffer
-      // (917 MB 154.5 us; through 161.7, written back by a buffer 166.5).
-      if ((long long)A.nthreads * nc * 16 > (384ll << 20))
-        hipLaunchKernelGGL((ftl_expand_batched_kernel<NV, 6, B, kCacheDefault>), dim3(nbatch), dim3(64), lds, stream, A);
-      else
-        hipLaunchKernelGGL((ftl_expand_batched_kernel<NV, 6, B, kCacheThrough>), dim3(nbatch), dim3(64), lds, stream, A);
+      hipLaunchKernelGGL((cp == kCacheThrough ? ftl_expand_batched_kernel<NV, 6, B, kCacheThrough>
+                                              : ftl_expand_batched_kernel<NV, 6, B, kCacheDefault>),
+                         dim3(nbatch), dim3(64), lds, stream, A);
       return;
     }
   }
-  if (run_cache(A, false) == kCacheStream)
-    hipLaunchKernelGGL((ftl_expand_batched_kernel<NV, 0, B, kCacheStream>), dim3(nbatch), dim3(64), lds, stream, A);
-  else
-    hipLaunchKernelGGL((ftl_expand_batched_kernel<NV, 0, B, kCacheThrough>), dim3(nbatch), dim3(64), lds, stream, A);
+  hipLaunchKernelGGL((cp == kCacheStream ? ftl_expand_batched_kernel<NV, 0, B, kCacheStream>
+                                         : ftl_expand_batched_kernel<NV, 0, B, kCacheThrough>),
+                     dim3(nbatch), dim3(64), lds, stream, A);
 }
 
 // Launches the batched pass where it measured faster than ftl_expand_kernel

@@ -54,3 +54,13 @@ def test_cache_lines(ctx, mb, ninst, nlines, nsub, above):
 def test_ends(ctx, T, ninst, nlines, nsub):
     """The last batch and the last workgroup hold fewer patches."""
     check(ctx, 40, 4, T, ninst, nlines, nsub)
+
+
+@pytest.mark.parametrize("above", [-1, 2])
+@pytest.mark.parametrize("mb,ninst,nlines,nsub", [(256, 3, 1, 8), (256, 5, 1, 8), (384, 2, 2, 12), (384, 4, 2, 8), (384, 1, 4, 16),
+                                                  (224, 2, 1, 26), (256, 4, 4, 8), (400, 4, 4, 8)])
+def test_store_lines(ctx, mb, ninst, nlines, nsub, above):
+    """The same for batches of few and of many vertices a patch, one-line pages
+    of many, and the per-vertex form's plain stores."""
+    per = 2 * ninst * nlines * nsub * 15
+    check(ctx, 2000, 16, (mb << 20) // (16 * per) + above, ninst, nlines, nsub)
