@@ -78,12 +78,19 @@ constexpr int ftl_chunk_of(int m, int g, bool guarded) {
 
 // Wide forms (ftl_wide.h): X(points per lane M, lanes per strand G); a form
 // takes any point count N with M = ceil(N / G).  Not launch classes: the
-// library picks them by the size of a launch (ftl_wide_lanes).
-#define FTL_WIDE_FORMS_2(X) X(3, 2) X(4, 2) X(5, 2) X(6, 2) X(7, 2) X(8, 2)
-#define FTL_WIDE_FORMS_4(X) X(1, 4) X(2, 4) X(3, 4) X(4, 4) X(5, 4) X(6, 4) X(7, 4) X(8, 4)
-#define FTL_WIDE_FORMS_8(X) X(1, 8) X(2, 8) X(3, 8) X(4, 8) X(5, 8) X(6, 8) X(7, 8) X(8, 8)
-#define FTL_WIDE_FORMS_16(X) X(1, 16) X(2, 16) X(3, 16) X(4, 16)
-#define FTL_WIDE_FORMS(X) FTL_WIDE_FORMS_2(X) FTL_WIDE_FORMS_4(X) FTL_WIDE_FORMS_8(X) FTL_WIDE_FORMS_16(X)
+// library picks them by the size of a launch (ftl_wide_level, ftl_wide_form).
+// FTL_LEVEL_FORMS: only in launches smaller than the chip, whose state of at most
+// 16 waves a CU, 64 MB on 256 CUs, is always written through.
+// FTL_DEFAULT_FORMS: also in launches that fill it.
+#define FTL_LEVEL_FORMS_2(X)
+#define FTL_LEVEL_FORMS_4(X) X(1, 4) X(2, 4) X(3, 4) X(4, 4)
+#define FTL_LEVEL_FORMS_8(X) X(1, 8) X(2, 8) X(3, 8) X(4, 8)
+#define FTL_LEVEL_FORMS_16(X) X(1, 16) X(2, 16) X(3, 16) X(4, 16)
+#define FTL_DEFAULT_FORMS_2(X) X(3, 2) X(4, 2) X(5, 2) X(6, 2) X(7, 2) X(8, 2)
+#define FTL_DEFAULT_FORMS_4(X) X(5, 4) X(6, 4) X(7, 4) X(8, 4)
+#define FTL_DEFAULT_FORMS_8(X) X(5, 8) X(6, 8) X(7, 8) X(8, 8)
+#define FTL_DEFAULT_FORMS_16(X)
+#define FTL_DEFAULT_FORMS(X) FTL_DEFAULT_FORMS_2(X) FTL_DEFAULT_FORMS_4(X) FTL_DEFAULT_FORMS_8(X)
 
 // How a step kernel's loads and stores use the caches (ftl_cache_for).
 enum FtlCache : int { kCacheDefault, kCacheThrough, kCacheStream };
@@ -102,6 +109,3 @@ constexpr int ftl_wide_g(int id) { return (id - 256) % 32; }
 #define FTL_DEFAULT_CLASSES(X)                                                              \
   X(0, 4, 1, false) X(1, 8, 1, false) X(2, 16, 1, false) X(4, 8, 2, false) X(5, 16, 2, false) \
   X(7, 4, 4, false) X(8, 8, 4, false) X(9, 16, 4, false) X(10, 4, 1, true) X(15, 4, 2, false)
-#define FTL_DEFAULT_FORMS(X)                                            \
-  X(3, 2) X(4, 2) X(5, 2) X(6, 2) X(7, 2) X(8, 2)                       \
-  X(5, 4) X(6, 4) X(7, 4) X(8, 4) X(5, 8) X(6, 8) X(7, 8) X(8, 8)

@@ -206,13 +206,17 @@ hipError_t ftl_launch_plain(int cls, const FtlStep& A, hipStream_t stream, hipEv
   return hipErrorInvalidValue;
 }
 
-#define FTL_WDECL(G)                                                                                               \
-  hipError_t ftl_launch_wide_##G(int m, const FtlStep& A, hipStream_t, hipEvent_t, hipEvent_t, FtlCache);              \
-  hipError_t ftl_launch_wide_tiles_##G(int m, const FtlStep*, const FtlSpan*, int, int, hipStream_t, FtlCache);
+#define FTL_WDECL(G) hipError_t ftl_launch_wide_##G(int m, const FtlStep& A, hipStream_t, hipEvent_t, hipEvent_t, FtlCache);
 FTL_WDECL(2)
 FTL_WDECL(4)
 FTL_WDECL(8)
 FTL_WDECL(16)
+#undef FTL_WDECL
+#define FTL_WDECL(G) \
+  hipError_t ftl_launch_wide_tiles_##G(int m, const FtlStep*, const FtlSpan*, int, int, hipStream_t, FtlCache);
+FTL_WDECL(2)
+FTL_WDECL(4)
+FTL_WDECL(8)
 #undef FTL_WDECL
 hipError_t ftl_launch_wide_all(const FtlStep*, const FtlSpan*, int, int, hipStream_t);
 #define FTL_ADECL(C) hipError_t ftl_launch_tiles_all_##C(const FtlStep*, const FtlSpan*, int, int, hipStream_t);

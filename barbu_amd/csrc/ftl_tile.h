@@ -330,7 +330,7 @@ __device__ __forceinline__ void sweep_points(float3 (&p)[M], Len len) {
 template <int M, bool GUARD, bool FINAL, FtlCache CP>
 __device__ __forceinline__ void sweep(const FtlStep& A, const VelArgs& V, const Spheres& S, float3 (&p)[M],
                                       const LenLds& l, int nl,
-                                      const float4* __restrict__ pp, float3& last_pre, float3& clast,
+                                      const float4* __restrict__ pp, float3& clast,
                                       float4* __restrict__ stage, BufferRsrc bvel, int N, int lane, int cm) {
   constexpr int C = Tile<M, 1, GUARD>::C;
   // Opaque per sweep: keeps the compiler from hoisting sigma * l[j] out of the
@@ -340,9 +340,6 @@ __device__ __forceinline__ void sweep(const FtlStep& A, const VelArgs& V, const 
   const float dl = V.delta;
   if (!FINAL) {
     sweep_points<M>(p, [&](int j) { return sg * l.get(j); });
-#pragma unroll
-    for (int j = 1; j < M; ++j)
-      if (GUARD ? j == nl - 1 : j == M - 1) last_pre = p[j];
     // Collisions of points 1 .. last (the root never collides; with GUARD the
     // slots past the last point are not collided at all).
     collide_sweep<M>(S, p, true, false, GUARD ? nl : M, cm);
@@ -374,10 +371,7 @@ __device__ __forceinline__ void sweep(const FtlStep& A, const VelArgs& V, const 
       stage[slot<C>(lane, m % C)] = make_float4(v.x, v.y, v.z, 0.0f);
       if (m % C == C - 1) flush_chunk<M, 1, GUARD, CP>(bvel, N, m / C, stage, lane);
     }
-    if (GUARD ? (j == nl - 1) : (j == M - 1)) {
-      clast = c;
-      last_pre = pn;
-    }
+    if (GUARD ? (j == nl - 1) : (j == M - 1)) clast = c;
   }
 }
 
@@ -642,12 +636,11 @@ __device__ __forceinline__ void ftl_tile(const FtlStep& A, int strand0, TileLds<
   const int K = A.iterations;
   bool bad = false;
   if constexpr (G == 1) {
-    float3 last_pre = p[0];
     float3 clast = f3(0.f, 0.f, 0.f);
     float3 u;
     for (int it = 0; it < K - 1; ++it)
-      sweep<M, GUARD, false, CP>(A, V, S, p, l, nl, pp, last_pre, clast, stage, bvel, N, lane, cm);
-    sweep<M, GUARD, true, CP>(A, V, S, p, l, nl, pp, last_pre, clast, stage, bvel, N, lane, cm);
+      sweep<M, GUARD, false, CP>(A, V, S, p, l, nl, pp, clast, stage, bvel, N, lane, cm);
+    sweep<M, GUARD, true, CP>(A, V, S, p, l, nl, pp, clast, stage, bvel, N, lane, cm);
     // The last point: velocity = raw correction, collisions deferred to here.
     u = clast;
 #pragma unroll

@@ -1,6 +1,7 @@
 // Kernels of the wide forms (ftl_wide.h) with FTL_WIDE_LANES lanes per strand
-// (one translation unit per lane count): the plain step of one groom, and the
-// tile-list kernel of batched frames.  FTL_WIDE_LANES = 0: the tile-list
+// (one translation unit per lane count): the plain step of one groom, and, of
+// the forms of launches that fill the chip, the tile-list kernel of batched
+// frames.  FTL_WIDE_LANES = 0: the tile-list
 // kernel that holds every form, for batches small enough to be one launch.
 #include <hip/hip_ext.h>
 
@@ -32,6 +33,7 @@ __global__ __launch_bounds__(FTL_WAVE) void ftl_wide_kernel(FtlStep arg) {
   ftl_wide_tile<M, G, CP>(A, blockIdx.x * (FTL_WAVE / G), sh);
 }
 
+#if FTL_WIDE_LANES != 16
 template <int M, int G, FtlCache CP>
 __global__ __launch_bounds__(FTL_WAVE) void ftl_wide_tiles_kernel(const FtlStep* __restrict__ grooms,
                                                                   const FtlSpan* __restrict__ spans, int nspans) {
@@ -42,8 +44,10 @@ __global__ __launch_bounds__(FTL_WAVE) void ftl_wide_tiles_kernel(const FtlStep*
   const int s0 = (t - __builtin_amdgcn_readfirstlane(spans[s].tile0)) * (FTL_WAVE / G);
   ftl_wide_tile<M, G, CP>(grooms[gi], s0, sh);
 }
+#endif
 
-#define FTL_FORMS FTL_PASTE(FTL_WIDE_FORMS_, FTL_WIDE_LANES)
+#define FTL_LEVEL FTL_PASTE(FTL_LEVEL_FORMS_, FTL_WIDE_LANES)
+#define FTL_DEFAULT FTL_PASTE(FTL_DEFAULT_FORMS_, FTL_WIDE_LANES)
 
 }  // namespace
 
@@ -56,12 +60,19 @@ hipError_t FTL_PASTE(ftl_launch_wide_, FTL_WIDE_LANES)(int m, const FtlStep& A, 
   case M:                                                                                                 \
     FTL_WITH_CACHE(cp, hipExtLaunchKernelGGL((ftl_wide_kernel<M, G, CP>), grid, block, 0, stream, start, stop, 0, A)) \
     return hipGetLastError();
-    FTL_FORMS(FTL_WL)
+    FTL_DEFAULT(FTL_WL)
+#undef FTL_WL
+#define FTL_WL(M, G)                                                                                                \
+  case M:                                                                                                          \
+    hipExtLaunchKernelGGL((ftl_wide_kernel<M, G, kCacheThrough>), grid, block, 0, stream, start, stop, 0, A);      \
+    return hipGetLastError();
+    FTL_LEVEL(FTL_WL)
 #undef FTL_WL
   }
   return hipErrorInvalidValue;
 }
 
+#if FTL_WIDE_LANES != 16
 hipError_t FTL_PASTE(ftl_launch_wide_tiles_, FTL_WIDE_LANES)(int m, const FtlStep* grooms, const FtlSpan* spans,
                                                              int nspans, int ntiles, hipStream_t stream, FtlCache cp) {
   const dim3 grid(ntiles), block(FTL_WAVE);
@@ -70,15 +81,16 @@ hipError_t FTL_PASTE(ftl_launch_wide_tiles_, FTL_WIDE_LANES)(int m, const FtlSte
   case M:                                                                                                         \
     FTL_WITH_CACHE(cp, hipLaunchKernelGGL((ftl_wide_tiles_kernel<M, G, CP>), grid, block, 0, stream, grooms, spans, nspans)) \
     return hipGetLastError();
-    FTL_FORMS(FTL_WT)
+    FTL_DEFAULT(FTL_WT)
 #undef FTL_WT
   }
   return hipErrorInvalidValue;
 }
+#endif
 
 #else  // every form in one kernel
 
-// A batch whose waves all fit the chip at once (ftl_wide_lanes) is one launch
+// A batch whose waves all fit the chip at once (ftl_wide_level) is one launch
 // of this kernel, whatever the point counts of its grooms: a span names its
 // form.  The kernel carries the registers of its largest form, which costs
 // such a batch nothing.  (Class kernels side by side, forked and joined in the
@@ -96,7 +108,8 @@ __global__ __launch_bounds__(FTL_WAVE) void ftl_wide_all_kernel(const FtlStep* _
   case ftl_wide_id(M, G):                                                         \
     ftl_wide_tile<M, G, kCacheThrough>(grooms[gi], tile * (FTL_WAVE / G), sh);    \
     break;
-    FTL_WIDE_FORMS_4(FTL_WA) FTL_WIDE_FORMS_8(FTL_WA) FTL_WIDE_FORMS_16(FTL_WA)
+    FTL_LEVEL_FORMS_4(FTL_WA) FTL_DEFAULT_FORMS_4(FTL_WA) FTL_LEVEL_FORMS_8(FTL_WA) FTL_DEFAULT_FORMS_8(FTL_WA)
+    FTL_LEVEL_FORMS_16(FTL_WA)
 #undef FTL_WA
   }
 }

@@ -88,3 +88,25 @@ def test_guarded_one_lane_classes_write_back(units, cls):
     use of the caches only (FtlCache 0): partial lines merge in the L2."""
     uses = {m for k in units[cls] for m in re.findall(r"FtlCache(\d)", k[".name"])}
     assert uses == {"0"}
+
+
+def test_wide_forms_built(units):
+    """The wide kernels that a launch can name: (points per lane, lanes) of
+    launches smaller than the chip written through only and never in a tile
+    list of their own; those of launches that fill it in every use of the
+    caches."""
+    src = open(os.path.join(build.CSRC, "ftl_classes.h")).read()
+
+    def forms(kind):
+        rows = re.findall(r"#define FTL_%s_FORMS_\d+\(X\)(.*)" % kind, src)
+        return {tuple(map(int, f)) for r in rows for f in re.findall(r"X\((\d+), (\d+)\)", r)}
+
+    def built(kernel):
+        names = [k[".name"] for u in units for k in u]
+        found = [re.search(kernel + r"ILi(\d+)ELi(\d+)EL\w*FtlCache(\d)E", n) for n in names]
+        return {tuple(map(int, f.groups())) for f in found if f}
+
+    assert len(forms("LEVEL")) == 12 and len(forms("DEFAULT")) == 14
+    tiles = {f + (c,) for f in forms("DEFAULT") for c in range(3)}
+    assert built("ftl_wide_tiles_kernel") == tiles
+    assert built("ftl_wide_kernel") == tiles | {f + (1,) for f in forms("LEVEL")}
