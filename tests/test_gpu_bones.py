@@ -1,6 +1,8 @@
 """Bones that change every frame, frames in a row: on one stream they are
 uploaded behind the frame before; once a second stream or a batch has used the
 skin, by copies that wait.  Bit for bit the oracle's frames in both."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -54,3 +56,77 @@ def test_frames_in_a_row(ctx, mode, uses):
     assert_bitexact(gv, V, "velocities")
     g.close()
     skin.close()
+
+
+def _frames(ctx):
+    """A skinned groom with its skin, a function that makes the bones of frame k
+    and steps the oracle `steps` times on them, and the final comparison."""
+    sc = ba.skinned_scene(4000, 8, ntris=2000, nbones=16, seed=6)
+    skin = ba.Skin(ctx, sc["rest"], sc["joints"], sc["weights"], sc["tris"], sc["nbones"])
+    g = ba.Groom(ctx, sc["pos"], sc["vel"])
+    g.bind_skin(skin, sc["tri"], sc["bary"])
+    params = ba.make_params(force_scale=1.0, damping=0.9, length_scale=1.0)
+    g.set_params(params)
+    g.set_colliders(np.float32([[0, 0, 0, 1.0]]))
+    P, V = sc["pos"].copy(), sc["vel"].copy()
+
+    def bones(k, steps=1):
+        b = ba.bones(sc, (k + 1) * float(DT) * 10)
+        roots = orc.bary_roots_f32(sc["tris"], sc["tri"], sc["bary"], orc.skin_f32(b, sc["joints"], sc["weights"], sc["rest"]))
+        op = oracle_params_for(params, 8, DT, spheres=[(0, 0, 0, 1.0)], root_mode=ba.FTL_ROOT_REST)
+        for _ in range(steps):
+            orc.step_f32(op, P, V, roots)
+        return b
+
+    def finish():
+        hipm.device_synchronize()
+        gp, gv = g.download()
+        assert_bitexact(gp, P, "positions")
+        assert_bitexact(gv, V, "velocities")
+        g.close()
+        skin.close()
+
+    return skin, g, bones, finish
+
+
+def test_second_stream_only_steps(ctx):
+    """Another stream than the updates' steps the grooms (the caller orders the
+    two): from then on new bones wait."""
+    skin, g, bones, finish = _frames(ctx)
+    a, b = hipm.Stream(), hipm.Stream()
+    for k in range(8):
+        skin.set_bones(bones(k))
+        skin.update(a.h)
+        if k < 3:
+            g.step(DT, a.h)
+        else:
+            a.synchronize()
+            g.step(DT, b.h)
+            b.synchronize()
+    finish()
+
+
+def test_captured_frame(ctx):
+    """An update and a step recorded into a graph between frames with new bones:
+    replays use the bones of the time, later frames the new ones."""
+    skin, g, bones, finish = _frames(ctx)
+    st, graph, run = hipm.Stream(), C.c_void_p(), C.c_void_p()
+    hip = hipm.hip()
+    for k in range(4):
+        skin.set_bones(bones(k, 1 if k < 3 else 4))
+        skin.update(st.h)
+        g.step(DT, st.h)
+    st.synchronize()
+    assert hip.hipStreamBeginCapture(st.h, 1) == 0  # hipStreamCaptureModeThreadLocal
+    skin.update(st.h)
+    g.step(DT, st.h)
+    assert hip.hipStreamEndCapture(st.h, C.byref(graph)) == 0
+    assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, C.c_size_t(0)) == 0
+    for _ in range(3):
+        assert hip.hipGraphLaunch(run, st.h) == 0
+    for k in range(4, 9):
+        skin.set_bones(bones(k))
+        skin.update(st.h)
+        g.step(DT, st.h)
+    finish()
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
