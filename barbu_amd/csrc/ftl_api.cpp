@@ -5,7 +5,7 @@
 // uBoundingSphere, glDispatchCompute(nroots), barrier, copy the write buffer
 // back.  Here a step is one kernel launch over device-resident state that is
 // updated in place; parameters travel as kernel arguments (plain step) or as a
-// device table uploaded inside a captured HIP graph (batched frames).
+// device table uploaded ahead of the kernel (batched frames).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

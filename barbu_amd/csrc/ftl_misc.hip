@@ -257,6 +257,13 @@ static int wide_lanes(int level, int npoints) {
 //   64 points: 16,384          16 lanes 32.1, 8 lanes 33.1, class 43.6
 //              32,768           8 lanes 44.0, class 52.0;                65,536  74.7, class 68.2
 //    4 points: 65,536           4 lanes 8.8, class 10.1;                131,072  13.3, class 11.9
+// The lines were drawn at 8 iterations without wind.  Just below them, 4 to 64
+// points, the level against the class: at 16 iterations and more 5 to 60% less,
+// in wind too (16 points, 65,529 strands, 16 iterations 28.4, 35.1, in wind 32.3,
+// 35.8; 256 iterations 247, 359); at 8 in wind 5% more to 40% less (16 and 32
+// points 24.1, 24.3 and 42.8, 42.6; 64 points, 32,761 strands, 50.0, 47.5); at 4
+// in wind up to 15% more (32 points 34.6, 31.6; 64 points 42.2, 36.7) and at 1 up
+// to 20% (32 points, 32,761 strands, 20.1, 16.8).
 int ftl_wide_level(int ncu, const int* nstrands, const int* npoints, int n) {
   for (int level = 16; level >= 4; level /= 2) {
     int64_t waves = 0;

@@ -13,9 +13,15 @@
 //   5 of 16 and 32 in wind 92.4, 73.7;               27 of 8 to 64 84.8, 52.0
 //   25 of 8 to 64 275, 240;                          26 of 12 to 64 in wind 322, 297
 //   32 of 8 to 64, every groom moving, 497, 460
-// The small classes run at the large ones' four waves per SIMD here.  In a
-// mixed batch that costs nothing that shows; a batch of one class keeps its
-// own kernel, as does one with grooms whose lanes were set.
+// (The kernels per class then were branches of a graph.  As launches forked
+// from the caller's stream, over 1,462 drawn mixes, those small enough for
+// FTL_WIDE_ALL either way among them: 0.97 to 4.3 times this one, 1.7 in the mean.)
+// The small classes run at the large ones' four waves per SIMD here, also where
+// one fills most of the batch: 1M strands of 4 points, whose own kernel runs
+// eight, beside 3,000 of 8 took 65.1 us by class and 49.8 here, in wind 67.0 and
+// 61.5, at 2 iterations in wind 62.5 and 59.8.  A batch of one class keeps its own
+// kernel, as does one with grooms whose lanes were set or whose class the tables
+// pick from outside FTL_DEFAULT_CLASSES.
 #include "ftl_launch.h"
 #include "ftl_wide.h"
 

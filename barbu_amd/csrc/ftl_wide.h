@@ -2,7 +2,7 @@
 // lane (M <= 8), any point count N <= G * M.
 //
 // The step of a strand is a serial chain of (K + lanes - 1) * M point updates
-// (the lane pipeline of ftl_tile.h), about 22 dependent vector instructions
+// (the lane pipeline of ftl_tile.h), about 17 dependent vector instructions
 // each.  A launch too small to fill the chip is bound by that chain and by the
 // round trips of its loads, not by throughput, so these forms trade vector
 // work (lanes idle while the pipeline fills and drains) for a shorter chain:

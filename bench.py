@@ -517,7 +517,7 @@ def main():
                      "copy_reference_gbs": r["copy_gbs"]},
     }
     if args.workload in ("batched", "all"):
-        log("batched: 64 uneven grooms, %d frames (graph) and %d frames of per-groom launches"
+        log("batched: 64 uneven grooms, %d frames and %d frames of per-groom launches"
             % (args.batched_frames, args.batched_frames))
         b = bench_batched(ba, hipm, args.batched_frames, 3)
         fb = b["batched"]
@@ -528,7 +528,7 @@ def main():
         gb = b["cps"] * BYTES_PER_CP / frame_s / 1e9
         out["batched"] = {
             "workload": "64 grooms, strands log-uniform [1024, 262144], points {8,16,32,64}, lengths U(0.05,0.4), "
-                        "random rigid motion, 1-3 spheres; one graph launch per frame",
+                        "random rigid motion, 1-3 spheres; one batch launch per frame",
             "control_points": b["cps"], "tiles": b["ntiles"], "grid": b["grid"], "frames": args.batched_frames,
             "value": v_b, "unit": "CP updates/s", "ms_per_frame": 1000.0 * fb["wall_s"] / args.batched_frames,
             "gpu_ms_per_frame": fb["gpu_ms"] / args.batched_frames,
@@ -538,9 +538,8 @@ def main():
             "roofline": {"bound": "hbm", "achieved": gb, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": gb / HBM_PEAK_GBS, "traffic": load_traffic("batched"),
                          "frame_us": frame_s * 1e6, "bytes_per_frame": b["cps"] * BYTES_PER_CP,
-                         "timing": "HIP events around the timed graph launches on their stream; a frame is "
-                                   "the descriptor upload plus one tile-list kernel per launch class, the "
-                                   "classes running side by side"},
+                         "timing": "HIP events around the timed frames on their stream; a frame is the "
+                                   "descriptor upload plus one tile-list kernel for all launch classes"},
         }
     if args.workload in ("served", "all"):
         target = args.served_target_mb << 20

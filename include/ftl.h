@@ -276,8 +276,9 @@ ftl_status ftl_groom_root_frames(ftl_groom* g, float* roots, float* normals);
 /* -- batched steps --------------------------------------------------------- */
 
 /* Steps n grooms of one context as one batch: the grooms are cut into 64-lane
-   tiles, which one kernel steps (where grooms have their lanes set, one kernel
-   per launch class present).  dt: one value per groom.  For repeated frames over the same
+   tiles, which one kernel steps (where grooms have their lanes set, or a tuned
+   class that the common kernel does not hold, one kernel per launch class
+   present).  dt: one value per groom.  For repeated frames over the same
    grooms, ftl_batch_create / ftl_batch_launch avoid re-planning. */
 ftl_status ftl_batch_step(ftl_ctx* ctx, ftl_groom* const* grooms, int n, const float* dt,
                           void* stream);
@@ -302,12 +303,13 @@ ftl_status ftl_batch_step_noalloc(ftl_ctx* ctx, ftl_groom* const* grooms, int n,
 
 /* A fixed set of grooms stepped as one frame, planned once: ftl_batch_launch
    uploads the parameters and launches the kernel that steps them all, or,
-   where they need a kernel per launch class, replays a HIP graph of the
-   upload and those. */
+   where they need a kernel per launch class, those side by side on streams
+   forked from the caller's and joined back to it. */
 ftl_status ftl_batch_create(ftl_ctx* ctx, ftl_groom* const* grooms, int n, ftl_batch** out);
 void ftl_batch_destroy(ftl_batch* b);
 /* One frame: per-groom dt (n values).  Colliders, transforms, params and time
-   are read from the grooms at call time.  Asynchronous on `stream`.  Refused
+   are read from the grooms at call time.  Asynchronous on `stream`; on a stream
+   that is being captured the frame runs at once and is not recorded.  Refused
    with FTL_ERR_INVALID_ARGUMENT once one of the batch's grooms has been
    destroyed. */
 ftl_status ftl_batch_launch(ftl_batch* b, const float* dt, void* stream);
