@@ -6,7 +6,10 @@
 
 // X(id, points per lane, lanes per strand, guarded, waves per SIMD targeted
 // by the register allocator: the highest at which neither the plain nor the
-// tile-list kernel of the class spills to memory, points per lane of a load/store
+// tile-list kernel of the class spills to memory (1 and 11 fit six, where they
+// hold one row of loads in flight instead of three: us a step, six and five, 134
+// MB of 8 points 68.5, 52.7, in wind 69.2, 66.1; of 7 76.9, 65.3, in wind 75.8,
+// 76.6), points per lane of a load/store
 // chunk: 8 float4 make one 128-byte line, so each line of the groom is read
 // by one request; 4 halves the LDS stage where a bigger one would cost
 // occupancy, at the price of two requests per line)
